@@ -2,9 +2,10 @@
 // f16/bf16 output (src/tklab/kernels/matmul.py:72-164 computes the same
 // product; here the tiling is MI355X's own).
 //
-// tk_gemm sends row-major operands with K % 32 == 0 to the buffer->LDS DMA kernel
-// in gemm_dma.hip. This file's register-staged kernel takes everything else:
-// arbitrary strides (transposed views), K tails, unaligned rows.
+// tk_gemm sends operands stored by aligned rows (row-major or transposed) to the
+// buffer->LDS DMA kernels in gemm_dma.hip. This file's register-staged kernel takes
+// everything else: two non-unit strides, unaligned rows, odd row lengths, operands of 2 GiB
+// and more.
 //
 // Block tile 256 x 256, K step 64, 256 threads = 4 wave64s in a 2 x 2 grid;
 // each wave owns a 128 x 128 sub-tile as 4 x 4 MFMA tiles of
@@ -268,8 +269,9 @@ extern "C" int tk_gemm(int dtype, const void* a, const void* b, void* c, int64_t
   Problem p{(int)m, (int)n, (int)k, stride_am, stride_ak, stride_bk, stride_bn,
             stride_cm, stride_cn, (int)tiles_m, (int)tiles_n};
   hipStream_t s = tk::as_stream(stream);
-  if (tk::gemm_dma_applies(a, b, m, n, k, stride_am, stride_ak, stride_bk, stride_bn)) {
-    tk::gemm_dma_launch(dtype, a, b, c, m, n, k, stride_am, stride_bk, stride_cm, stride_cn, s);
+  tk::gemm_dma::Plan plan;
+  if (tk::gemm_dma::plan(a, b, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, &plan)) {
+    tk::gemm_dma_launch(plan, dtype, a, b, c, m, n, k, stride_cm, stride_cn, s);
     return tk::check_launch("gemm");
   }
   const bool fast = stride_ak == 1 && stride_bn == 1 && k % 8 == 0 && n % 8 == 0 &&
@@ -337,7 +339,8 @@ extern "C" int tk_gemm_rowscale(int dtype, const void* a, const void* b, const f
     return tk::fail("gemm_rowscale: needs unit inner strides, 16-byte aligned rows, k %% 32 == 0, "
                     "n %% 8 == 0 and operands below 2 GiB");
   if (tk::cdiv(m, BM) * tk::cdiv(n, BN) > INT32_MAX) return tk::fail("gemm_rowscale: too many tiles");
-  tk::gemm_dma_launch(dtype, a, b, c, m, n, k, stride_am, stride_bk, stride_cm, stride_cn,
-                      tk::as_stream(stream), row_scale);
+  const tk::gemm_dma::Plan plan{tk::gemm_dma::Layout::NN, false, false, stride_am, stride_bk};
+  tk::gemm_dma_launch(plan, dtype, a, b, c, m, n, k, stride_cm, stride_cn, tk::as_stream(stream),
+                      row_scale);
   return tk::check_launch("gemm_rowscale");
 }

@@ -6,16 +6,36 @@
 
 namespace tk {
 
-// True when the DMA kernel handles this problem: row-major f16/bf16 operands with unit
-// inner strides, 16-byte aligned rows, K a multiple of 32 and byte extents below 2 GiB.
+namespace gemm_dma {
+
+// How the operands are stored, BLAS letters: N row-major, T transposed. NN: A [M][K], B [K][N];
+// NT: A [M][K], B [N][K]; TN: A [K][M], B [K][N].
+enum class Layout { NN, NT, TN };
+
+struct Plan {
+  Layout layout;
+  bool swap;      // compute C^T = B^T A^T (both operands transposed)
+  bool k_tail;    // K may end inside a 32-wide K tile
+  int64_t lda, ldb;  // row strides of the stored matrices, in elements (after the swap)
+};
+
+// True when the DMA kernels handle this problem: f16/bf16 operands, each stored with one unit
+// stride, a contiguous extent and a row stride that are multiples of 8 elements, a 16-byte
+// aligned base and a byte extent below 2 GiB.
+bool plan(const void* a, const void* b, int64_t m, int64_t n, int64_t k, int64_t stride_am,
+          int64_t stride_ak, int64_t stride_bk, int64_t stride_bn, Plan* plan);
+
+}  // namespace gemm_dma
+
+// True when that is a row-major problem with K a multiple of 32 (the fused kernels' contract).
 bool gemm_dma_applies(const void* a, const void* b, int64_t m, int64_t n, int64_t k,
                       int64_t stride_am, int64_t stride_ak, int64_t stride_bk, int64_t stride_bn);
 
-// Enqueues the DMA kernel; arguments are checked by the caller. With `row_scale`
-// (float32[m]) row m of C is round(row_scale[m] * acc).
-void gemm_dma_launch(int dtype, const void* a, const void* b, void* c, int64_t m, int64_t n,
-                     int64_t k, int64_t stride_am, int64_t stride_bk, int64_t stride_cm,
-                     int64_t stride_cn, hipStream_t stream, const float* row_scale = nullptr);
+// Enqueues the DMA kernel for a plan; arguments are checked by the caller. With `row_scale`
+// (float32[m], row-major problems only) row m of C is round(row_scale[m] * acc).
+void gemm_dma_launch(const gemm_dma::Plan& plan, int dtype, const void* a, const void* b, void* c,
+                     int64_t m, int64_t n, int64_t k, int64_t stride_cm, int64_t stride_cn,
+                     hipStream_t stream, const float* row_scale = nullptr);
 
 // Enqueues the SwiGLU-fused DMA kernel: y = swiglu(value = a * b_up, gate = a * b_gate),
 // both weights [K, N] row-major; each must satisfy gemm_dma_applies with `a`.

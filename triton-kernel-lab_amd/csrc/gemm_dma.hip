@@ -1,4 +1,4 @@
-// GEMM C = A * B for row-major f16/bf16 A [M, K] and B [K, N] (unit inner stride),
+// GEMM C = A * B for f16/bf16 A [M, K] and B [K, N], each stored row-major or transposed,
 // float32 accumulation: the fast path behind tk_gemm (src/tklab/kernels/matmul.py:72-164
 // computes the same product with a Triton tile loop).
 //
@@ -46,6 +46,14 @@
 // Tile order: workgroup w runs on XCD w % 8; tiles are renumbered so each XCD walks a
 // contiguous range in groups of 4 M-tiles, sharing A and B panels in that XCD's L2.
 //
+// Transposed operands (a linear layer's gradients dy * w^T and x^T * dy) keep the tiles, the
+// steps and the order of every sum; only what a stage holds and how its fragments are read
+// changes. A [K][M] comes in 32-wide k-row tiles like B and is read transposed (TN); B [N][K]
+// comes in 64-wide tiles like A and is read as rows (NT). Loading them element by element
+// through registers (the general kernel in gemm.hip) ran 8192 x 4096 x 4096 in 4.1 ms each
+// way, bound by its 2-byte loads; these run dy * w^T and x^T * dy at the row-major product's
+// speed (all three products: 8.41 -> 0.584 ms, 1.41 PFLOP/s bf16).
+//
 // Row-scaled variant (kRowScale): C[m, :] = round(s[m] * acc),
 // one float32 multiply before the rounding. With s = rstd of a normalization whose
 // weight is folded into B, this is the normalized GEMM rms_norm(a) * B' without the
@@ -63,6 +71,9 @@
 #include "gemm.hpp"
 #include "tk_common.hpp"
 
+#include <type_traits>
+#include <utility>
+
 // No floating-point contraction in this file: the SwiGLU epilogue must round
 // value * gate * sigmoid(gate) to float32 and then to the storage type, as the SwiGLU
 // kernel and the reference do (a fused multiply-convert would round once).
@@ -70,17 +81,20 @@
 
 namespace {
 
+using tk::gemm_dma::Layout;
+
 constexpr int BM = 256, BN = 256, BK = 32;
 constexpr int kThreads = 512;  // 8 waves
 constexpr int kGroupM = 4;
 constexpr int kXcds = 8;
-// A ring: kAStages stages of one 64-wide K tile (256 rows x 128 B); B ring: kBStages stages
-// of one 32-wide K tile (32 k-rows x 512 B). 96 + 64 KiB: all of the CU's LDS.
+// K-contiguous operands come in 64-wide K tiles (256 rows x 128 B), the others in 32-wide K
+// tiles (32 k-rows x 512 B). NN: three 64-wide A stages and four 32-wide B stages; NT: three
+// 64-wide A and two 64-wide B stages; TN: four 32-wide stages of each. At most 160 KiB: all
+// of the CU's LDS.
 constexpr int kAStages = 3, kBStages = 4;
-constexpr int kABytes = 256 * 64 * 2;        // 32 KiB per A stage
-constexpr int kOperandBytes = 256 * BK * 2;  // 16 KiB per B stage
-constexpr int kBRing = kAStages * kABytes;   // B ring offset
-constexpr int kLdsBytes = kBRing + kBStages * kOperandBytes;
+constexpr int kABytes = 256 * 64 * 2;        // 32 KiB per 64-wide stage
+constexpr int kOperandBytes = 256 * BK * 2;  // 16 KiB per 32-wide stage
+constexpr int kLdsBytes = kAStages * kABytes + kBStages * kOperandBytes;
 constexpr uint32_t kOob = 0x80000000u;  // past every buffer's num_records: reads as zero
 // Epilogue: the C tile is staged in the ring's LDS (at most 256 rows of 528 bytes), the row
 // scales of the row-scaled variant after it.
@@ -96,7 +110,7 @@ typedef __attribute__((address_space(3))) void lds_void;
 
 struct Problem {
   int m, n, k;
-  int lda, ldb, ldb2;  // ldb2: the up weight's k stride (SwiGLU variant)
+  int lda, ldb, ldb2;  // row strides of the stored matrices; ldb2: the up weight's k stride (SwiGLU variant)
   int64_t scm, scn;
   int tiles_m, tiles_n;
   uint32_t a_bytes, b_bytes, b2_bytes;
@@ -187,6 +201,15 @@ __device__ __forceinline__ i32x4 read_b(uint32_t addr) {
   return i32x4{lo[0], lo[1], hi[0], hi[1]};
 }
 
+// f(0) .. f(3) with compile-time indices.
+template <typename F>
+__device__ __forceinline__ void unroll4(F&& f) {
+  f(std::integral_constant<int, 0>{});
+  f(std::integral_constant<int, 1>{});
+  f(std::integral_constant<int, 2>{});
+  f(std::integral_constant<int, 3>{});
+}
+
 template <int N>
 __device__ __forceinline__ void wait_lgkm_pin(i32x4 (&f)[N]) {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -194,11 +217,40 @@ __device__ __forceinline__ void wait_lgkm_pin(i32x4 (&f)[N]) {
   for (int i = 0; i < N; ++i) asm volatile("" : "+v"(f[i]));
 }
 
-template <typename T, bool kSwiGLU, bool kRowScale>
-__global__ __attribute__((amdgpu_flat_work_group_size(kThreads, kThreads),
-                          amdgpu_waves_per_eu(2, 2))) void
-gemm_dma_kernel(const T* __restrict__ A, const T* __restrict__ B, const T* __restrict__ B2,
-                  T* __restrict__ C, Problem p) {
+// Sources of the DMA instructions a wave issues per tile: src for full tiles, last for the
+// operand's last tile, of which kv K columns (or k-rows) lie inside K. A tile's offset travels
+// in soffset, which the buffer range check does not cover, so lanes past kv must read nothing
+// (kOob) on their own. K % 8 == 0 wherever K is contiguous, so a lane's chunk is wholly inside
+// or outside.
+//
+// 64-wide tile of a K-contiguous operand, instruction x (0..3): rows 8 (4 wave + x) .. +7,
+// eight lanes per 128-byte row; each lane fetches the chunk that belongs at its LDS slot.
+__device__ __forceinline__ void wide_source(int x, int wave, int lane, int row0, int rows, int ld,
+                                            int kv, uint32_t& src, uint32_t& last) {
+  const int r = (wave * 4 + x) * 8 + (lane >> 3);
+  const int c = (lane & 7) ^ a_swz(r);
+  src = (row0 + r < rows) ? uint32_t((row0 + r) * ld + c * 8) * 2u : kOob;
+  last = c * 8 < kv ? src : kOob;
+}
+
+// 32-wide tile of an operand stored by k-rows, instruction i (0, 1): two k-rows of 512 B.
+__device__ __forceinline__ void krow_source(int i, int wave, int lane, int col0, int cols, int ld,
+                                            int kv, uint32_t& src, uint32_t& last) {
+  const int kr = (wave * 2 + i) * 2 + (lane >> 5);
+  const int slot = lane & 31;
+  const int chunk = (((slot >> 1) ^ b_swz(kr)) << 1) | (slot & 1);
+  src = (col0 + chunk * 8 < cols) ? uint32_t(kr * ld + col0 + chunk * 8) * 2u : kOob;
+  last = kr < kv ? src : kOob;
+}
+
+// One 256 x 256 tile (256 x 128 of Y with kSwiGLU). kKTail: K need not be a multiple of 32.
+template <typename T, Layout kLayout, bool kKTail, bool kSwiGLU, bool kRowScale>
+__device__ __forceinline__ void gemm_tile_256(const T* __restrict__ A, const T* __restrict__ B,
+                                              const T* __restrict__ B2, T* __restrict__ C,
+                                              const Problem& p) {
+  constexpr bool kARows = kLayout == Layout::TN;  // A stored by k-rows [K][M]
+  constexpr bool kBWide = kLayout == Layout::NT;  // B stored K-contiguous [N][K]
+  constexpr int kBRing = kARows ? kBStages * kOperandBytes : kAStages * kABytes;
   constexpr int kTileN = kSwiGLU ? 128 : BN;
   constexpr int kRowB = kSwiGLU ? 256 : 512;
   __shared__ __attribute__((aligned(1024))) char lds[kLdsBytes];
@@ -226,82 +278,109 @@ gemm_dma_kernel(const T* __restrict__ A, const T* __restrict__ B, const T* __res
   const int ldb = up_half ? p.ldb2 : p.ldb;
   const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_void*)lds;
 
-  // A DMA x (0..3) of a 64-wide K tile: rows 8 (4 wave + x) .. +7, eight lanes per 128-byte
-  // row; each lane fetches the chunk that belongs at its LDS slot.
-  // a_last: the same sources for the last 64-wide tile when only its first 32 columns lie
-  // inside K (kt odd): lanes whose chunk falls in the second half read nothing. The tile's
-  // offset travels in soffset, which the buffer range check does not cover, so without
-  // this the last row of A would be read up to 64 bytes past its end.
-  uint32_t a_src[4], a_last[4], b_src[2];
+  const int kt = (p.k + BK - 1) / BK;  // 32-wide K tiles
+  const int kt64 = (kt + 1) / 2;       // 64-wide K tiles (the last one half used when kt is odd)
+  const int kv64 = p.k - (kt64 - 1) * 64, kv32 = p.k - (kt - 1) * 32;
+  constexpr int kADma = kARows ? 2 : 4, kBDma = kBWide ? 4 : 2;
+  uint32_t a_src[kADma], a_last[kADma], b_src[kBDma], b_last[kBDma];
 #pragma unroll
-  for (int x = 0; x < 4; ++x) {
-    const int r = (wave * 4 + x) * 8 + (lane >> 3);
-    const int c = (lane & 7) ^ a_swz(r);
-    a_src[x] = (m0 + r < p.m) ? uint32_t((m0 + r) * p.lda + c * 8) * 2u : kOob;
-    a_last[x] = c < 4 ? a_src[x] : kOob;
+  for (int x = 0; x < kADma; ++x) {
+    if constexpr (kARows)
+      krow_source(x, wave, lane, m0, p.m, p.lda, kv32, a_src[x], a_last[x]);
+    else
+      wide_source(x, wave, lane, m0, p.m, p.lda, kv64, a_src[x], a_last[x]);
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < kBDma; ++i) {
     if constexpr (kSwiGLU) {
       const int L = wave * 2 + i;
       const int kr = 4 * (L & 7) + (lane >> 4);
       const int slot = lane & 15;
       const int chunk = (((slot >> 1) ^ b_swz(kr)) << 1) | (slot & 1);
       b_src[i] = (n0 + chunk * 8 < p.n) ? uint32_t(kr * ldb + n0 + chunk * 8) * 2u : kOob;
+    } else if constexpr (kBWide) {
+      wide_source(i, wave, lane, n0, p.n, ldb, kv64, b_src[i], b_last[i]);
     } else {
-      const int kr = (wave * 2 + i) * 2 + (lane >> 5);
-      const int slot = lane & 31;
-      const int chunk = (((slot >> 1) ^ b_swz(kr)) << 1) | (slot & 1);
-      b_src[i] = (n0 + chunk * 8 < p.n) ? uint32_t(kr * ldb + n0 + chunk * 8) * 2u : kOob;
+      krow_source(i, wave, lane, n0, p.n, ldb, kv32, b_src[i], b_last[i]);
     }
   }
-  const uint32_t b_tile_bytes = uint32_t(BK * ldb) * 2u;
-  const int kt = p.k / BK;      // 32-wide K tiles
-  const int kt64 = (kt + 1) / 2;  // 64-wide A tiles (the last one half used when kt is odd)
+  const uint32_t a_tile_bytes = kARows ? uint32_t(BK * p.lda) * 2u : 128u;
+  const uint32_t b_tile_bytes = kBWide ? 128u : uint32_t(BK * ldb) * 2u;
 
   float row_scale = 0.f;
   if constexpr (kRowScale)
     if (threadIdx.x < BM) row_scale = p.row_scale[min(m0 + (int)threadIdx.x, p.m - 1)];
 
   // Tiles past the end reload the last one into a stage that is never read, keeping every
-  // step's DMA count constant.
-  const int half_tile = (kt & 1) ? kt64 - 1 : kt64;  // index of a half-used A tile, if any
-  auto dma_a = [&](int x, int tile, int slot) {
-    tile = min(tile, kt64 - 1);
+  // step's DMA count constant. `stage`: the stage's byte offset in the operand's ring.
+  auto dma_a = [&](int x, int tile, int stage) {
+    const int end = (kARows ? kt : kt64) - 1;
+    tile = min(tile, end);
+    const bool last = tile == end && (!kARows || kKTail);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        ra, (lds_void*)(lds + slot * kABytes + (wave * 4 + x) * 1024), 16,
-        tile == half_tile ? a_last[x] : a_src[x], tile * 128, 0, 0);
+        ra, (lds_void*)(lds + stage + (wave * kADma + x) * 1024), 16,
+        last ? a_last[x] : a_src[x], tile * a_tile_bytes, 0, 0);
   };
-  auto dma_b = [&](int x, int tile, int slot) {
-    tile = min(tile, kt - 1);
+  auto dma_b = [&](int x, int tile, int stage) {
+    const int end = (kBWide ? kt64 : kt) - 1;
+    tile = min(tile, end);
+    const bool last = tile == end && (kBWide || kKTail);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        rb, (lds_void*)(lds + kBRing + slot * kOperandBytes + (wave * 2 + x) * 1024), 16,
-        b_src[x], tile * b_tile_bytes, 0, 0);
+        rb, (lds_void*)(lds + kBRing + stage + (wave * kBDma + x) * 1024), 16,
+        last ? b_last[x] : b_src[x], tile * b_tile_bytes, 0, 0);
   };
 
   // A: row wm + l16 (+16 per row tile), chunk lg (first 32-wide half of the 64-wide tile)
   // or 4 + lg (second half), swizzled (a_swz reads only the row's low four bits, the same
   // for every row tile). B: k-rows 8 lg + (l16 >> 2) (+4), columns of N tile j starting at
-  // 4 (l16 & 3).
-  const uint32_t a_addr0 = (wm + l16) * 128 + ((lg ^ a_swz(l16)) * 16);
-  const uint32_t a_addr1 = (wm + l16) * 128 + (((4 + lg) ^ a_swz(l16)) * 16);
-  uint32_t b_addr[4];
+  // 4 (l16 & 3). A by k-rows is read like B, a wide B like A.
+  uint32_t a_addr0, a_addr1, b_addr[4];
   {
     const int jj = l16 >> 2, q = l16 & 3;
     const int kr = 8 * lg + jj;
     const int sw = b_swz(kr);
+    if constexpr (kARows) {
+      // Row tile I's granule is (wm / 16 + I) ^ sw; wm / 16 is a multiple of 8, so I flips
+      // address bits 5..7 (read_a_frag).
+      a_addr0 = a_addr1 = kr * 512 + (((wm / 16) ^ sw) * 32) + q * 8;
+    } else {
+      a_addr0 = (wm + l16) * 128 + ((lg ^ a_swz(l16)) * 16);
+      a_addr1 = (wm + l16) * 128 + (((4 + lg) ^ a_swz(l16)) * 16);
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       if constexpr (kSwiGLU) {
         // N tiles 0, 1: gate columns 32 (wave & 3) + 16 j; tiles 2, 3: the same up columns.
         const int g = 2 * (wave & 3) + (j & 1);
         b_addr[j] = (j >> 1) * 8192 + kr * 256 + ((g ^ sw) * 32) + q * 8;
+      } else if constexpr (kBWide) {
+        b_addr[j] = (wn + l16) * 128 + ((((j & 1) * 4 + lg) ^ a_swz(l16)) * 16);  // [half]
       } else {
         const int g = wn / 16 + j;
         b_addr[j] = kr * 512 + ((g ^ sw) * 32) + q * 8;
       }
     }
   }
+  // Where the reads of half H of the A stage at LDS offset `stage` start, and row tile I's
+  // fragment from there. The start is formed ahead of the pinned MFMA sequence.
+  auto a_base = [&](auto half, uint32_t stage) {
+    return lds_base + stage + (kARows ? 0 : decltype(half)::value ? a_addr1 : a_addr0);
+  };
+  auto read_a_frag = [&](auto tile, uint32_t base) {
+    constexpr int I = decltype(tile)::value;
+    if constexpr (kARows)
+      return read_b<512>(base + (a_addr0 ^ (I << 5)));
+    else
+      return read_a<I>(base);
+  };
+  // N tile J's fragment of the B stage at `base` (64-wide half H of a wide B).
+  auto read_b_frag = [&](auto tile, auto half, uint32_t base) {
+    constexpr int J = decltype(tile)::value;
+    if constexpr (kBWide)
+      return read_a<J>(base + b_addr[decltype(half)::value]);
+    else
+      return read_b<kRowB>(base + b_addr[J]);
+  };
 
   f32x4 acc[8][4];
 #pragma unroll
@@ -309,7 +388,7 @@ gemm_dma_kernel(const T* __restrict__ A, const T* __restrict__ B, const T* __res
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // DMA schedule. 32-wide step t issues B tile t + 3 (two instructions per wave) into B
+  // DMA schedule (NN). 32-wide step t issues B tile t + 3 (two instructions per wave) into B
   // stage (t + 3) % 4 and, when t is odd, the 64-wide A tile (t + 3) / 2 (four per wave)
   // into A stage ((t + 3) / 2) % 3. A stage reuse: A tile v's last fragments (rows 4-7 of
   // step 2v + 1) are read in the first half of step 2v + 1 and waited for after that step's
@@ -319,84 +398,105 @@ gemm_dma_kernel(const T* __restrict__ A, const T* __restrict__ B, const T* __res
   // the stage in step t + 1. Step t's barrier needs 32-wide tile t + 1 landed, issued in
   // step t - 2 or earlier, so each wave waits until at most the 8 instructions of steps
   // t - 1 and t are in flight. The prologue is steps -3 .. -1 of the same schedule.
-  dma_a(0, 0, 0); dma_a(1, 0, 0); dma_a(2, 0, 0); dma_a(3, 0, 0);
-  dma_b(0, 0, 0); dma_b(1, 0, 0);
-  dma_b(0, 1, 1); dma_b(1, 1, 1);
-  dma_a(0, 1, 1); dma_a(1, 1, 1); dma_a(2, 1, 1); dma_a(3, 1, 1);
-  dma_b(0, 2, 2); dma_b(1, 2, 2);
+  //
+  // TN. A comes by k-rows in a ring like B's. Its tile t's last fragments (rows 4-7) are
+  // waited for after the barrier of step t, so the refill of that stage (tile t + 4) is
+  // issued in the second half of step t + 1, after the next barrier. At the barrier of step
+  // t, tile t + 1 of both must have landed: A's was issued in the second half of step t - 2,
+  // and B t + 2, A t + 2 and B t + 3 (6 instructions) came after it.
+  //
+  // NT. B comes in 64-wide tiles, two stages. Tile v's last fragments (step 2v + 1's, read in
+  // the second half of step 2v) are waited for at the start of step 2v + 1, so tile v + 2
+  // refills the stage in the second half of step 2v + 1, two steps before the barrier that
+  // publishes it (step 2v + 3's, where only A tile v + 3's 4 instructions may be in flight).
+  constexpr int kAStage = kARows ? kOperandBytes : kABytes;
+  constexpr int kBStage = kBWide ? kABytes : kOperandBytes;
+  auto tile_a = [&](int tile) {
+#pragma unroll
+    for (int x = 0; x < kADma; ++x) dma_a(x, tile, tile * kAStage);
+  };
+  auto tile_b = [&](int tile) {
+#pragma unroll
+    for (int x = 0; x < kBDma; ++x) dma_b(x, tile, tile * kBStage);
+  };
+  if constexpr (kARows) {
+    tile_b(0); tile_a(0); tile_b(1); tile_a(1); tile_b(2); tile_a(2);
+  } else if constexpr (kBWide) {
+    tile_a(0); tile_b(0); tile_a(1); tile_b(1);
+  } else {
+    tile_a(0); tile_b(0); tile_b(1); tile_a(1); tile_b(2);
+  }
   wait_vmcnt<8>();
   barrier_no_fence();
 
+  using Half0 = std::integral_constant<int, 0>;
+  using Half1 = std::integral_constant<int, 1>;
   i32x4 a_lo[4], a_hi[4], b0[4], b1[4];
-  a_lo[0] = read_a<0>(lds_base + a_addr0);
-  a_lo[1] = read_a<1>(lds_base + a_addr0);
-  a_lo[2] = read_a<2>(lds_base + a_addr0);
-  a_lo[3] = read_a<3>(lds_base + a_addr0);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) b0[j] = read_b<kRowB>(lds_base + kBRing + b_addr[j]);
+  unroll4([&](auto i) {
+    constexpr int x = decltype(i)::value;
+    a_lo[x] = read_a_frag(i, a_base(Half0{}, 0));
+    b0[x] = read_b_frag(i, Half0{}, lds_base + kBRing);
+  });
 
-  // One 32-wide step t (half H of the 64-wide A tile in A stage sa; B stage sb). Bc holds
-  // this step's B fragments, Bn receives the next step's. The next step reads A stage
-  // sa_next (the same stage when H == 0) and B stage sb_next.
-  auto step = [&](auto half, int t, int sa, int sa_next, int sb, int sb_next, i32x4 (&Bc)[4],
+  // One 32-wide step t, half H of 64-wide K tile u = t / 2. `ao` is the tile's stage in a
+  // 64-wide A ring, `ao_next` the next tile's, `ao_fill` the third one; `bo` is the stage of
+  // step 2u in a 32-wide ring (0 or 2 stages in, so the others are XORs away) or of tile u in
+  // the two-stage 64-wide B ring. All are byte offsets. Bc holds this step's B fragments, Bn
+  // receives the next step's.
+  auto step = [&](auto half, int t, int ao, int ao_next, int ao_fill, int bo, i32x4 (&Bc)[4],
                   i32x4 (&Bn)[4]) {
     constexpr int H = decltype(half)::value;
-    const uint32_t a_cur = lds_base + sa * kABytes + (H ? a_addr1 : a_addr0);
-    const uint32_t a_next = lds_base + sa_next * kABytes + (H ? a_addr0 : a_addr1);
-    const uint32_t b_next = lds_base + kBRing + sb_next * kOperandBytes;
-    // Refill targets: B stage (t + 3) % 4 == (sb + 3) % 4, A stage of tile (t + 3) / 2.
-    const int fill_b = sb == 0 ? 3 : sb - 1;
-    const int fill_a = sa == 0 ? 2 : sa - 1;
+    using Next = std::integral_constant<int, 1 - H>;
+    const int rows_cur = H ? bo ^ kOperandBytes : bo;
+    const int rows_next = H ? bo ^ 2 * kOperandBytes : bo ^ kOperandBytes;
+    const int rows_fill = H ? bo : bo ^ 3 * kOperandBytes;  // stage (t + 3) % 4
+    const int wide_next = H ? bo ^ kABytes : bo;
+    const uint32_t a_cur = a_base(half, kARows ? rows_cur : ao);
+    const uint32_t a_next = a_base(Next{}, kARows ? rows_next : H ? ao_next : ao);
+    const uint32_t b_next = lds_base + kBRing + (kBWide ? wide_next : rows_next);
     wait_lgkm_pin(a_lo);
     wait_lgkm_pin(Bc);
     sched_fence();
     // Rows 0-3; read rows 4-7 of this step, issue the DMA.
-#pragma unroll
-    for (int x = 0; x < 16; ++x) {
-      const int i = x >> 2, j = x & 3;
-      acc[i][j] = Mfma<T>::run(Bc[j], a_lo[i], acc[i][j]);
-      sched_fence();
-      if (j == 0) {
-        if (i == 0) a_hi[0] = read_a<4>(a_cur);
-        if (i == 1) a_hi[1] = read_a<5>(a_cur);
-        if (i == 2) a_hi[2] = read_a<6>(a_cur);
-        if (i == 3) a_hi[3] = read_a<7>(a_cur);
-      }
-      if (H == 1 && j == 1) dma_a(i, (t + 3) >> 1, fill_a);
-      if (j == 3 && (i & 1) == 0) dma_b(i >> 1, t + 3, fill_b);
-      sched_fence();
-    }
-    wait_vmcnt<8>();
+    unroll4([&](auto row) {
+      unroll4([&](auto col) {
+        constexpr int i = decltype(row)::value, j = decltype(col)::value;
+        acc[i][j] = Mfma<T>::run(Bc[j], a_lo[i], acc[i][j]);
+        sched_fence();
+        if constexpr (j == 0)
+          a_hi[i] = read_a_frag(std::integral_constant<int, 4 + i>{}, a_cur);
+        if constexpr (!kARows && H == 1 && j == 1) dma_a(i, (t + 3) >> 1, ao_fill);
+        if constexpr (!kBWide && j == 3 && (i & 1) == 0) dma_b(i >> 1, t + 3, rows_fill);
+        sched_fence();
+      });
+    });
+    wait_vmcnt<kARows ? 6 : kBWide && H == 1 ? 4 : 8>();
     barrier_no_fence();
     wait_lgkm_pin(a_hi);
     sched_fence();
     // Rows 4-7; read rows 0-3 and B of step t + 1.
-#pragma unroll
-    for (int x = 0; x < 16; ++x) {
-      const int i = x >> 2, j = x & 3;
-      acc[4 + i][j] = Mfma<T>::run(Bc[j], a_hi[i], acc[4 + i][j]);
-      sched_fence();
-      if (j == 0) {
-        if (i == 0) a_lo[0] = read_a<0>(a_next);
-        if (i == 1) a_lo[1] = read_a<1>(a_next);
-        if (i == 2) a_lo[2] = read_a<2>(a_next);
-        if (i == 3) a_lo[3] = read_a<3>(a_next);
-      }
-      if (j == 2) Bn[i] = read_b<kRowB>(b_next + b_addr[i]);
-      sched_fence();
-    }
+    unroll4([&](auto row) {
+      unroll4([&](auto col) {
+        constexpr int i = decltype(row)::value, j = decltype(col)::value;
+        acc[4 + i][j] = Mfma<T>::run(Bc[j], a_hi[i], acc[4 + i][j]);
+        sched_fence();
+        if constexpr (j == 0) a_lo[i] = read_a_frag(row, a_next);
+        if constexpr (kARows && j == 1 && (i & 1) == 0) dma_a(i >> 1, t + 3, rows_fill);
+        if constexpr (j == 2) Bn[i] = read_b_frag(row, Next{}, b_next);
+        if constexpr (kBWide && H == 1 && j == 3) dma_b(i, (t + 3) >> 1, bo);
+        sched_fence();
+      });
+    });
   };
 
-  // 64-wide A tile u: steps 2u (B stage sb) and 2u + 1 (sb + 1), A stage sa.
-  int sa = 0, sb = 0;
+  int ao = 0, bo = 0;
   for (int u = 0; 2 * u < kt; ++u) {
-    const int sa_next = sa == kAStages - 1 ? 0 : sa + 1;
-    step(std::integral_constant<int, 0>{}, 2 * u, sa, sa, sb, sb + 1, b0, b1);
-    if (2 * u + 1 < kt)
-      step(std::integral_constant<int, 1>{}, 2 * u + 1, sa, sa_next, sb + 1,
-           sb + 2 == kBStages ? 0 : sb + 2, b1, b0);
-    sa = sa_next;
-    sb = sb + 2 == kBStages ? 0 : sb + 2;
+    const int ao_next = ao == (kAStages - 1) * kABytes ? 0 : ao + kABytes;
+    const int ao_fill = 3 * kABytes - ao - ao_next;
+    step(Half0{}, 2 * u, ao, ao_next, ao_fill, bo, b0, b1);
+    if (2 * u + 1 < kt) step(Half1{}, 2 * u + 1, ao, ao_next, ao_fill, bo, b1, b0);
+    ao = ao_next;
+    bo ^= kBWide ? kABytes : 2 * kOperandBytes;
   }
   wait_vmcnt<0>();
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -452,8 +552,8 @@ gemm_dma_kernel(const T* __restrict__ A, const T* __restrict__ B, const T* __res
                         (uint32_t(__builtin_bit_cast(uint16_t, tk::from_f32<T>(v[3]))) << 16);
     return uint2{lo, hi};
   };
-  const bool rows16 =
-      p.scn == 1 && (p.scm & 7) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
+  const bool rows16 = p.scn == 1 && (p.n & 7) == 0 && (p.scm & 7) == 0 &&
+                      (reinterpret_cast<uintptr_t>(C) & 15) == 0;
   if (rows16) {
     // Stage rows of kTileN values at a stride of kTileN * 2 + 16 bytes (4 dwords past a
     // multiple of the 64 banks), so the 16 rows x 2 lane groups of an 8-byte write phase hit
@@ -477,12 +577,13 @@ gemm_dma_kernel(const T* __restrict__ A, const T* __restrict__ B, const T* __res
     }
     return;
   }
-  const bool vec = p.scn == 1 && (p.scm & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 7) == 0;
+  const bool vec = p.scn == 1 && (p.n & 3) == 0 && (p.scm & 3) == 0 &&
+                   (reinterpret_cast<uintptr_t>(C) & 7) == 0;
   for_each_out([&](int r, int c, const float (&v)[4]) {
     const int m = m0 + r, n = n0 + c;
     if (m >= p.m || n >= p.n) return;
     T* dst = C + m * p.scm + n * p.scn;
-    if (vec) {  // p.n % 8 == 0, so n .. n+3 are in range
+    if (vec) {  // p.n % 4 == 0, so n .. n+3 are in range
       *reinterpret_cast<uint2*>(dst) = pack4(v);
     } else {
 #pragma unroll
@@ -492,64 +593,120 @@ gemm_dma_kernel(const T* __restrict__ A, const T* __restrict__ B, const T* __res
   });
 }
 
+// Row-major operands with K % 32 == 0 (NN), and the fused variants.
+template <typename T, bool kSwiGLU, bool kRowScale>
+__global__ __attribute__((amdgpu_flat_work_group_size(kThreads, kThreads),
+                          amdgpu_waves_per_eu(2, 2))) void
+gemm_dma_kernel(const T* __restrict__ A, const T* __restrict__ B, const T* __restrict__ B2,
+                T* __restrict__ C, Problem p) {
+  gemm_tile_256<T, Layout::NN, false, kSwiGLU, kRowScale>(A, B, B2, C, p);
+}
+
+// Transposed operands and K % 32 != 0.
+template <typename T, Layout kLayout>
+__global__ __attribute__((amdgpu_flat_work_group_size(kThreads, kThreads),
+                          amdgpu_waves_per_eu(2, 2))) void
+gemm_kernel(const T* __restrict__ A, const T* __restrict__ B, T* __restrict__ C, Problem p) {
+  gemm_tile_256<T, kLayout, true, false, false>(A, B, B, C, p);
+}
 
 }  // namespace
 
 namespace tk {
 
+namespace gemm_dma {
+
+bool plan(const void* a, const void* b, int64_t m, int64_t n, int64_t k, int64_t stride_am,
+          int64_t stride_ak, int64_t stride_bk, int64_t stride_bn, Plan* plan) {
+  // Buffer offsets are 32-bit with kOob (2^31) reserved as "outside"; strides are positive (the
+  // offsets are unsigned). An operand is stored as `rows` rows of `cols` contiguous values.
+  if (m <= 0 || n <= 0 || k <= 0 || stride_am <= 0 || stride_ak <= 0 || stride_bk <= 0 ||
+      stride_bn <= 0)
+    return false;
+  auto stored = [](const void* p, int64_t rows, int64_t cols, int64_t row_stride,
+                   int64_t col_stride) {
+    return col_stride == 1 && cols % 8 == 0 && row_stride % 8 == 0 && aligned16(p) &&
+           (extent(rows, row_stride, 1, 0) + cols) * 2 < int64_t(kOob);
+  };
+  const bool a_k = stored(a, m, k, stride_am, stride_ak);  // [M][K]
+  const bool a_m = stored(a, k, m, stride_ak, stride_am);  // [K][M]
+  const bool b_n = stored(b, k, n, stride_bk, stride_bn);  // [K][N]
+  const bool b_k = stored(b, n, k, stride_bn, stride_bk);  // [N][K]
+  if (a_k && b_n)
+    *plan = {Layout::NN, false, k % BK != 0, stride_am, stride_bk};
+  else if (a_k && b_k)
+    *plan = {Layout::NT, false, true, stride_am, stride_bn};
+  else if (a_m && b_n)
+    *plan = {Layout::TN, false, true, stride_ak, stride_bk};
+  else if (a_m && b_k)  // C^T = B^T A^T, both row-major
+    *plan = {Layout::NN, true, true, stride_bn, stride_ak};
+  else
+    return false;
+  return true;
+}
+
+}  // namespace gemm_dma
+
 bool gemm_dma_applies(const void* a, const void* b, int64_t m, int64_t n, int64_t k,
                       int64_t stride_am, int64_t stride_ak, int64_t stride_bk,
                       int64_t stride_bn) {
-  // Buffer offsets are 32-bit with kOob (2^31) reserved as "outside"; row strides are
-  // positive (the offsets are unsigned).
-  if (m <= 0 || n <= 0 || k <= 0 || stride_am <= 0 || stride_bk <= 0) return false;
-  const __int128 a_bytes = (extent(m, stride_am, 1, 0) + k) * 2;
-  const __int128 b_bytes = (extent(k, stride_bk, 1, 0) + n) * 2;
-  return stride_ak == 1 && stride_bn == 1 && k % BK == 0 && n % 8 == 0 && stride_am % 8 == 0 &&
-         stride_bk % 8 == 0 && aligned16(a) && aligned16(b) && a_bytes < int64_t(kOob) &&
-         b_bytes < int64_t(kOob);
+  gemm_dma::Plan p;
+  return gemm_dma::plan(a, b, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, &p) &&
+         p.layout == gemm_dma::Layout::NN && !p.swap && !p.k_tail;
 }
 
-void gemm_dma_launch(int dtype, const void* a, const void* b, void* c, int64_t m, int64_t n,
-                     int64_t k, int64_t stride_am, int64_t stride_bk, int64_t stride_cm,
-                     int64_t stride_cn, hipStream_t stream, const float* row_scale) {
-  const uint32_t b_bytes = (uint32_t)(((k - 1) * stride_bk + n) * 2);
+namespace {
+
+template <typename T>
+void launch_256(const gemm_dma::Plan& plan, const void* a, const void* b, void* c,
+                const Problem& p, hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n)), block(kThreads);
+  const T* pa = static_cast<const T*>(a);
+  const T* pb = static_cast<const T*>(b);
+  T* pc = static_cast<T*>(c);
+  if (p.row_scale != nullptr)
+    hipLaunchKernelGGL((gemm_dma_kernel<T, false, true>), grid, block, 0, stream, pa, pb, pb, pc, p);
+  else if (plan.layout == Layout::NN && !plan.k_tail)
+    hipLaunchKernelGGL((gemm_dma_kernel<T, false, false>), grid, block, 0, stream, pa, pb, pb, pc, p);
+  else if (plan.layout == Layout::NN)
+    hipLaunchKernelGGL((gemm_kernel<T, Layout::NN>), grid, block, 0, stream, pa, pb, pc, p);
+  else if (plan.layout == Layout::NT)
+    hipLaunchKernelGGL((gemm_kernel<T, Layout::NT>), grid, block, 0, stream, pa, pb, pc, p);
+  else
+    hipLaunchKernelGGL((gemm_kernel<T, Layout::TN>), grid, block, 0, stream, pa, pb, pc, p);
+}
+
+}  // namespace
+
+void gemm_dma_launch(const gemm_dma::Plan& plan, int dtype, const void* a, const void* b, void* c,
+                     int64_t m, int64_t n, int64_t k, int64_t stride_cm, int64_t stride_cn,
+                     hipStream_t stream, const float* row_scale) {
+  if (plan.swap) {
+    std::swap(a, b);
+    std::swap(m, n);
+    std::swap(stride_cm, stride_cn);
+  }
+  const int64_t a_rows = plan.layout == Layout::TN ? k : m, a_cols = plan.layout == Layout::TN ? m : k;
+  const int64_t b_rows = plan.layout == Layout::NT ? n : k, b_cols = plan.layout == Layout::NT ? k : n;
+  const uint32_t b_bytes = (uint32_t)(((b_rows - 1) * plan.ldb + b_cols) * 2);
   Problem p{(int)m,
             (int)n,
             (int)k,
-            (int)stride_am,
-            (int)stride_bk,
-            (int)stride_bk,
+            (int)plan.lda,
+            (int)plan.ldb,
+            (int)plan.ldb,
             stride_cm,
             stride_cn,
             (int)cdiv(m, BM),
             (int)cdiv(n, BN),
-            (uint32_t)(((m - 1) * stride_am + k) * 2),
+            (uint32_t)(((a_rows - 1) * plan.lda + a_cols) * 2),
             b_bytes,
             b_bytes,
             row_scale};
-  const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n));
-  if (dtype == TK_DTYPE_F16) {
-    using T = _Float16;
-    if (row_scale != nullptr)
-      hipLaunchKernelGGL((gemm_dma_kernel<T, false, true>), grid, dim3(kThreads), 0, stream,
-                         static_cast<const T*>(a), static_cast<const T*>(b),
-                         static_cast<const T*>(b), static_cast<T*>(c), p);
-    else
-      hipLaunchKernelGGL((gemm_dma_kernel<T, false, false>), grid, dim3(kThreads), 0, stream,
-                         static_cast<const T*>(a), static_cast<const T*>(b),
-                         static_cast<const T*>(b), static_cast<T*>(c), p);
-  } else {
-    using T = __bf16;
-    if (row_scale != nullptr)
-      hipLaunchKernelGGL((gemm_dma_kernel<T, false, true>), grid, dim3(kThreads), 0, stream,
-                         static_cast<const T*>(a), static_cast<const T*>(b),
-                         static_cast<const T*>(b), static_cast<T*>(c), p);
-    else
-      hipLaunchKernelGGL((gemm_dma_kernel<T, false, false>), grid, dim3(kThreads), 0, stream,
-                         static_cast<const T*>(a), static_cast<const T*>(b),
-                         static_cast<const T*>(b), static_cast<T*>(c), p);
-  }
+  if (dtype == TK_DTYPE_F16)
+    launch_256<_Float16>(plan, a, b, c, p, stream);
+  else
+    launch_256<__bf16>(plan, a, b, c, p, stream);
 }
 
 void gemm_swiglu_dma_launch(int dtype, const void* a, const void* b_gate, const void* b_up,

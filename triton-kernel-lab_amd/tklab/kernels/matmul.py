@@ -6,12 +6,14 @@ int32 range, float16 (and here also bfloat16) inputs, a contiguous output of
 the input dtype. Validation order and messages follow ``matmul.py:167-186``.
 
 The reference autotunes 25 Triton configurations per shape
-(``matmul.py:23-75``); this build has a static choice between two kernels and
-reports the one a shape launches in the same metadata keys: row-major operands
-with K % 32 == 0 (every registry shape) take ``gemm_dma_kernel`` (256 x 256
-tiles, K step 32, eight wave64s, buffer->LDS rings of four 32-wide B stages and
-three 64-wide A stages, ``v_mfma_f32_16x16x32``); strided operands or other K take the register-staged
-``gemm_kernel`` (256 x 256 x 64, four wave64s, ``v_mfma_f32_32x32x16``).
+(``matmul.py:23-75``); this build picks a kernel from the operands' layout and
+reports it in the same metadata keys. Operands whose rows are 16-byte aligned and
+multiples of 8 elements long, each row-major or transposed, take buffer->LDS DMA
+kernels (256 x 256 tiles, K step 32, eight wave64s, ``v_mfma_f32_16x16x32``):
+``gemm_dma_kernel`` for row-major operands with K % 32 == 0 (every registry shape),
+``gemm_kernel`` for transposed ones (a linear layer's gradients) and other K.
+Every other layout takes the register-staged ``gemm_kernel`` (256 x 256 x 64, four
+wave64s, ``v_mfma_f32_32x32x16``).
 ``matmul_fp16acc`` keeps its registry entry, but gfx950 MFMA
 accumulates f16 products in float32 only, so both entry points run the same
 FP32-accumulate kernel (its result is at least as accurate as an FP16
@@ -41,6 +43,8 @@ _DTYPES = (torch.float16, torch.bfloat16)
 # (the B operand's; A is loaded in 64-wide tiles into a ring of kAStages = 3).
 TILE = {"hip_kernel": "gemm_dma_kernel", "block_m": 256, "block_n": 256, "block_k": 32, "group_m": 4,
         "num_warps": 8, "num_stages": 4}
+# The same tiles on transposed operands or with K % 32 != 0.
+TRANSPOSED_TILE = {**TILE, "hip_kernel": "gemm_kernel"}
 _MFMA = {
     torch.float16: "v_mfma_f32_16x16x32_f16",
     torch.bfloat16: "v_mfma_f32_16x16x32_bf16",
@@ -54,29 +58,29 @@ _FALLBACK_MFMA = {
 }
 
 
+def _dma_rows(t: torch.Tensor) -> bool:
+    """Rows the DMA kernels can load: unit inner stride, whole aligned 16-byte groups, < 2 GiB."""
+    rows, cols = t.shape
+    return (
+        t.stride(1) == 1
+        and cols % 8 == 0
+        and t.stride(0) % 8 == 0
+        and t.data_ptr() % 16 == 0
+        and ((rows - 1) * t.stride(0) + cols) * 2 < 2**31
+    )
+
+
 def launch_config(a: torch.Tensor, b: torch.Tensor) -> dict[str, BenchmarkScalar]:
     """Tile configuration and MFMA of the kernel ``tk_gemm`` launches for ``a @ b``.
 
-    Mirrors ``gemm_dma_applies`` (csrc/gemm_dma.hip): unit column strides, K % 32 == 0,
-    N and both row strides multiples of 8, 16-byte aligned bases and operand extents
-    under 2 GiB take the DMA kernel.
+    Mirrors ``gemm_dma::plan`` (csrc/gemm_dma.hip).
     """
-    (m, k), n = a.shape, b.shape[1]
-    dma = (
-        a.stride(1) == 1
-        and b.stride(1) == 1
-        and k % 32 == 0
-        and n % 8 == 0
-        and a.stride(0) % 8 == 0
-        and b.stride(0) % 8 == 0
-        and a.data_ptr() % 16 == 0
-        and b.data_ptr() % 16 == 0
-        and ((m - 1) * a.stride(0) + k) * 2 < 2**31
-        and ((k - 1) * b.stride(0) + n) * 2 < 2**31
-    )
-    if dma:
-        return {**TILE, "mma_opcode": _MFMA.get(a.dtype, _MFMA[torch.float16])}
-    return {**FALLBACK_TILE, "mma_opcode": _FALLBACK_MFMA.get(a.dtype, _FALLBACK_MFMA[torch.float16])}
+    if not ((_dma_rows(a) or _dma_rows(a.t())) and (_dma_rows(b) or _dma_rows(b.t()))):
+        return {**FALLBACK_TILE,
+                "mma_opcode": _FALLBACK_MFMA.get(a.dtype, _FALLBACK_MFMA[torch.float16])}
+    plain = _dma_rows(a) and _dma_rows(b) and a.shape[1] % 32 == 0
+    return {**(TILE if plain else TRANSPOSED_TILE),
+            "mma_opcode": _MFMA.get(a.dtype, _MFMA[torch.float16])}
 
 
 def _validate(a: torch.Tensor, b: torch.Tensor) -> None:
