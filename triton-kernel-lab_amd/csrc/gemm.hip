@@ -316,7 +316,7 @@ extern "C" int tk_gemm_swiglu(int dtype, const void* a, const void* b_gate, cons
       !tk::gemm_dma_applies(a, b_up, m, n, k, stride_am, stride_ak, stride_uk, stride_un))
     return tk::fail("gemm_swiglu: needs unit inner strides, 16-byte aligned rows, k %% 32 == 0, "
                     "n %% 8 == 0 and operands below 2 GiB");
-  if (tk::cdiv(m, BM) * tk::cdiv(n, 128) > INT32_MAX) return tk::fail("gemm_swiglu: too many tiles");
+  if (tk::cdiv(m, 64) * tk::cdiv(n, 64) > INT32_MAX) return tk::fail("gemm_swiglu: too many tiles");
   tk::gemm_swiglu_dma_launch(dtype, a, b_gate, b_up, y, m, n, k, stride_am, stride_gk, stride_uk,
                              stride_ym, stride_yn, tk::as_stream(stream));
   return tk::check_launch("gemm_swiglu");

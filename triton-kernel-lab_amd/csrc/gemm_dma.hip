@@ -68,25 +68,20 @@
 // the epilogue rounds both to the storage type (as the unfused GEMMs store them) and
 // writes value * gate * sigmoid(gate): the two M x N intermediates never reach HBM and
 // the result is bitwise that of the two GEMMs followed by the SwiGLU kernel.
-#include "gemm.hpp"
-#include "tk_common.hpp"
+#include "gemm_device.hpp"
+#include "gemm_tile.hpp"
 
-#include <type_traits>
-#include <utility>
+#include <algorithm>
 
-// No floating-point contraction in this file: the SwiGLU epilogue must round
-// value * gate * sigmoid(gate) to float32 and then to the storage type, as the SwiGLU
-// kernel and the reference do (a fused multiply-convert would round once).
 #pragma clang fp contract(off)
 
 namespace {
 
-using tk::gemm_dma::Layout;
+using namespace tk::gemm_dma;
 
 constexpr int BM = 256, BN = 256, BK = 32;
 constexpr int kThreads = 512;  // 8 waves
 constexpr int kGroupM = 4;
-constexpr int kXcds = 8;
 // K-contiguous operands come in 64-wide K tiles (256 rows x 128 B), the others in 32-wide K
 // tiles (32 k-rows x 512 B). NN: three 64-wide A stages and four 32-wide B stages; NT: three
 // 64-wide A and two 64-wide B stages; TN: four 32-wide stages of each. At most 160 KiB: all
@@ -95,127 +90,10 @@ constexpr int kAStages = 3, kBStages = 4;
 constexpr int kABytes = 256 * 64 * 2;        // 32 KiB per 64-wide stage
 constexpr int kOperandBytes = 256 * BK * 2;  // 16 KiB per 32-wide stage
 constexpr int kLdsBytes = kAStages * kABytes + kBStages * kOperandBytes;
-constexpr uint32_t kOob = 0x80000000u;  // past every buffer's num_records: reads as zero
 // Epilogue: the C tile is staged in the ring's LDS (at most 256 rows of 528 bytes), the row
 // scales of the row-scaled variant after it.
 constexpr int kScaleOff = 256 * 528;
 static_assert(kScaleOff + 256 * 4 <= kLdsBytes, "row scales past the LDS block");
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) void lds_void;
-
-
-struct Problem {
-  int m, n, k;
-  int lda, ldb, ldb2;  // row strides of the stored matrices; ldb2: the up weight's k stride (SwiGLU variant)
-  int64_t scm, scn;
-  int tiles_m, tiles_n;
-  uint32_t a_bytes, b_bytes, b2_bytes;
-  const float* row_scale;  // kRowScale: C[m, :] = round(row_scale[m] * acc)
-};
-
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-  // s_waitcnt fields: vmcnt[3:0], expcnt[6:4] (7 = no wait), lgkmcnt[11:8] (15 = no wait),
-  // vmcnt[5:4] at [15:14].
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
-// Workgroup barrier without the release/acquire fence __syncthreads() carries: the
-// fence would wait for every outstanding DMA, while each caller has already waited
-// for exactly the tile it is about to read.
-__device__ __forceinline__ void barrier_no_fence() { asm volatile("s_barrier" ::: "memory"); }
-
-__device__ __forceinline__ void sched_fence() { __builtin_amdgcn_sched_barrier(0); }
-
-template <int OFF>
-__device__ __forceinline__ i32x4 lds_read_b128(uint32_t addr) {
-  i32x4 r;
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "i"(OFF));
-  return r;
-}
-
-template <int OFF>
-__device__ __forceinline__ i32x2 lds_read_tr16(uint32_t addr) {
-  i32x2 r;
-  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "i"(OFF));
-  return r;
-}
-
-// Y = value * gate * sigmoid(gate) on values already rounded to T, in the SwiGLU
-// kernel's operation order (contraction off: each product rounded separately).
-template <typename T>
-__device__ __forceinline__ T swiglu_out(float gate_acc, float up_acc) {
-  const float g = tk::round_to<T>(gate_acc);
-  const float v = tk::round_to<T>(up_acc);
-  return tk::from_f32<T>(v * g * tk::stable_sigmoid(g));
-}
-
-// v_mfma_f32_16x16x32: A lane l holds row l % 16, k = 8 (l / 16) .. +7; B lane l holds
-// column l % 16, the same k; D lane l holds column l % 16, rows 4 (l / 16) .. +3.
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-template <typename T>
-struct Mfma;
-template <>
-struct Mfma<_Float16> {
-  static __device__ __forceinline__ f32x4 run(i32x4 a, i32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  }
-};
-template <>
-struct Mfma<__bf16> {
-  static __device__ __forceinline__ f32x4 run(i32x4 a, i32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  }
-};
-
-// A row swizzle (128-byte rows): 16-byte chunk c of row r sits at c ^ a_swz(r). A fragment
-// read phase takes one chunk of 16 consecutive rows: even and odd rows fall in opposite
-// halves of a 256-byte bank row, and (r >> 1) & 7 puts the 8 rows of each half on distinct
-// 16-byte slots.
-__device__ __forceinline__ int a_swz(int r) { return (r >> 1) & 7; }
-
-// B k-row swizzle: 32-byte granule g of k-row k sits at g ^ b_swz(k). A 16x16x32 B
-// fragment read phase covers two 16-lane groups reading k-rows 8 apart, so the swizzle
-// carries bit 3 of k besides the (k & 3) term that separates the 4 rows of one read.
-__device__ __forceinline__ int b_swz(int k) { return 2 * (k & 3) + ((k >> 3) & 1); }
-
-// A fragment of row tile I (16 rows = 2 KiB of the stage).
-template <int I>
-__device__ __forceinline__ i32x4 read_a(uint32_t addr) {
-  return lds_read_b128<I * 2048>(addr);
-}
-
-// B fragment: k-rows +0..3 and +4..7 of this lane group (ROWB bytes per k-row).
-template <int ROWB>
-__device__ __forceinline__ i32x4 read_b(uint32_t addr) {
-  const i32x2 lo = lds_read_tr16<0>(addr);
-  const i32x2 hi = lds_read_tr16<4 * ROWB>(addr);
-  return i32x4{lo[0], lo[1], hi[0], hi[1]};
-}
-
-// f(0) .. f(3) with compile-time indices.
-template <typename F>
-__device__ __forceinline__ void unroll4(F&& f) {
-  f(std::integral_constant<int, 0>{});
-  f(std::integral_constant<int, 1>{});
-  f(std::integral_constant<int, 2>{});
-  f(std::integral_constant<int, 3>{});
-}
-
-template <int N>
-__device__ __forceinline__ void wait_lgkm_pin(i32x4 (&f)[N]) {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(f[i]));
-}
 
 // Sources of the DMA instructions a wave issues per tile: src for full tiles, last for the
 // operand's last tile, of which kv K columns (or k-rows) lie inside K. A tile's offset travels
@@ -503,14 +381,7 @@ __device__ __forceinline__ void gemm_tile_256(const T* __restrict__ A, const T* 
 
   // acc[i][j] holds C^T: register r of lane l is C[m][n] with m = m0 + wm + 16 i + l % 16 and
   // n = n0 + (N tile j's first column) + 4 (l / 16) + r: four consecutive columns of one row.
-  // The rings are idle once every wave is here, so when C rows are 16-byte aligned the block
-  // stages its rounded tile in LDS and writes it back as whole rows, 16 bytes per lane, with
-  // non-temporal stores of full 128-byte lines; otherwise each lane stores its four columns.
-  // Staged, the epilogue of fp16 4096^3 took ~4 instead of ~8 us of a ~108 us launch (a
-  // timing-only copy without stores ran 102 us): 4096^3 108.1 -> 104.3 us, 8192^3 784 ->
-  // 773 us, the row-scaled 16384x6144x4096 GEMM 675 -> 645 us. Staged with default-policy
-  // stores: 105.1, 773 and 654 us. Per-lane non-temporal stores write 32-byte segments of
-  // four lines and were 5-14 % slower than default-policy ones.
+  // The rings are idle once every wave is here.
   __syncthreads();
   const float* scales = reinterpret_cast<const float*>(lds + kScaleOff);
   if constexpr (kRowScale) {
@@ -545,53 +416,10 @@ __device__ __forceinline__ void gemm_tile_256(const T* __restrict__ A, const T* 
       }
     }
   };
-  auto pack4 = [](const float (&v)[4]) {
-    const uint32_t lo = uint32_t(__builtin_bit_cast(uint16_t, tk::from_f32<T>(v[0]))) |
-                        (uint32_t(__builtin_bit_cast(uint16_t, tk::from_f32<T>(v[1]))) << 16);
-    const uint32_t hi = uint32_t(__builtin_bit_cast(uint16_t, tk::from_f32<T>(v[2]))) |
-                        (uint32_t(__builtin_bit_cast(uint16_t, tk::from_f32<T>(v[3]))) << 16);
-    return uint2{lo, hi};
-  };
-  const bool rows16 = p.scn == 1 && (p.n & 7) == 0 && (p.scm & 7) == 0 &&
-                      (reinterpret_cast<uintptr_t>(C) & 15) == 0;
-  if (rows16) {
-    // Stage rows of kTileN values at a stride of kTileN * 2 + 16 bytes (4 dwords past a
-    // multiple of the 64 banks), so the 16 rows x 2 lane groups of an 8-byte write phase hit
-    // distinct banks; then kTileN / 8 lanes per row copy 16 bytes each (p.n % 8 == 0, so a
-    // 16-byte group is wholly inside or outside N).
-    constexpr int kStride = kTileN * 2 + 16;
-    static_assert(BM * kStride <= kScaleOff, "staged tile overlaps the row scales");
-    for_each_out([&](int r, int c, const float (&v)[4]) {
-      *reinterpret_cast<uint2*>(lds + r * kStride + c * 2) = pack4(v);
-    });
-    __syncthreads();
-    constexpr int kLanesPerRow = kTileN / 8;
-    constexpr int kRowsPerPass = kThreads / kLanesPerRow;
-    const int cr = threadIdx.x / kLanesPerRow, cc = (threadIdx.x % kLanesPerRow) * 8;
-#pragma unroll 4
-    for (int pass = 0; pass < BM / kRowsPerPass; ++pass) {
-      const int r = pass * kRowsPerPass + cr;
-      const i32x4 v = *reinterpret_cast<const i32x4*>(lds + r * kStride + cc * 2);
-      if (m0 + r < p.m && n0 + cc < p.n)
-        __builtin_nontemporal_store(v, reinterpret_cast<i32x4*>(C + (m0 + r) * p.scm + n0 + cc));
-    }
-    return;
-  }
-  const bool vec = p.scn == 1 && (p.n & 3) == 0 && (p.scm & 3) == 0 &&
-                   (reinterpret_cast<uintptr_t>(C) & 7) == 0;
-  for_each_out([&](int r, int c, const float (&v)[4]) {
-    const int m = m0 + r, n = n0 + c;
-    if (m >= p.m || n >= p.n) return;
-    T* dst = C + m * p.scm + n * p.scn;
-    if (vec) {  // p.n % 4 == 0, so n .. n+3 are in range
-      *reinterpret_cast<uint2*>(dst) = pack4(v);
-    } else {
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        if (n + q < p.n) dst[q * p.scn] = tk::from_f32<T>(v[q]);
-    }
-  });
+  static_assert(BM * stage_stride(kTileN) <= kScaleOff, "staged tile overlaps the row scales");
+  store_tile<T, BM, kTileN, kThreads>(C, p, m0, n0, lds, for_each_out);
 }
+
 
 // Row-major operands with K % 32 == 0 (NN), and the fused variants.
 template <typename T, bool kSwiGLU, bool kRowScale>
@@ -645,6 +473,34 @@ bool plan(const void* a, const void* b, int64_t m, int64_t n, int64_t k, int64_t
   return true;
 }
 
+// A launch takes about (tiles a CU gets) x (operand lines per tile): see gemm_tile_kernels.hpp.
+// The constants are cycles: kPerLine for each 128-byte line of a 64-wide K tile (one tile row
+// or column; rows past the problem's edge count, their DMA slots carry nothing else), kPerTile
+// for a tile's first loads and its epilogue. Against every tile of kTiles on 30 problems from
+// 1x4096x4096 to 5000x5000x2048 (three layouts, SwiGLU) the choice is the fastest or within 6 %
+// of it. 256 x 256 against the chosen tile, bf16: 1024^3 22.3 -> 11.3 us (64 x 64; 11 us is the
+// host's time per call), 2048^3 39.0 -> 20.0 (128 x 128), 1000x6144x4096 74.9 -> 49.0 (128 x
+// 192), 3000^3 61.5 -> 53.0 (192 x 192), 8192x1024x4096 71.5 -> 59.6 (128 x 256), 16x4096x4096
+// 66.5 -> 15.3 (64 x 64); 4096^3 100 (256 x 256) against 121 (256 x 128).
+int pick_tile(int64_t m, int64_t n, int64_t k, Variant variant) {
+  constexpr double kPerLine = 6.1, kPerTile = 4000.0;
+  constexpr int64_t kCus = 256;
+  int best = 0;
+  double best_cost = 0;
+  for (int i = 0; i < kTileCount; ++i) {
+    const Tile& t = kTiles[i];
+    if (variant == Variant::kSwiGLU && t.n % 128 != 0) continue;
+    const int64_t out_n = variant == Variant::kSwiGLU ? t.n / 2 : t.n;
+    const int64_t rounds = cdiv(cdiv(m, t.m) * cdiv(n, out_n), kCus);
+    const double cost = double(rounds) * (kPerTile + kPerLine * (t.m + t.n) * double(cdiv(k, 64)));
+    if (i == 0 || cost < best_cost) {
+      best = i;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 }  // namespace gemm_dma
 
 bool gemm_dma_applies(const void* a, const void* b, int64_t m, int64_t n, int64_t k,
@@ -686,6 +542,8 @@ void gemm_dma_launch(const gemm_dma::Plan& plan, int dtype, const void* a, const
     std::swap(m, n);
     std::swap(stride_cm, stride_cn);
   }
+  const Variant variant = row_scale != nullptr ? Variant::kRowScale : Variant::kPlain;
+  const int tile = pick_tile(m, n, k, variant);
   const int64_t a_rows = plan.layout == Layout::TN ? k : m, a_cols = plan.layout == Layout::TN ? m : k;
   const int64_t b_rows = plan.layout == Layout::NT ? n : k, b_cols = plan.layout == Layout::NT ? k : n;
   const uint32_t b_bytes = (uint32_t)(((b_rows - 1) * plan.ldb + b_cols) * 2);
@@ -697,22 +555,29 @@ void gemm_dma_launch(const gemm_dma::Plan& plan, int dtype, const void* a, const
             (int)plan.ldb,
             stride_cm,
             stride_cn,
-            (int)cdiv(m, BM),
-            (int)cdiv(n, BN),
+            (int)cdiv(m, kTiles[tile].m),
+            (int)cdiv(n, kTiles[tile].n),
             (uint32_t)(((a_rows - 1) * plan.lda + a_cols) * 2),
             b_bytes,
             b_bytes,
             row_scale};
-  if (dtype == TK_DTYPE_F16)
+  if (tile != 0) {
+    if (dtype == TK_DTYPE_F16)
+      launch_tile<_Float16>(tile, variant, plan, a, b, b, c, p, stream);
+    else
+      launch_tile<__bf16>(tile, variant, plan, a, b, b, c, p, stream);
+  } else if (dtype == TK_DTYPE_F16) {
     launch_256<_Float16>(plan, a, b, c, p, stream);
-  else
+  } else {
     launch_256<__bf16>(plan, a, b, c, p, stream);
+  }
 }
 
 void gemm_swiglu_dma_launch(int dtype, const void* a, const void* b_gate, const void* b_up,
                             void* y, int64_t m, int64_t n, int64_t k, int64_t stride_am,
                             int64_t stride_gk, int64_t stride_uk, int64_t stride_ym,
                             int64_t stride_yn, hipStream_t stream) {
+  const int tile = pick_tile(m, n, k, Variant::kSwiGLU);
   Problem p{(int)m,
             (int)n,
             (int)k,
@@ -721,13 +586,21 @@ void gemm_swiglu_dma_launch(int dtype, const void* a, const void* b_gate, const 
             (int)stride_uk,
             stride_ym,
             stride_yn,
-            (int)cdiv(m, BM),
-            (int)cdiv(n, 128),
+            (int)cdiv(m, kTiles[tile].m),
+            (int)cdiv(n, kTiles[tile].n / 2),
             (uint32_t)(((m - 1) * stride_am + k) * 2),
             (uint32_t)(((k - 1) * stride_gk + n) * 2),
             (uint32_t)(((k - 1) * stride_uk + n) * 2),
             nullptr};
   const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n));
+  const gemm_dma::Plan plan{Layout::NN, false, false, stride_am, stride_gk};
+  if (tile != 0) {
+    if (dtype == TK_DTYPE_F16)
+      launch_tile<_Float16>(tile, Variant::kSwiGLU, plan, a, b_gate, b_up, y, p, stream);
+    else
+      launch_tile<__bf16>(tile, Variant::kSwiGLU, plan, a, b_gate, b_up, y, p, stream);
+    return;
+  }
   if (dtype == TK_DTYPE_F16)
     hipLaunchKernelGGL((gemm_dma_kernel<_Float16, true, false>), grid, dim3(kThreads), 0, stream,
                        static_cast<const _Float16*>(a), static_cast<const _Float16*>(b_gate),

@@ -9,8 +9,8 @@ The reference autotunes 25 Triton configurations per shape
 (``matmul.py:23-75``); this build picks a kernel from the operands' layout and
 reports it in the same metadata keys. Operands whose rows are 16-byte aligned and
 multiples of 8 elements long, each row-major or transposed, take buffer->LDS DMA
-kernels (256 x 256 tiles, K step 32, eight wave64s, ``v_mfma_f32_16x16x32``):
-``gemm_dma_kernel`` for row-major operands with K % 32 == 0 (every registry shape),
+kernels (tiles from 64 x 64 to 256 x 256 by problem size, eight wave64s,
+``v_mfma_f32_16x16x32``): ``gemm_dma_kernel`` for row-major operands with K % 32 == 0 (every registry shape),
 ``gemm_kernel`` for transposed ones (a linear layer's gradients) and other K.
 Every other layout takes the register-staged ``gemm_kernel`` (256 x 256 x 64, four
 wave64s, ``v_mfma_f32_32x32x16``).
@@ -43,8 +43,10 @@ _DTYPES = (torch.float16, torch.bfloat16)
 # (the B operand's; A is loaded in 64-wide tiles into a ring of kAStages = 3).
 TILE = {"hip_kernel": "gemm_dma_kernel", "block_m": 256, "block_n": 256, "block_k": 32, "group_m": 4,
         "num_warps": 8, "num_stages": 4}
-# The same tiles on transposed operands or with K % 32 != 0.
-TRANSPOSED_TILE = {**TILE, "hip_kernel": "gemm_kernel"}
+# csrc/gemm_tile.hpp (kTiles): the tiles of problems too small to fill the chip with those; K step
+# 64, the stages that fit a CU's LDS (half of it for the smallest tiles, two workgroups per CU).
+_TILES = ((256, 256), (256, 128), (128, 256), (192, 192), (128, 192), (192, 128), (128, 128),
+          (128, 64), (64, 128), (64, 64))
 _MFMA = {
     torch.float16: "v_mfma_f32_16x16x32_f16",
     torch.bfloat16: "v_mfma_f32_16x16x32_bf16",
@@ -70,16 +72,35 @@ def _dma_rows(t: torch.Tensor) -> bool:
     )
 
 
+def _pick_tile(m: int, n: int, k: int) -> dict[str, BenchmarkScalar]:
+    """The DMA kernels' tile for a problem (``pick_tile``, csrc/gemm_dma.hip)."""
+
+    def cost(tile: tuple[int, int]) -> float:
+        rounds = -(-(-(-m // tile[0]) * -(-n // tile[1])) // 256)
+        return rounds * (4000.0 + 6.1 * sum(tile) * -(-k // 64))
+
+    block_m, block_n = min(_TILES, key=cost)
+    if (block_m, block_n) == _TILES[0]:
+        return TILE
+    stage = (block_m + block_n) * 128
+    stages = 81920 // stage if block_m + block_n <= 192 else min(5, 163840 // stage)
+    return {**TILE, "block_m": block_m, "block_n": block_n, "block_k": 64,
+            "group_m": 8 if block_n > block_m else 4, "num_stages": stages}
+
+
 def launch_config(a: torch.Tensor, b: torch.Tensor) -> dict[str, BenchmarkScalar]:
     """Tile configuration and MFMA of the kernel ``tk_gemm`` launches for ``a @ b``.
 
-    Mirrors ``gemm_dma::plan`` (csrc/gemm_dma.hip).
+    Mirrors ``gemm_dma::plan`` and ``pick_tile`` (csrc/gemm_dma.hip).
     """
     if not ((_dma_rows(a) or _dma_rows(a.t())) and (_dma_rows(b) or _dma_rows(b.t()))):
         return {**FALLBACK_TILE,
                 "mma_opcode": _FALLBACK_MFMA.get(a.dtype, _FALLBACK_MFMA[torch.float16])}
-    plain = _dma_rows(a) and _dma_rows(b) and a.shape[1] % 32 == 0
-    return {**(TILE if plain else TRANSPOSED_TILE),
+    (m, k), n = a.shape, b.shape[1]
+    plain = _dma_rows(a) and _dma_rows(b) and k % 32 == 0
+    swapped = not _dma_rows(a) and not _dma_rows(b)  # computed as C^T = B^T A^T
+    return {**(_pick_tile(n, m, k) if swapped else _pick_tile(m, n, k)),
+            "hip_kernel": "gemm_dma_kernel" if plain else "gemm_kernel",
             "mma_opcode": _MFMA.get(a.dtype, _MFMA[torch.float16])}
 
 
@@ -203,8 +224,7 @@ def _metadata_factory() -> BenchmarkMetadataFn:
 
     def metadata(size: int, dtype: torch.dtype) -> dict[str, BenchmarkScalar]:
         # Registry inputs are contiguous size x size matrices (size % 32 == 0).
-        del size
-        return {**TILE, "mma_opcode": _MFMA.get(dtype, _MFMA[torch.float16])}
+        return {**_pick_tile(size, size, size), "mma_opcode": _MFMA.get(dtype, _MFMA[torch.float16])}
 
     return metadata
 
