@@ -73,3 +73,33 @@ def test_input_gradient_of_any_width(m, n, k) -> None:
     expected = dev(oracle.gemm(host(dy), host(w.t()), name(dy.dtype)), got)
     assert_close(got, expected)
     assert_relative_frobenius(got, expected, max_relative_error=1e-3)
+
+
+def _odd_view(rows: int, cols: int, dtype: torch.dtype, layout: str) -> torch.Tensor:
+    """A (rows, cols) view at an odd element offset and row stride, by rows ("n"), by columns
+    ("t") or with a column stride of 3 ("s"), with NaN all round and between."""
+    shape = (cols, rows) if layout == "t" else (rows, cols)
+    step = 3 if layout == "s" else 1
+    width = shape[1] * step + 3 + shape[1] * step % 2  # odd
+    storage = torch.full((shape[0] + 2, width), float("nan"), device="cuda", dtype=dtype)
+    inner = storage[1:1 + shape[0], 1:1 + shape[1] * step:step]
+    inner.copy_(torch.randn(shape, device="cuda") * max(rows, cols) ** -0.25)
+    return inner.t() if layout == "t" else inner
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout", [*LAYOUTS, "sn", "ns", "ss", "st", "ts"])
+@pytest.mark.parametrize(
+    ("m", "n", "k"),
+    [(1, 1, 1), (3, 5, 7), (65, 63, 64), (64, 129, 65), (129, 257, 193), (2047, 1500, 129),
+     (700, 4099, 200), (4100, 4100, 66), (31, 1000, 1501)],
+)
+def test_unaligned_and_strided_operands(dtype, layout, m, n, k) -> None:
+    """The register-staged kernel's three tiles: the bits of the aligned problem."""
+    torch.manual_seed(m + n + k)
+    a, b = _odd_view(m, k, dtype, layout[0]), _odd_view(k, n, dtype, layout[1])
+    m8, n8, k32 = -(-m // 8) * 8, -(-n // 8) * 8, -(-k // 32) * 32
+    want = matmul_fp32acc(_padded(a, m8, k32), _padded(b, k32, n8))[:m, :n]
+    got = matmul_fp32acc(a, b)
+    assert bits_equal(got, want)
+    assert_close(got, a.float() @ b.float())

@@ -1,248 +1,280 @@
-// GEMM C = A * B on CDNA4 MFMA: f16/bf16 inputs, float32 accumulation,
-// f16/bf16 output (src/tklab/kernels/matmul.py:72-164 computes the same
-// product; here the tiling is MI355X's own).
+// GEMM entry points, C = A * B on CDNA4 MFMA: f16/bf16 inputs, float32 accumulation, f16/bf16
+// output (src/tklab/kernels/matmul.py:72-164 computes the same product; here the tiling is
+// MI355X's own), and the kernels for operands the DMA cannot load.
 //
-// tk_gemm sends operands stored by aligned rows (row-major or transposed) to the
-// buffer->LDS DMA kernels in gemm_dma.hip. This file's register-staged kernel takes
-// everything else: two non-unit strides, unaligned rows, odd row lengths, operands of 2 GiB
-// and more.
+// tk_gemm sends operands stored by aligned rows (row-major or transposed) to the buffer->LDS
+// DMA kernels (gemm_dma.hip, gemm_tile_kernels.hpp). This file's register-staged kernel takes
+// everything else: odd row lengths and row strides, unaligned bases, two non-unit strides,
+// operands of 2 GiB and more.
 //
-// Block tile 256 x 256, K step 64, 256 threads = 4 wave64s in a 2 x 2 grid;
-// each wave owns a 128 x 128 sub-tile as 4 x 4 MFMA tiles of
-// v_mfma_f32_32x32x16 (256 float32 accumulators per lane, one wave per SIMD).
-//
-// LDS holds both operands K-contiguous, [256 rows][64 k] per operand, two
-// buffers (128 KiB): a row is 8 chunks of 16 bytes (8 elements) and chunk c
-// of row r is stored at chunk c ^ swz(r), so that the MFMA operand reads
-// (8 consecutive rows, same chunk) and the tile writes both hit 8 distinct
-// 16-byte bank groups.
-//   A rows are m: swz = m % 8. A 16-byte global load is 8 consecutive k of
-//   one row and goes to LDS unchanged.
-//   B is stored transposed (rows are n): each thread loads an 8 k x 8 n block
-//   (eight 16-byte loads from eight k rows), transposes it in registers, and
-//   writes eight 16-byte chunks; swz = (n % 8) ^ ((n / 8) % 8).
-// MFMA operand layout (32x32x16): lane l supplies row l % 32 of A (resp.
-// column l % 32 of B) at k = 8*(l / 32) .. +7; accumulator register r of lane
-// l is D[8*(r/4) + 4*(l/32) + r%4][l % 32].
-//
-// Tile order: workgroup w runs on XCD w % 8; tiles are renumbered so each XCD
-// works through a contiguous range, walked in groups of 4 M-tiles so
-// concurrently running tiles share A and B panels in that XCD's L2.
-#include "gemm.hpp"
-#include "tk_common.hpp"
+// It keeps the DMA tile kernel's block tiles, wave grid, LDS stage layout and fragment reads;
+// only how a stage is filled differs. Each thread loads the 16-byte chunks that the DMA would
+// have put at its LDS slots into registers, two K tiles ahead, and writes them to LDS one tile
+// ahead: two register sets, two LDS stages, one barrier per 64-wide K tile. A chunk starts at
+// any element: with one unit stride it is one 16-byte load at 2-byte alignment, strided operands
+// load element by element. The loads have no branches (with them every load waited for the one
+// before: 125 us below), and what lies past K is zeroed on the way to LDS.
+// What bounds it is the vector memory path: an unaligned 128-byte row piece touches two lines.
+// bf16 1500x1500x6000: 1651 us with the per-element loads of a 256 x 256 x 64 kernel -> 67 us
+// (406 TFLOP/s; 64-bit offsets per load 72 us); fp16 4097^3 3150 -> 262 us; bf16 7x4001x4100
+// 598 -> 28 us; a linear layer's three products at 1111x4099x2050 2467 -> 166 us.
+#include "gemm_tile_kernels.hpp"
+
+#include <algorithm>
+#include <utility>
+
+#pragma clang fp contract(off)
 
 namespace {
 
-constexpr int BM = 256, BN = 256, BK = 64;
-constexpr int kThreads = 256;
-constexpr int kGroupM = 4;
-constexpr int kXcds = 8;
+using namespace tk::gemm_dma;
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+constexpr Tile kStagedTiles[] = {{256, 128}, {128, 128}, {64, 64}};
+constexpr int kStagedTileCount = sizeof(kStagedTiles) / sizeof(kStagedTiles[0]);
+constexpr int kFirstStrided = 1;  // element loads of a 256 x 128 tile do not fit the registers
 
-template <typename T>
-struct Mfma;
-template <>
-struct Mfma<_Float16> {
-  using Frag = f16x8;
-  static __device__ __forceinline__ f32x16 run(Frag a, Frag b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-  }
-};
-template <>
-struct Mfma<__bf16> {
-  using Frag = bf16x8;
-  static __device__ __forceinline__ f32x16 run(Frag a, Frag b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-  }
+// An operand: element (row, k) of a K-contiguous one at row * ld + k * inner, element (k, col)
+// of one stored by k-rows at k * ld + col * inner. Element offsets of the problem fit 31 bits;
+// 32-bit arithmetic may wrap for elements outside it.
+struct Operand {
+  uint32_t ld, inner;
+  uint32_t extent;  // elements from the base to the last one, inclusive
 };
 
-__device__ __forceinline__ int swz_a(int m) { return m & 7; }
-__device__ __forceinline__ int swz_b(int n) { return (n & 7) ^ ((n >> 3) & 7); }
-
-// One operand tile in LDS: 256 rows x 64 halves, 32 KiB.
-constexpr int kTileHalves = 256 * 64;
-
-struct Problem {
-  int m, n, k;
-  int64_t sam, sak, sbk, sbn, scm, scn;
-  int tiles_m, tiles_n;
+struct StagedProblem {
+  Problem p;
+  Operand a, b;
 };
 
-// Registers holding the next K tile: A chunks (8 x 16 B) and the B block (8 x 16 B).
-struct Staged {
-  uint4 a[8];
-  uint4 b[8];
-};
-
-template <typename T>
-__device__ __forceinline__ uint16_t bits_of(T v) {
-  return __builtin_bit_cast(uint16_t, v);
+// The element at offset `off` (below 2^31), as a scalar base plus a 32-bit byte offset.
+template <typename V>
+__device__ __forceinline__ const V* at(const uint16_t* base, uint32_t off) {
+  return reinterpret_cast<const V*>(reinterpret_cast<const char*>(base) + off * 2u);
 }
 
-// Global -> registers for the K tile starting at k0.
-// FAST: unit-stride rows, 16-byte aligned rows, K and N multiples of 8.
-// Otherwise every element is loaded on its own with full strides and bounds.
-template <typename T, bool FAST>
-__device__ __forceinline__ void load_tile(const T* __restrict__ A, const T* __restrict__ B,
-                                          const Problem& p, int m0, int n0, int k0, Staged& s) {
-  const int t = threadIdx.x;
+// Eight elements off, off + inner, ...; no branch, so that a tile's loads are all in flight at
+// once. Offsets past the operand's end are moved back inside it: fix_chunk undoes that.
+template <bool kUnit>
+__device__ __forceinline__ i32x4 load_chunk(const uint16_t* __restrict__ base, const Operand& o,
+                                            uint32_t off) {
+  if constexpr (kUnit) {
+    return at<Unaligned16>(base, min(off, o.extent - 8))->v;
+  } else {
+    typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+    u16x8 v;
 #pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const int idx = c * kThreads + t;
-    const int row = idx >> 3, chunk = idx & 7;
-    const int m = m0 + row, k = k0 + chunk * 8;
-    if constexpr (FAST) {
-      if (m < p.m && k < p.k)
-        s.a[c] = *reinterpret_cast<const uint4*>(A + m * p.sam + k);
-      else
-        s.a[c] = make_uint4(0, 0, 0, 0);
-    } else {
-      uint16_t h[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        h[e] = (m < p.m && k + e < p.k) ? bits_of(A[m * p.sam + (k + e) * p.sak]) : uint16_t(0);
-      s.a[c] = make_uint4(h[0] | (uint32_t(h[1]) << 16), h[2] | (uint32_t(h[3]) << 16),
-                          h[4] | (uint32_t(h[5]) << 16), h[6] | (uint32_t(h[7]) << 16));
-    }
-  }
-  const int nc = t & 31, kb = t >> 5;
-  const int n = n0 + nc * 8;
-#pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    const int k = k0 + kb * 8 + r;
-    if constexpr (FAST) {
-      if (k < p.k && n < p.n)
-        s.b[r] = *reinterpret_cast<const uint4*>(B + k * p.sbk + n);
-      else
-        s.b[r] = make_uint4(0, 0, 0, 0);
-    } else {
-      uint16_t h[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        h[e] = (k < p.k && n + e < p.n) ? bits_of(B[k * p.sbk + (n + e) * p.sbn]) : uint16_t(0);
-      s.b[r] = make_uint4(h[0] | (uint32_t(h[1]) << 16), h[2] | (uint32_t(h[3]) << 16),
-                          h[4] | (uint32_t(h[5]) << 16), h[6] | (uint32_t(h[7]) << 16));
-    }
+    for (int e = 0; e < 8; ++e) v[e] = *at<uint16_t>(base, min(off + e * o.inner, o.extent - 1));
+    return __builtin_bit_cast(i32x4, v);
   }
 }
 
-__device__ __forceinline__ uint32_t word(const uint4& v, int i) {
-  return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
+// The chunk loaded for `off` as its first `valid` elements followed by zeros.
+template <bool kUnit>
+__device__ __forceinline__ i32x4 fix_chunk(i32x4 v, const Operand& o, uint32_t off, int valid) {
+  if constexpr (kUnit) {
+    const uint32_t shift = off > o.extent - 8 ? off - (o.extent - 8) : 0u;
+    if (shift & 4) v = i32x4{v[2], v[3], 0, 0};
+    if (shift & 2) v = i32x4{v[1], v[2], v[3], 0};
+    if (shift & 1)
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+        v[d] = int((uint32_t(v[d]) >> 16) | (d < 3 ? uint32_t(v[d + 1]) << 16 : 0u));
+  }
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const int left = valid - 2 * d;
+    v[d] = left >= 2 ? v[d] : left == 1 ? v[d] & 0xffff : 0;
+  }
+  return v;
 }
 
-// Registers -> LDS buffer. B's 8 x 8 block is transposed on the way:
-// out[e] holds column n + e for k = kb*8 .. kb*8+7.
-__device__ __forceinline__ void store_tile(uint16_t* __restrict__ lds_a,
-                                           uint16_t* __restrict__ lds_b, const Staged& s) {
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const int idx = c * kThreads + t;
-    const int row = idx >> 3, chunk = idx & 7;
-    *reinterpret_cast<uint4*>(lds_a + row * 64 + ((chunk ^ swz_a(row)) << 3)) = s.a[c];
-  }
-  const int nc = t & 31, kb = t >> 5;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    uint32_t w[4];
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const uint32_t lo = word(s.b[2 * d], e >> 1);
-      const uint32_t hi = word(s.b[2 * d + 1], e >> 1);
-      w[d] = (e & 1) ? ((lo >> 16) | (hi & 0xffff0000u)) : ((lo & 0xffffu) | (hi << 16));
-    }
-    const int n = nc * 8 + e;
-    *reinterpret_cast<uint4*>(lds_b + n * 64 + ((kb ^ swz_b(n)) << 3)) =
-        make_uint4(w[0], w[1], w[2], w[3]);
-  }
-}
+template <typename T, int BM, int BN, Layout kLayout, bool kUnit>
+__global__ __launch_bounds__(kTileThreads) void gemm_kernel(const T* __restrict__ A,
+                                                            const T* __restrict__ B,
+                                                            T* __restrict__ C, StagedProblem sp) {
+  constexpr bool kARows = kLayout == Layout::TN, kBRows = kLayout != Layout::NT;
+  constexpr int WM = Grid<BM, BN>::WM, WN = Grid<BM, BN>::WN;
+  constexpr int MT = BM / WM / 16, NT = BN / WN / 16;
+  constexpr int kStageBytes = (BM + BN) * 128;
+  constexpr int kA = BM / 64, kB = BN / 64;  // chunks per thread and K tile
+  constexpr int kStaged = BM * stage_stride(BN);
+  __shared__ __attribute__((aligned(1024))) char lds[2 * kStageBytes > kStaged ? 2 * kStageBytes : kStaged];
+  const Problem& p = sp.p;
 
-template <typename T, bool FAST>
-__global__ __attribute__((amdgpu_flat_work_group_size(kThreads, kThreads),
-                          amdgpu_waves_per_eu(1, 1))) void
-gemm_kernel(const T* __restrict__ A, const T* __restrict__ B, T* __restrict__ C, Problem p) {
-  using Frag = typename Mfma<T>::Frag;
-  __shared__ __attribute__((aligned(16))) uint16_t lds[2][2][kTileHalves];
-
-  // ---- tile order: XCD-contiguous ranges, grouped along M.
-  const int total = p.tiles_m * p.tiles_n;
-  int w = blockIdx.x;
-  if (total % kXcds == 0) w = (w % kXcds) * (total / kXcds) + w / kXcds;
-  const int per_group = kGroupM * p.tiles_n;
-  const int group = w / per_group;
-  const int first_m = group * kGroupM;
-  const int group_m = min(p.tiles_m - first_m, kGroupM);
-  const int tile_m = first_m + (w % per_group) % group_m;
-  const int tile_n = (w % per_group) / group_m;
-  const int m0 = tile_m * BM, n0 = tile_n * BN;
-
+  int m0, n0;
+  tile_origin<BM, BN, BN>(p, m0, n0);
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int wm = (wave >> 1) * 128, wn = (wave & 1) * 128;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
+  const int l16 = lane & 15, lg = lane >> 4;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_void*)lds;
+  const int kt = (p.k + kTileK - 1) / kTileK;
 
-  f32x16 acc[4][4];
+  // Chunk x of this thread is the one at byte x * 8192 + wave * 1024 + lane * 16 of the
+  // operand's stage (tile_source's placement). Rows and columns past the operand's edge load
+  // the last one's values, which only reach outputs that are not stored; k past the edge must
+  // read as zero (`valid` of a chunk's elements lie inside K).
+  uint32_t a_off[kA], b_off[kB];  // of K tile 0
+  int a_k[kA], b_k[kB];
+  auto place = [&](auto rows, const Operand& o, int x, int first, int count, uint32_t& off, int& k) {
+    const int i = x * 8 + wave, slot = lane & 7;
+    if constexpr (decltype(rows)::value) {
+      k = (i & 7) * 8 + (lane >> 3);
+      const int col = first + (i >> 3) * 64 + ((((slot >> 1) ^ row_swz(k)) << 1) | (slot & 1)) * 8;
+      off = k * o.ld + min(col, count - 1) * o.inner;
+    } else {
+      const int r = i * 8 + (lane >> 3);
+      k = (slot ^ a_swz(r)) * 8;
+      off = min(first + r, count - 1) * o.ld + k * o.inner;
+    }
+  };
+  using ARows = std::integral_constant<bool, kARows>;
+  using BRows = std::integral_constant<bool, kBRows>;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int x = 0; x < kA; ++x) place(ARows{}, sp.a, x, m0, p.m, a_off[x], a_k[x]);
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+  for (int x = 0; x < kB; ++x) place(BRows{}, sp.b, x, n0, p.n, b_off[x], b_k[x]);
+  const uint32_t a_step = kTileK * (kARows ? sp.a.ld : sp.a.inner);
+  const uint32_t b_step = kTileK * (kBRows ? sp.b.ld : sp.b.inner);
+  auto valid = [&](bool rows, int k) { return rows ? (k < p.k ? 8 : 0) : max(0, min(8, p.k - k)); };
+  const uint16_t* a_base = reinterpret_cast<const uint16_t*>(A);
+  const uint16_t* b_base = reinterpret_cast<const uint16_t*>(B);
+  auto load = [&](int tile, i32x4 (&va)[kA], i32x4 (&vb)[kB]) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    for (int x = 0; x < kA; ++x) va[x] = load_chunk<kUnit>(a_base, sp.a, a_off[x] + tile * a_step);
+#pragma unroll
+    for (int x = 0; x < kB; ++x) vb[x] = load_chunk<kUnit>(b_base, sp.b, b_off[x] + tile * b_step);
+  };
+  // Only a chunk within 8 rows of K's end can be cut short or moved (a row may be shorter than
+  // a chunk).
+  auto store = [&](int tile, i32x4 (&va)[kA], i32x4 (&vb)[kB]) {
+    if ((tile + 1) * kTileK + 8 > p.k) {
+#pragma unroll
+      for (int x = 0; x < kA; ++x)
+        va[x] = fix_chunk<kUnit>(va[x], sp.a, a_off[x] + tile * a_step,
+                                 valid(kARows, tile * kTileK + a_k[x]));
+#pragma unroll
+      for (int x = 0; x < kB; ++x)
+        vb[x] = fix_chunk<kUnit>(vb[x], sp.b, b_off[x] + tile * b_step,
+                                 valid(kBRows, tile * kTileK + b_k[x]));
+    }
+    char* dst = lds + (tile & 1) * kStageBytes + wave * 1024 + lane * 16;
+#pragma unroll
+    for (int x = 0; x < kA; ++x) *reinterpret_cast<i32x4*>(dst + x * 8192) = va[x];
+#pragma unroll
+    for (int x = 0; x < kB; ++x) *reinterpret_cast<i32x4*>(dst + BM * 128 + x * 8192) = vb[x];
+  };
 
-  const int k_tiles = (p.k + BK - 1) / BK;
-  Staged st;
-  load_tile<T, FAST>(A, B, p, m0, n0, 0, st);
-  store_tile(lds[0][0], lds[0][1], st);
+  const Fragments<kARows, MT> fa(wm, l16, lg);
+  const Fragments<kBRows, NT> fb(wn, l16, lg);
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // Tile t: the barrier says that every wave's part of stage t % 2 is written and that stage
+  // (t + 1) % 2, which takes tile t + 1 below, has been read (tile t - 1).
+  auto step = [&](int t, i32x4 (&ahead_a)[kA], i32x4 (&ahead_b)[kB], i32x4 (&next_a)[kA],
+                  i32x4 (&next_b)[kB]) {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    load(t + 2, ahead_a, ahead_b);
+    const uint32_t base = lds_base + (t & 1) * kStageBytes;
+    unroll<0, 2>([&](auto half) {
+      constexpr int H = decltype(half)::value;
+      i32x4 a[MT], b[NT];
+      unroll<0, MT>([&](auto i) { a[decltype(i)::value] = fa.template read<decltype(i)::value, H>(base); });
+      unroll<0, NT>([&](auto j) { b[decltype(j)::value] = fb.template read<decltype(j)::value, H>(base + BM * 128); });
+      wait_lgkm_pin(a);
+      wait_lgkm_pin(b);
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = Mfma<T>::run(b[j], a[i], acc[i][j]);
+    });
+    store(t + 1, next_a, next_b);
+  };
+  i32x4 a0[kA], b0[kB], a1[kA], b1[kB];
+  load(0, a0, b0);
+  load(1, a1, b1);
+  store(0, a0, b0);
+  for (int t = 0; t < kt; t += 2) {
+    step(t, a0, b0, a1, b1);
+    if (t + 1 < kt) step(t + 1, a1, b1, a0, b0);
+  }
   __syncthreads();
 
-  const int lrow = lane & 31, lhalf = lane >> 5;
-  for (int kt = 0; kt < k_tiles; ++kt) {
-    const int buf = kt & 1;
-    const bool more = kt + 1 < k_tiles;
-    if (more) load_tile<T, FAST>(A, B, p, m0, n0, (kt + 1) * BK, st);
-
-    const uint16_t* la = lds[buf][0];
-    const uint16_t* lb = lds[buf][1];
+  store_tile<T, BM, BN, kTileThreads>(C, p, m0, n0, lds, [&](auto&& emit) {
 #pragma unroll
-    for (int kk = 0; kk < BK / 16; ++kk) {
-      const int chunk = kk * 2 + lhalf;
-      Frag af[4], bf[4];
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = wm + i * 32 + lrow;
-        af[i] = *reinterpret_cast<const Frag*>(la + m * 64 + ((chunk ^ swz_a(m)) << 3));
+      for (int j = 0; j < NT; ++j) {
+        const float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+        emit(wm + i * 16 + l16, wn + j * 16 + lg * 4, v);
       }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int n = wn + j * 32 + lrow;
-        bf[j] = *reinterpret_cast<const Frag*>(lb + n * 64 + ((chunk ^ swz_b(n)) << 3));
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = Mfma<T>::run(af[i], bf[j], acc[i][j]);
-    }
+  });
+}
 
-    if (more) store_tile(lds[buf ^ 1][0], lds[buf ^ 1][1], st);
-    __syncthreads();
+template <typename T, int BM, int BN>
+void launch_staged(Layout layout, bool unit, const T* a, const T* b, T* c, const StagedProblem& sp,
+                   hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>(sp.p.tiles_m * sp.p.tiles_n)), block(kTileThreads);
+  if (!unit) {
+    if constexpr (BM < kStagedTiles[0].m)
+      hipLaunchKernelGGL((gemm_kernel<T, BM, BN, Layout::NN, false>), grid, block, 0, stream, a, b, c, sp);
+  } else if (layout == Layout::NN) {
+    hipLaunchKernelGGL((gemm_kernel<T, BM, BN, Layout::NN, true>), grid, block, 0, stream, a, b, c, sp);
+  } else if (layout == Layout::NT) {
+    hipLaunchKernelGGL((gemm_kernel<T, BM, BN, Layout::NT, true>), grid, block, 0, stream, a, b, c, sp);
+  } else {
+    hipLaunchKernelGGL((gemm_kernel<T, BM, BN, Layout::TN, true>), grid, block, 0, stream, a, b, c, sp);
   }
+}
 
-  // ---- epilogue: D[8*(r/4) + 4*(l/32) + r%4][l%32] of each 32 x 32 tile.
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + wn + j * 32 + lrow;
-      if (n >= p.n) continue;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm + i * 32 + (r >> 2) * 8 + lhalf * 4 + (r & 3);
-        if (m < p.m) C[m * p.scm + n * p.scn] = tk::from_f32<T>(acc[i][j][r]);
-      }
-    }
+template <typename T>
+void gemm_staged(const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k,
+                 int64_t stride_am, int64_t stride_ak, int64_t stride_bk, int64_t stride_bn,
+                 int64_t stride_cm, int64_t stride_cn, hipStream_t stream) {
+  if (stride_ak != 1 && stride_am == 1 && stride_bn != 1 && stride_bk == 1) {
+    // Both transposed: C^T = B^T A^T, both row-major.
+    std::swap(a, b);
+    std::swap(m, n);
+    std::swap(stride_am, stride_bn);
+    std::swap(stride_ak, stride_bk);
+    std::swap(stride_cm, stride_cn);
   }
+  const bool a_rows = stride_ak != 1 && stride_am == 1, b_wide = stride_bn != 1 && stride_bk == 1;
+  const int64_t a_extent = (m - 1) * stride_am + (k - 1) * stride_ak + 1;
+  const int64_t b_extent = (k - 1) * stride_bk + (n - 1) * stride_bn + 1;
+  // Wide loads need eight elements to load from.
+  const bool unit = (stride_ak == 1 || a_rows) && (stride_bn == 1 || b_wide) && a_extent >= 8 &&
+                    b_extent >= 8;
+  const Layout layout = unit && a_rows ? Layout::TN : unit && b_wide ? Layout::NT : Layout::NN;
+  const int first = unit ? 0 : kFirstStrided;
+  const int tile = first + pick_tile(kStagedTiles + first, kStagedTileCount - first, m, n, k,
+                                     Variant::kPlain);
+  StagedProblem sp{};
+  sp.p.m = (int)m;
+  sp.p.n = (int)n;
+  sp.p.k = (int)k;
+  sp.p.scm = stride_cm;
+  sp.p.scn = stride_cn;
+  sp.p.tiles_m = (int)tk::cdiv(m, kStagedTiles[tile].m);
+  sp.p.tiles_n = (int)tk::cdiv(n, kStagedTiles[tile].n);
+  auto operand = [](int64_t ld, int64_t inner, int64_t extent) {
+    return Operand{(uint32_t)ld, (uint32_t)inner, (uint32_t)extent};
+  };
+  sp.a = layout == Layout::TN ? operand(stride_ak, 1, a_extent) : operand(stride_am, stride_ak, a_extent);
+  sp.b = layout == Layout::NT ? operand(stride_bn, 1, b_extent) : operand(stride_bk, stride_bn, b_extent);
+  const T* pa = static_cast<const T*>(a);
+  const T* pb = static_cast<const T*>(b);
+  T* pc = static_cast<T*>(c);
+  if (tile == 0)
+    launch_staged<T, 256, 128>(layout, unit, pa, pb, pc, sp, stream);
+  else if (tile == 1)
+    launch_staged<T, 128, 128>(layout, unit, pa, pb, pc, sp, stream);
+  else
+    launch_staged<T, 64, 64>(layout, unit, pa, pb, pc, sp, stream);
 }
 
 }  // namespace
@@ -264,37 +296,19 @@ extern "C" int tk_gemm(int dtype, const void* a, const void* b, void* c, int64_t
   if (m > lim || n > lim || k > lim || tk::extent(m, stride_am, k, stride_ak) > lim ||
       tk::extent(k, stride_bk, n, stride_bn) > lim || tk::extent(m, stride_cm, n, stride_cn) > lim)
     return tk::fail("gemm: operand exceeds the int32 offset range");
-  const int64_t tiles_m = tk::cdiv(m, BM), tiles_n = tk::cdiv(n, BN);
-  if (tiles_m * tiles_n > INT32_MAX) return tk::fail("gemm: too many tiles");
-  Problem p{(int)m, (int)n, (int)k, stride_am, stride_ak, stride_bk, stride_bn,
-            stride_cm, stride_cn, (int)tiles_m, (int)tiles_n};
+  if (tk::cdiv(m, 64) * tk::cdiv(n, 64) > INT32_MAX) return tk::fail("gemm: too many tiles");
   hipStream_t s = tk::as_stream(stream);
   tk::gemm_dma::Plan plan;
   if (tk::gemm_dma::plan(a, b, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, &plan)) {
     tk::gemm_dma_launch(plan, dtype, a, b, c, m, n, k, stride_cm, stride_cn, s);
     return tk::check_launch("gemm");
   }
-  const bool fast = stride_ak == 1 && stride_bn == 1 && k % 8 == 0 && n % 8 == 0 &&
-                    stride_am % 8 == 0 && stride_bk % 8 == 0 && tk::aligned16(a) &&
-                    tk::aligned16(b);
-  const dim3 grid(static_cast<unsigned>(tiles_m * tiles_n));
-  if (dtype == TK_DTYPE_F16) {
-    using T = _Float16;
-    if (fast)
-      hipLaunchKernelGGL((gemm_kernel<T, true>), grid, dim3(kThreads), 0, s,
-                         static_cast<const T*>(a), static_cast<const T*>(b), static_cast<T*>(c), p);
-    else
-      hipLaunchKernelGGL((gemm_kernel<T, false>), grid, dim3(kThreads), 0, s,
-                         static_cast<const T*>(a), static_cast<const T*>(b), static_cast<T*>(c), p);
-  } else {
-    using T = __bf16;
-    if (fast)
-      hipLaunchKernelGGL((gemm_kernel<T, true>), grid, dim3(kThreads), 0, s,
-                         static_cast<const T*>(a), static_cast<const T*>(b), static_cast<T*>(c), p);
-    else
-      hipLaunchKernelGGL((gemm_kernel<T, false>), grid, dim3(kThreads), 0, s,
-                         static_cast<const T*>(a), static_cast<const T*>(b), static_cast<T*>(c), p);
-  }
+  if (dtype == TK_DTYPE_F16)
+    gemm_staged<_Float16>(a, b, c, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, stride_cm,
+                          stride_cn, s);
+  else
+    gemm_staged<__bf16>(a, b, c, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, stride_cm,
+                        stride_cn, s);
   return tk::check_launch("gemm");
 }
 
@@ -338,7 +352,7 @@ extern "C" int tk_gemm_rowscale(int dtype, const void* a, const void* b, const f
   if (!tk::gemm_dma_applies(a, b, m, n, k, stride_am, stride_ak, stride_bk, stride_bn))
     return tk::fail("gemm_rowscale: needs unit inner strides, 16-byte aligned rows, k %% 32 == 0, "
                     "n %% 8 == 0 and operands below 2 GiB");
-  if (tk::cdiv(m, BM) * tk::cdiv(n, BN) > INT32_MAX) return tk::fail("gemm_rowscale: too many tiles");
+  if (tk::cdiv(m, 64) * tk::cdiv(n, 64) > INT32_MAX) return tk::fail("gemm_rowscale: too many tiles");
   const tk::gemm_dma::Plan plan{tk::gemm_dma::Layout::NN, false, false, stride_am, stride_bk};
   tk::gemm_dma_launch(plan, dtype, a, b, c, m, n, k, stride_cm, stride_cn, tk::as_stream(stream),
                       row_scale);

@@ -149,65 +149,76 @@ __device__ __forceinline__ uint2 pack4(const float (&v)[4]) {
 // banks.
 constexpr int stage_stride(int cols) { return cols * 2 + 16; }
 
+// 16 bytes at any element boundary (the compiler emits one dwordx4 access).
+struct __attribute__((packed, aligned(2))) Unaligned16 {
+  i32x4 v;
+};
+
 // Writes a kRows x kCols tile of C at (m0, n0). for_each(emit) calls emit(row, column, values)
 // for every group of four consecutive columns this lane holds; the kThreads threads of the
-// workgroup run it together and `lds` (kRows * stage_stride(kCols) bytes) is idle. When C rows
-// are 16-byte aligned the rounded tile is staged in LDS and written back as whole rows, 16
-// bytes per lane, with non-temporal stores of full 128-byte lines; otherwise each lane stores
-// its four columns. Staged, the epilogue of fp16 4096^3 on 256 x 256 tiles took ~4 instead of
-// ~8 us of a ~108 us launch (a timing-only copy without stores ran 102 us): 4096^3 108.1 ->
-// 104.3 us, 8192^3 784 -> 773 us, the row-scaled 16384x6144x4096 GEMM 675 -> 645 us. Staged
-// with default-policy stores: 105.1, 773 and 654 us. Per-lane non-temporal stores write
-// 32-byte segments of four lines and were 5-14 % slower than default-policy ones.
+// workgroup run it together and `lds` (kRows * stage_stride(kCols) bytes) is idle. With unit
+// column stride the rounded tile is staged in LDS and written back as whole rows, 16 bytes per
+// lane: non-temporal stores of full 128-byte lines when C rows are 16-byte aligned, stores at
+// 2-byte alignment otherwise. Other layouts store element by element.
+// Staged, the epilogue of fp16 4096^3 on 256 x 256 tiles took ~4 instead of ~8 us of a ~108 us
+// launch (a timing-only copy without stores ran 102 us): 4096^3 108.1 -> 104.3 us, 8192^3 784
+// -> 773 us, the row-scaled 16384x6144x4096 GEMM 675 -> 645 us. Staged with default-policy
+// stores: 105.1, 773 and 654 us. Per-lane non-temporal stores write 32-byte segments of four
+// lines and were 5-14 % slower than default-policy ones.
 template <typename T, int kRows, int kCols, int kThreads, typename ForEach>
 __device__ __forceinline__ void store_tile(T* __restrict__ C, const Problem& p, int m0, int n0,
                                            char* lds, ForEach&& for_each) {
-  const bool rows16 = p.scn == 1 && (p.n & 7) == 0 && (p.scm & 7) == 0 &&
-                      (reinterpret_cast<uintptr_t>(C) & 15) == 0;
-  if (rows16) {
-    // p.n % 8 == 0, so a 16-byte group is wholly inside or outside N.
-    constexpr int kStride = stage_stride(kCols);
+  if (p.scn != 1) {
     for_each([&](int r, int c, const float (&v)[4]) {
-      *reinterpret_cast<uint2*>(lds + r * kStride + c * 2) = pack4<T>(v);
-    });
-    __syncthreads();
-    constexpr int kLanesPerRow = kCols / 8;
-    if constexpr (kThreads % kLanesPerRow == 0) {
-      constexpr int kRowsPerPass = kThreads / kLanesPerRow;
-      const int cr = threadIdx.x / kLanesPerRow, cc = (threadIdx.x % kLanesPerRow) * 8;
-#pragma unroll 4
-      for (int pass = 0; pass < kRows / kRowsPerPass; ++pass) {
-        const int r = pass * kRowsPerPass + cr;
-        const i32x4 v = *reinterpret_cast<const i32x4*>(lds + r * kStride + cc * 2);
-        if (m0 + r < p.m && n0 + cc < p.n)
-          __builtin_nontemporal_store(v, reinterpret_cast<i32x4*>(C + (m0 + r) * p.scm + n0 + cc));
-      }
-    } else {  // 192 columns: 24 lanes per row
-      static_assert(kRows * kLanesPerRow % kThreads == 0, "whole passes");
-#pragma unroll 4
-      for (int g = threadIdx.x; g < kRows * kLanesPerRow; g += kThreads) {
-        const int r = g / kLanesPerRow, cc = (g % kLanesPerRow) * 8;
-        const i32x4 v = *reinterpret_cast<const i32x4*>(lds + r * kStride + cc * 2);
-        if (m0 + r < p.m && n0 + cc < p.n)
-          __builtin_nontemporal_store(v, reinterpret_cast<i32x4*>(C + (m0 + r) * p.scm + n0 + cc));
-      }
-    }
-    return;
-  }
-  const bool vec = p.scn == 1 && (p.n & 3) == 0 && (p.scm & 3) == 0 &&
-                   (reinterpret_cast<uintptr_t>(C) & 7) == 0;
-  for_each([&](int r, int c, const float (&v)[4]) {
-    const int m = m0 + r, n = n0 + c;
-    if (m >= p.m || n >= p.n) return;
-    T* dst = C + m * p.scm + n * p.scn;
-    if (vec) {  // p.n % 4 == 0, so n .. n+3 are in range
-      *reinterpret_cast<uint2*>(dst) = pack4<T>(v);
-    } else {
+      const int m = m0 + r, n = n0 + c;
+      if (m >= p.m || n >= p.n) return;
+      T* dst = C + m * p.scm + n * p.scn;
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         if (n + q < p.n) dst[q * p.scn] = tk::from_f32<T>(v[q]);
-    }
+    });
+    return;
+  }
+  constexpr int kStride = stage_stride(kCols), kLanesPerRow = kCols / 8;
+  for_each([&](int r, int c, const float (&v)[4]) {
+    *reinterpret_cast<uint2*>(lds + r * kStride + c * 2) = pack4<T>(v);
   });
+  __syncthreads();
+  // Groups of 16 bytes, in order: kThreads / kLanesPerRow rows per pass where that is whole.
+  constexpr bool kWhole = kThreads % kLanesPerRow == 0;
+  constexpr int kRowStep = kWhole ? kThreads / kLanesPerRow : 1;
+  static_assert(kRows * kLanesPerRow % kThreads == 0, "whole passes");
+  auto each_group = [&](auto&& store) {
+    int r = threadIdx.x / kLanesPerRow, c = (threadIdx.x % kLanesPerRow) * 8;
+#pragma unroll 4
+    for (int pass = 0; pass < kRows * kLanesPerRow / kThreads; ++pass) {
+      if constexpr (!kWhole) {
+        const int g = pass * kThreads + threadIdx.x;
+        r = g / kLanesPerRow;
+        c = (g % kLanesPerRow) * 8;
+      }
+      const int row = kWhole ? pass * kRowStep + r : r;
+      const i32x4 v = *reinterpret_cast<const i32x4*>(lds + row * kStride + c * 2);
+      if (m0 + row < p.m && n0 + c < p.n) store(C + (m0 + row) * p.scm + n0 + c, n0 + c, v);
+    }
+  };
+  if ((p.n & 7) == 0 && (p.scm & 7) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0) {
+    // p.n % 8 == 0, so a 16-byte group is wholly inside or outside N.
+    each_group([&](T* dst, int, i32x4 v) {
+      __builtin_nontemporal_store(v, reinterpret_cast<i32x4*>(dst));
+    });
+  } else {
+    each_group([&](T* dst, int n, i32x4 v) {
+      if (n + 8 <= p.n) {
+        reinterpret_cast<Unaligned16*>(dst)->v = v;
+      } else {
+#pragma unroll
+        for (int q = 0; q < 7; ++q)
+          if (n + q < p.n)
+            reinterpret_cast<uint16_t*>(dst)[q] = uint16_t(uint32_t(v[q >> 1]) >> (16 * (q & 1)));
+      }
+    });
+  }
 }
 
 }  // namespace gemm_dma

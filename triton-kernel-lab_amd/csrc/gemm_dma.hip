@@ -482,13 +482,13 @@ bool plan(const void* a, const void* b, int64_t m, int64_t n, int64_t k, int64_t
 // host's time per call), 2048^3 39.0 -> 20.0 (128 x 128), 1000x6144x4096 74.9 -> 49.0 (128 x
 // 192), 3000^3 61.5 -> 53.0 (192 x 192), 8192x1024x4096 71.5 -> 59.6 (128 x 256), 16x4096x4096
 // 66.5 -> 15.3 (64 x 64); 4096^3 100 (256 x 256) against 121 (256 x 128).
-int pick_tile(int64_t m, int64_t n, int64_t k, Variant variant) {
+int pick_tile(const Tile* tiles, int count, int64_t m, int64_t n, int64_t k, Variant variant) {
   constexpr double kPerLine = 6.1, kPerTile = 4000.0;
   constexpr int64_t kCus = 256;
   int best = 0;
   double best_cost = 0;
-  for (int i = 0; i < kTileCount; ++i) {
-    const Tile& t = kTiles[i];
+  for (int i = 0; i < count; ++i) {
+    const Tile& t = tiles[i];
     if (variant == Variant::kSwiGLU && t.n % 128 != 0) continue;
     const int64_t out_n = variant == Variant::kSwiGLU ? t.n / 2 : t.n;
     const int64_t rounds = cdiv(cdiv(m, t.m) * cdiv(n, out_n), kCus);
@@ -543,7 +543,7 @@ void gemm_dma_launch(const gemm_dma::Plan& plan, int dtype, const void* a, const
     std::swap(stride_cm, stride_cn);
   }
   const Variant variant = row_scale != nullptr ? Variant::kRowScale : Variant::kPlain;
-  const int tile = pick_tile(m, n, k, variant);
+  const int tile = pick_tile(kTiles, kTileCount, m, n, k, variant);
   const int64_t a_rows = plan.layout == Layout::TN ? k : m, a_cols = plan.layout == Layout::TN ? m : k;
   const int64_t b_rows = plan.layout == Layout::NT ? n : k, b_cols = plan.layout == Layout::NT ? k : n;
   const uint32_t b_bytes = (uint32_t)(((b_rows - 1) * plan.ldb + b_cols) * 2);
@@ -577,7 +577,7 @@ void gemm_swiglu_dma_launch(int dtype, const void* a, const void* b_gate, const 
                             void* y, int64_t m, int64_t n, int64_t k, int64_t stride_am,
                             int64_t stride_gk, int64_t stride_uk, int64_t stride_ym,
                             int64_t stride_yn, hipStream_t stream) {
-  const int tile = pick_tile(m, n, k, Variant::kSwiGLU);
+  const int tile = pick_tile(kTiles, kTileCount, m, n, k, Variant::kSwiGLU);
   Problem p{(int)m,
             (int)n,
             (int)k,

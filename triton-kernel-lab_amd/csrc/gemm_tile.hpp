@@ -17,9 +17,9 @@ constexpr Tile kTiles[] = {{256, 256}, {256, 128}, {128, 256}, {192, 192}, {128,
                            {192, 128}, {128, 128}, {128, 64},  {64, 128},  {64, 64}};
 constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
 
-// Index of the tile for a problem (0 is the 256 x 256 kernel of gemm_dma.hip). Every tile sums
-// K in the same order, so the choice never changes a result.
-int pick_tile(int64_t m, int64_t n, int64_t k, Variant variant);
+// Index of the tile for a problem (0 of kTiles is the 256 x 256 kernel of gemm_dma.hip). Every
+// tile sums K in the same order, so the choice never changes a result.
+int pick_tile(const Tile* tiles, int count, int64_t m, int64_t n, int64_t k, Variant variant);
 
 // Enqueues the small-tile kernel `tile` (1 ..) for a problem whose tile counts are filled in.
 template <typename T>

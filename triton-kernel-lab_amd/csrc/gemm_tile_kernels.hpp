@@ -89,6 +89,21 @@ struct Fragments {
   }
 };
 
+// First row and column of this workgroup's tile: workgroup w runs on XCD w % 8; each XCD walks a
+// contiguous range of tiles in groups of kGroup M-tiles, sharing A and B panels in its L2.
+template <int BM, int BN, int kOutN>
+__device__ __forceinline__ void tile_origin(const Problem& p, int& m0, int& n0) {
+  constexpr int kGroup = BN > BM ? 8 : 4;
+  const int total = p.tiles_m * p.tiles_n;
+  const int xcd = blockIdx.x % kXcds;
+  const int w = xcd * (total / kXcds) + min(xcd, total % kXcds) + blockIdx.x / kXcds;
+  const int per_group = kGroup * p.tiles_n;
+  const int first_m = (w / per_group) * kGroup;
+  const int group_m = min(p.tiles_m - first_m, kGroup);
+  m0 = (first_m + (w % per_group) % group_m) * BM;
+  n0 = ((w % per_group) / group_m) * kOutN;
+}
+
 template <int I, int N, typename F>
 __device__ __forceinline__ void unroll(F&& f) {
   if constexpr (I < N) {
@@ -116,17 +131,8 @@ __device__ __forceinline__ void gemm_tile(const T* __restrict__ A, const T* __re
   static_assert(!kSwiGLU || (NT % 2 == 0 && BN % 128 == 0), "gate and up columns per wave and block");
   __shared__ __attribute__((aligned(1024))) char lds[kLds];
 
-  // Tile order: workgroup w runs on XCD w % 8; each XCD walks a contiguous range of tiles in
-  // groups of kGroup M-tiles, sharing A and B panels in its L2.
-  constexpr int kGroup = BN > BM ? 8 : 4;
-  const int total = p.tiles_m * p.tiles_n;
-  const int xcd = blockIdx.x % kXcds;
-  const int w = xcd * (total / kXcds) + min(xcd, total % kXcds) + blockIdx.x / kXcds;
-  const int per_group = kGroup * p.tiles_n;
-  const int first_m = (w / per_group) * kGroup;
-  const int group_m = min(p.tiles_m - first_m, kGroup);
-  const int m0 = (first_m + (w % per_group) % group_m) * BM;
-  const int n0 = ((w % per_group) / group_m) * kOutN;
+  int m0, n0;
+  tile_origin<BM, BN, kOutN>(p, m0, n0);
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

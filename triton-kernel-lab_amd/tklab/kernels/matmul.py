@@ -12,8 +12,7 @@ multiples of 8 elements long, each row-major or transposed, take buffer->LDS DMA
 kernels (tiles from 64 x 64 to 256 x 256 by problem size, eight wave64s,
 ``v_mfma_f32_16x16x32``): ``gemm_dma_kernel`` for row-major operands with K % 32 == 0 (every registry shape),
 ``gemm_kernel`` for transposed ones (a linear layer's gradients) and other K.
-Every other layout takes the register-staged ``gemm_kernel`` (256 x 256 x 64, four
-wave64s, ``v_mfma_f32_32x32x16``).
+Every other layout takes the register-staged ``gemm_kernel`` (64 x 64 to 256 x 128).
 ``matmul_fp16acc`` keeps its registry entry, but gfx950 MFMA
 accumulates f16 products in float32 only, so both entry points run the same
 FP32-accumulate kernel (its result is at least as accurate as an FP16
@@ -51,13 +50,9 @@ _MFMA = {
     torch.float16: "v_mfma_f32_16x16x32_f16",
     torch.bfloat16: "v_mfma_f32_16x16x32_bf16",
 }
-# csrc/gemm.hip's register-staged kernel: every other operand layout (double-buffered in registers).
-FALLBACK_TILE = {"hip_kernel": "gemm_kernel", "block_m": 256, "block_n": 256, "block_k": 64,
-                 "group_m": 4, "num_warps": 4, "num_stages": 2}
-_FALLBACK_MFMA = {
-    torch.float16: "v_mfma_f32_32x32x16_f16",
-    torch.bfloat16: "v_mfma_f32_32x32x16_bf16",
-}
+# csrc/gemm.hip's register-staged kernel (kStagedTiles): every other operand layout, two LDS
+# stages. The first tile takes operands with one unit stride each only.
+_STAGED_TILES = ((256, 128), (128, 128), (64, 64))
 
 
 def _dma_rows(t: torch.Tensor) -> bool:
@@ -72,36 +67,47 @@ def _dma_rows(t: torch.Tensor) -> bool:
     )
 
 
-def _pick_tile(m: int, n: int, k: int) -> dict[str, BenchmarkScalar]:
-    """The DMA kernels' tile for a problem (``pick_tile``, csrc/gemm_dma.hip)."""
+def _pick_tile(m: int, n: int, k: int, tiles: tuple[tuple[int, int], ...] = _TILES) -> tuple[int, int]:
+    """The tile for a problem (``pick_tile``, csrc/gemm_dma.hip)."""
 
     def cost(tile: tuple[int, int]) -> float:
         rounds = -(-(-(-m // tile[0]) * -(-n // tile[1])) // 256)
         return rounds * (4000.0 + 6.1 * sum(tile) * -(-k // 64))
 
-    block_m, block_n = min(_TILES, key=cost)
-    if (block_m, block_n) == _TILES[0]:
+    return min(tiles, key=cost)
+
+
+def _tile_config(tile: tuple[int, int], *, staged: bool = False) -> dict[str, BenchmarkScalar]:
+    """Metadata of a tile: K step 64 and a ring that fits the LDS, except the 256 x 256 kernel's."""
+    if tile == _TILES[0]:
         return TILE
-    stage = (block_m + block_n) * 128
-    stages = 81920 // stage if block_m + block_n <= 192 else min(5, 163840 // stage)
-    return {**TILE, "block_m": block_m, "block_n": block_n, "block_k": 64,
-            "group_m": 8 if block_n > block_m else 4, "num_stages": stages}
+    stage = sum(tile) * 128
+    stages = 81920 // stage if sum(tile) <= 192 else min(5, 163840 // stage)
+    return {**TILE, "block_m": tile[0], "block_n": tile[1], "block_k": 64,
+            "group_m": 8 if tile[1] > tile[0] else 4, "num_stages": 2 if staged else stages}
 
 
 def launch_config(a: torch.Tensor, b: torch.Tensor) -> dict[str, BenchmarkScalar]:
     """Tile configuration and MFMA of the kernel ``tk_gemm`` launches for ``a @ b``.
 
-    Mirrors ``gemm_dma::plan`` and ``pick_tile`` (csrc/gemm_dma.hip).
+    Mirrors ``gemm_dma::plan`` and ``pick_tile`` (csrc/gemm_dma.hip) and ``gemm_staged``
+    (csrc/gemm.hip).
     """
-    if not ((_dma_rows(a) or _dma_rows(a.t())) and (_dma_rows(b) or _dma_rows(b.t()))):
-        return {**FALLBACK_TILE,
-                "mma_opcode": _FALLBACK_MFMA.get(a.dtype, _FALLBACK_MFMA[torch.float16])}
     (m, k), n = a.shape, b.shape[1]
-    plain = _dma_rows(a) and _dma_rows(b) and k % 32 == 0
-    swapped = not _dma_rows(a) and not _dma_rows(b)  # computed as C^T = B^T A^T
-    return {**(_pick_tile(n, m, k) if swapped else _pick_tile(m, n, k)),
-            "hip_kernel": "gemm_dma_kernel" if plain else "gemm_kernel",
-            "mma_opcode": _MFMA.get(a.dtype, _MFMA[torch.float16])}
+    mma = {"mma_opcode": _MFMA.get(a.dtype, _MFMA[torch.float16])}
+    if (_dma_rows(a) or _dma_rows(a.t())) and (_dma_rows(b) or _dma_rows(b.t())):
+        plain = _dma_rows(a) and _dma_rows(b) and k % 32 == 0
+        swapped = not _dma_rows(a) and not _dma_rows(b)  # computed as C^T = B^T A^T
+        tile = _pick_tile(n, m, k) if swapped else _pick_tile(m, n, k)
+        return {**_tile_config(tile), **mma,
+                "hip_kernel": "gemm_dma_kernel" if plain else "gemm_kernel"}
+    (am, ak), (bk, bn) = a.stride(), b.stride()
+    unit = (all(1 in t.stride() and (t.shape[0] - 1) * t.stride(0)
+                + (t.shape[1] - 1) * t.stride(1) >= 7 for t in (a, b)))
+    swapped = ak != 1 and am == 1 and bn != 1 and bk == 1
+    tiles = _STAGED_TILES if unit else _STAGED_TILES[1:]
+    tile = _pick_tile(n, m, k, tiles) if swapped else _pick_tile(m, n, k, tiles)
+    return {**_tile_config(tile, staged=True), **mma, "hip_kernel": "gemm_kernel"}
 
 
 def _validate(a: torch.Tensor, b: torch.Tensor) -> None:
@@ -224,7 +230,7 @@ def _metadata_factory() -> BenchmarkMetadataFn:
 
     def metadata(size: int, dtype: torch.dtype) -> dict[str, BenchmarkScalar]:
         # Registry inputs are contiguous size x size matrices (size % 32 == 0).
-        return {**_pick_tile(size, size, size), "mma_opcode": _MFMA.get(dtype, _MFMA[torch.float16])}
+        return {**_tile_config(_pick_tile(size, size, size)), "mma_opcode": _MFMA.get(dtype, _MFMA[torch.float16])}
 
     return metadata
 
