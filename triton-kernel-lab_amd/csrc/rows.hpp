@@ -6,8 +6,9 @@
 // contiguous elements: vector i of thread `lane` covers columns
 // [(i*RT + lane)*VEC, +VEC). With VEC = 16/sizeof(T) every access is one
 // 128-bit load or store and a wave touches 1 KiB of contiguous row per
-// vector index; VEC = 1 is the fallback for rows whose base or stride is not
-// 16-byte aligned or whose width is not a multiple of VEC.
+// vector index. Rows whose base or stride is not 16-byte aligned, or whose width is not a
+// multiple of VEC, keep the vectors and access them at any element boundary (the *_any
+// functions); VEC = 1 is left to rows narrower than one vector.
 #pragma once
 
 #include "tk_common.hpp"
@@ -87,6 +88,170 @@ __device__ __forceinline__ void store_row_buf(T* row, int cols, int lane, const 
     for (int j = 0; j < VEC; ++j) r.v[j] = from_f32<T>(v[i * VEC + j]);
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, r), rs,
                                            uint32_t(c * int(sizeof(T))), 0, CPOL);
+  }
+}
+
+// 16-byte access at any element boundary (one dwordx4 instruction). Neighbouring lanes share the
+// lines, so loads keep the default policy (non-temporal ones: softmax fp16 16384 x 1001 12.0 ->
+// 14.6 us, bf16 4096 x 8191 24.4 -> 28.0, bf16 512 x 65535 39.0 -> 35.7); stores are streamed.
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+
+__device__ __forceinline__ u32x4 load_any(const void* p) {
+  return *static_cast<const u32x4_any*>(p);
+}
+__device__ __forceinline__ void store_any(void* p, u32x4 v) {
+  __builtin_nontemporal_store(v, static_cast<u32x4_any*>(p));
+}
+
+// Elements s .. of a 16-byte vector moved to its front (0 <= s < its length; zeros behind).
+template <int ES>
+__device__ __forceinline__ u32x4 drop_elements(u32x4 v, int s) {
+  const int words = s * ES / 4;
+  if (words & 2) v = u32x4{v[2], v[3], 0u, 0u};
+  if (words & 1) v = u32x4{v[1], v[2], v[3], 0u};
+  if constexpr (ES == 2)
+    if (s & 1)
+      v = u32x4{(v[0] >> 16) | (v[1] << 16), (v[1] >> 16) | (v[2] << 16),
+                (v[2] >> 16) | (v[3] << 16), v[3] >> 16};
+  return v;
+}
+
+// Vector of columns c .. c+VEC-1 of a row of `cols` columns. Every load has its VEC elements in
+// the row (near its end it starts at cols - VEC), with no branch around it, so all of a row's
+// loads are in flight at once; any_fix then moves the elements to their places and sets what
+// lies past the row to `fill` (the storage bits of one element). The row starts at least
+// VEC - cols elements after the first one of its tensor.
+template <typename T, int VEC>
+__device__ __forceinline__ u32x4 any_load(const T* row, int cols, int c) {
+  static_assert(VEC * sizeof(T) == 16, "16-byte vectors only");
+  return load_any(row + min(c, cols - VEC));
+}
+// `end`: one past the last column of the vectors the whole group loads together. It is uniform,
+// so the groups inside the row skip the work with a scalar branch.
+template <typename T, int VEC>
+__device__ __forceinline__ u32x4 any_fix(u32x4 v, int cols, int c, int end, uint32_t fill) {
+  if (end > cols) {
+    v = drop_elements<int(sizeof(T))>(v, min(max(c - (cols - VEC), 0), VEC - 1));
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      const bool in = c + j < cols;
+      if constexpr (sizeof(T) == 4)
+        v[j] = in ? v[j] : fill;
+      else if (j % 2)
+        v[j / 2] = in ? v[j / 2] : (v[j / 2] & 0xffffu) | (fill << 16);
+      else
+        v[j / 2] = in ? v[j / 2] : (v[j / 2] & 0xffff0000u) | fill;
+    }
+  }
+  return v;
+}
+template <typename T, int VEC>
+__device__ __forceinline__ void any_store(T* row, int cols, int c, int end, u32x4 v) {
+  if (end <= cols || c + VEC <= cols) {
+    store_any(row + c, v);
+  } else {
+    const Vec<T, VEC> e = __builtin_bit_cast(Vec<T, VEC>, v);
+#pragma unroll
+    for (int j = 0; j < VEC - 1; ++j)
+      if (c + j < cols) row[c + j] = e.v[j];
+  }
+}
+
+// Rows at any element boundary through aligned vectors: the row is taken to start `shift`
+// elements earlier, at the 16-byte boundary before it, and what lies outside it is set to `fill`
+// on loading and not stored. The buffer ends with the dword that holds the row's last element.
+// A group must cover cols + VEC - 1 columns (RT * VALS).
+template <typename T>
+__device__ __forceinline__ int row_shift(const T* row) {
+  return static_cast<int>((reinterpret_cast<uintptr_t>(row) & 15) / sizeof(T));
+}
+
+template <typename T, int VEC, int RT, int VALS, int CPOL>
+__device__ __forceinline__ void load_row_shift(const T* row, int shift, int cols, int lane,
+                                               float* v, float fill) {
+  static_assert(VEC * sizeof(T) == 16, "16-byte vectors only");
+  constexpr int ITEMS = VALS / VEC;
+  const int end = shift + cols;
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T*>(row - shift), (short)0, (uint32_t(end) * uint32_t(sizeof(T)) + 3) & ~3u,
+      0x00020000);
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const int c = (i * RT + lane) * VEC;
+    const Vec<T, VEC> r = __builtin_bit_cast(
+        Vec<T, VEC>, __builtin_amdgcn_raw_buffer_load_b128(rs, uint32_t(c * int(sizeof(T))), 0, CPOL));
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) v[i * VEC + j] = to_f32(r.v[j]);
+  }
+  // Only the first vectors and those past the row's end hold anything else (uniform branches).
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    if (i > 0 && (i + 1) * RT * VEC <= end) continue;
+    const int c = (i * RT + lane) * VEC;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j)
+      if (c + j < shift || c + j >= end) v[i * VEC + j] = fill;
+  }
+}
+
+template <typename T, int VEC, int RT, int VALS, int CPOL>
+__device__ __forceinline__ void store_row_shift(T* row, int shift, int cols, int lane,
+                                                const float* v) {
+  constexpr int ITEMS = VALS / VEC;
+  const int end = shift + cols;
+  T* base = row - shift;
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      base, (short)0, uint32_t(end) * uint32_t(sizeof(T)), 0x00020000);
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const int c = (i * RT + lane) * VEC;
+    Vec<T, VEC> r;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) r.v[j] = from_f32<T>(v[i * VEC + j]);
+    if ((i > 0 && (i + 1) * RT * VEC <= end) || (c >= shift && c + VEC <= end)) {
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, r), rs,
+                                             uint32_t(c * int(sizeof(T))), 0, CPOL);
+    } else {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j)
+        if (c + j >= shift && c + j < end) base[c + j] = r.v[j];
+    }
+  }
+}
+
+// load_row and store_row with 16-byte vectors at any element boundary; fill is -inf or 0.
+template <typename T, int VEC, int RT, int VALS>
+__device__ __forceinline__ void load_row_any(const T* row, int cols, int lane, float* v,
+                                             float fill) {
+  constexpr int ITEMS = VALS / VEC;
+  const T f = from_f32<T>(fill);
+  uint32_t bits;
+  if constexpr (sizeof(T) == 4)
+    bits = __builtin_bit_cast(uint32_t, f);
+  else
+    bits = __builtin_bit_cast(uint16_t, f);
+  u32x4 raw[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) raw[i] = any_load<T, VEC>(row, cols, (i * RT + lane) * VEC);
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const Vec<T, VEC> r = __builtin_bit_cast(
+        Vec<T, VEC>, any_fix<T, VEC>(raw[i], cols, (i * RT + lane) * VEC, (i + 1) * RT * VEC, bits));
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) v[i * VEC + j] = to_f32(r.v[j]);
+  }
+}
+
+template <typename T, int VEC, int RT, int VALS>
+__device__ __forceinline__ void store_row_any(T* row, int cols, int lane, const float* v) {
+  constexpr int ITEMS = VALS / VEC;
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    Vec<T, VEC> r;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) r.v[j] = from_f32<T>(v[i * VEC + j]);
+    any_store<T, VEC>(row, cols, (i * RT + lane) * VEC, (i + 1) * RT * VEC,
+                      __builtin_bit_cast(u32x4, r));
   }
 }
 
@@ -234,7 +399,56 @@ inline bool pick_row_shape(int64_t cols, RowShape* shape, int max_vals = 64) {
   return false;
 }
 
+// How a row kernel accesses its rows.
+enum class Access { kScalar, kAny, kShift, kAligned };
+
+// 16-byte vectors wherever a row has one.
+inline Access row_access(int dtype, int64_t cols, bool aligned) {
+  return aligned                          ? Access::kAligned
+         : cols >= 16 / elem_size(dtype) ? Access::kAny
+                                          : Access::kScalar;
+}
+
 }  // namespace tk
+
+// Expands `__VA_ARGS__` with constexpr VEC and ACCESS bound to `access`.
+#define TK_DISPATCH_ACCESS(T, access, ...)                                   \
+  if ((access) == tk::Access::kScalar) {                                     \
+    constexpr tk::Access ACCESS = tk::Access::kScalar;                       \
+    constexpr int VEC = 1;                                                   \
+    __VA_ARGS__;                                                             \
+  } else if ((access) == tk::Access::kAny) {                                 \
+    constexpr tk::Access ACCESS = tk::Access::kAny;                          \
+    constexpr int VEC = 16 / int(sizeof(T));                                 \
+    __VA_ARGS__;                                                             \
+  } else {                                                                   \
+    constexpr tk::Access ACCESS = tk::Access::kAligned;                      \
+    constexpr int VEC = 16 / int(sizeof(T));                                 \
+    __VA_ARGS__;                                                             \
+  }
+
+// Expands `__VA_ARGS__` with constexpr VEC, ACCESS, RT and VALS bound to `access` and `shape`
+// (scalar rows are narrower than one vector: a single shape; shifted ones take 1024 threads).
+#define TK_DISPATCH_ROWS(T, access, shape, ...)                              \
+  if ((access) == tk::Access::kScalar) {                                     \
+    constexpr tk::Access ACCESS = tk::Access::kScalar;                       \
+    constexpr int VEC = 1, RT = 64, VALS = 16;                               \
+    __VA_ARGS__;                                                             \
+  } else if ((access) == tk::Access::kAny) {                                 \
+    constexpr tk::Access ACCESS = tk::Access::kAny;                          \
+    constexpr int VEC = 16 / int(sizeof(T));                                 \
+    TK_DISPATCH_ROW_SHAPE(shape, __VA_ARGS__)                                \
+  } else if ((access) == tk::Access::kShift) {                               \
+    constexpr tk::Access ACCESS = tk::Access::kShift;                        \
+    constexpr int VEC = 16 / int(sizeof(T)), RT = 1024;                      \
+    if ((shape).vals == 16) { constexpr int VALS = 16; __VA_ARGS__; }        \
+    else if ((shape).vals == 32) { constexpr int VALS = 32; __VA_ARGS__; }   \
+    else { constexpr int VALS = 64; __VA_ARGS__; }                           \
+  } else {                                                                   \
+    constexpr tk::Access ACCESS = tk::Access::kAligned;                      \
+    constexpr int VEC = 16 / int(sizeof(T));                                 \
+    TK_DISPATCH_ROW_SHAPE(shape, __VA_ARGS__)                                \
+  }
 
 // Expands `__VA_ARGS__` with constexpr RT and VALS bound to `shape`.
 #define TK_DISPATCH_ROW_SHAPE(shape, ...)                                \

@@ -39,7 +39,12 @@ __device__ __forceinline__ void softmax_row(float* v, float* scratch) {
 // 23.2-23.6 us; three or four rows per wave through two register buffers 27-29 us (too
 // few waves per SIMD). One row group per workgroup (a single wave for rows of up to 4096
 // columns): 23.5-23.7 us against 23.9-24.0 us with four single-wave groups per workgroup.
-template <typename T, int VEC, int RT, int VALS, int P>
+//
+// Rows at any element boundary (odd widths) keep the 16-byte vectors, through load_row_any or,
+// 1024 threads wide, load_row_shift. With one element per access bf16 2048 x 32001 ran 157 us
+// (now 58, 4.6 TB/s), 2048 x 50257 530 us (95), 4096 x 8191 64 us (33), fp16 16384 x 1001 23 us
+// (12).
+template <typename T, int VEC, tk::Access ACCESS, int RT, int VALS, int P>
 __global__ __launch_bounds__(RT) void softmax_fwd_kernel(
     const T* __restrict__ x, T* __restrict__ y, int rows, int cols, int64_t x_stride,
     int64_t y_stride) {
@@ -49,7 +54,7 @@ __global__ __launch_bounds__(RT) void softmax_fwd_kernel(
   // Rows of 16-byte vectors are streamed once: non-temporal buffer loads and stores
   // (f32 4096 x 4096 went from 4.9 to 5.9 TB/s). The row index is wave-uniform and
   // readfirstlane lets the compiler keep each row's buffer resource scalar.
-  constexpr bool kBuf = VEC * sizeof(T) == 16;
+  constexpr bool kBuf = ACCESS == tk::Access::kAligned;
   const int row0 = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * P);
   if (row0 >= rows) return;  // the whole workgroup: row0 is uniform
 
@@ -61,6 +66,11 @@ __global__ __launch_bounds__(RT) void softmax_fwd_kernel(
     if constexpr (kBuf)
       tk::load_row_buf<T, VEC, RT, VALS, tk::kCpolStream>(x + r * x_stride, cols, lane, v[p],
                                                            -INFINITY);
+    else if constexpr (ACCESS == tk::Access::kShift)
+      tk::load_row_shift<T, VEC, RT, VALS, tk::kCpolStream>(
+          x + r * x_stride, tk::row_shift(x + r * x_stride), cols, lane, v[p], -INFINITY);
+    else if constexpr (ACCESS == tk::Access::kAny)
+      tk::load_row_any<T, VEC, RT, VALS>(x + r * x_stride, cols, lane, v[p], -INFINITY);
     else
       tk::load_row<T, VEC, RT, VALS>(x + r * x_stride, cols, lane, v[p], -INFINITY);
   }
@@ -71,6 +81,11 @@ __global__ __launch_bounds__(RT) void softmax_fwd_kernel(
     if (r >= rows) break;
     if constexpr (kBuf)
       tk::store_row_buf<T, VEC, RT, VALS, tk::kCpolStream>(y + r * y_stride, cols, lane, v[p]);
+    else if constexpr (ACCESS == tk::Access::kShift)
+      tk::store_row_shift<T, VEC, RT, VALS, tk::kCpolStream>(
+          y + r * y_stride, tk::row_shift(y + r * y_stride), cols, lane, v[p]);
+    else if constexpr (ACCESS == tk::Access::kAny)
+      tk::store_row_any<T, VEC, RT, VALS>(y + r * y_stride, cols, lane, v[p]);
     else
       tk::store_row<T, VEC, RT, VALS>(y + r * y_stride, cols, lane, v[p]);
   }
@@ -97,15 +112,27 @@ constexpr int kOnlineChunk = kOnlineThreads * kOnlineVals;  // 16384 columns
 
 // The first read keeps the default cache policy (a chunk may still be in the
 // last-level cache when the second pass reads it); the second read is the last use.
-template <typename T, int VEC, int CPOL>
+template <typename T, int VEC, tk::Access ACCESS, int CPOL>
 __device__ __forceinline__ void load_chunk(const T* p, int n, int lane, float* v) {
-  if constexpr (VEC * sizeof(T) == 16)
+  if constexpr (ACCESS == tk::Access::kAligned)
     tk::load_row_buf<T, VEC, kOnlineThreads, kOnlineVals, CPOL>(p, n, lane, v, -INFINITY);
+  else if constexpr (ACCESS == tk::Access::kAny)
+    tk::load_row_any<T, VEC, kOnlineThreads, kOnlineVals>(p, n, lane, v, -INFINITY);
   else
     tk::load_row<T, VEC, kOnlineThreads, kOnlineVals>(p, n, lane, v, -INFINITY);
 }
 
-template <typename T, int VEC>
+template <typename T, int VEC, tk::Access ACCESS>
+__device__ __forceinline__ void store_chunk(T* p, int n, int lane, const float* v) {
+  if constexpr (ACCESS == tk::Access::kAligned)
+    tk::store_row_buf<T, VEC, kOnlineThreads, kOnlineVals, tk::kCpolStream>(p, n, lane, v);
+  else if constexpr (ACCESS == tk::Access::kAny)
+    tk::store_row_any<T, VEC, kOnlineThreads, kOnlineVals>(p, n, lane, v);
+  else
+    tk::store_row<T, VEC, kOnlineThreads, kOnlineVals>(p, n, lane, v);
+}
+
+template <typename T, int VEC, tk::Access ACCESS>
 __global__ __launch_bounds__(kOnlineThreads) void softmax_online_partial_kernel(
     const T* __restrict__ x, float* __restrict__ partials, int cols, int chunks,
     int64_t x_stride) {
@@ -115,7 +142,7 @@ __global__ __launch_bounds__(kOnlineThreads) void softmax_online_partial_kernel(
   const int c0 = chunk * kOnlineChunk;
   const int n = min(kOnlineChunk, cols - c0);
   float v[kOnlineVals];
-  load_chunk<T, VEC, tk::kCpolDefault>(x + row * x_stride + c0, n, threadIdx.x, v);
+  load_chunk<T, VEC, ACCESS, tk::kCpolDefault>(x + row * x_stride + c0, n, threadIdx.x, v);
   float m = v[0];
 #pragma unroll
   for (int e = 1; e < kOnlineVals; ++e) m = fmaxf(m, v[e]);
@@ -133,7 +160,7 @@ __global__ __launch_bounds__(kOnlineThreads) void softmax_online_partial_kernel(
   }
 }
 
-template <typename T, int VEC>
+template <typename T, int VEC, tk::Access ACCESS>
 __global__ __launch_bounds__(kOnlineThreads) void softmax_online_apply_kernel(
     const T* __restrict__ x, T* __restrict__ y, const float* __restrict__ partials, int cols,
     int chunks, int64_t x_stride, int64_t y_stride) {
@@ -143,7 +170,7 @@ __global__ __launch_bounds__(kOnlineThreads) void softmax_online_apply_kernel(
   const int c0 = chunk * kOnlineChunk;
   const int n = min(kOnlineChunk, cols - c0);
   float v[kOnlineVals];
-  load_chunk<T, VEC, tk::kCpolStream>(x + row * x_stride + c0, n, threadIdx.x, v);
+  load_chunk<T, VEC, ACCESS, tk::kCpolStream>(x + row * x_stride + c0, n, threadIdx.x, v);
   // Row statistics from the chunk partials, in a fixed order (identical in every
   // workgroup of the row).
   const float* pr = partials + 2 * static_cast<int64_t>(row) * chunks;
@@ -160,11 +187,7 @@ __global__ __launch_bounds__(kOnlineThreads) void softmax_online_apply_kernel(
 #pragma unroll
   for (int e = 0; e < kOnlineVals; ++e) v[e] = tk::hw_exp(v[e] - m) * inv;
   T* yr = y + row * y_stride + c0;
-  if constexpr (VEC * sizeof(T) == 16)
-    tk::store_row_buf<T, VEC, kOnlineThreads, kOnlineVals, tk::kCpolStream>(yr, n, threadIdx.x,
-                                                                             v);
-  else
-    tk::store_row<T, VEC, kOnlineThreads, kOnlineVals>(yr, n, threadIdx.x, v);
+  store_chunk<T, VEC, ACCESS>(yr, n, threadIdx.x, v);
 }
 
 // ------------------------------------------------------------------ single-read online softmax
@@ -213,13 +236,16 @@ __device__ __forceinline__ void chunk_partial(const float* v, float* scratch, fl
 // same values in the same order (element e of the thread is column
 // ((e / VEC) * 256 + thread) * VEC + e % VEC), read twice, one vector at a time. Used only
 // when the bounded wait expires, so it trades reads for registers.
-template <typename T, int VEC>
+template <typename T, int VEC, tk::Access ACCESS>
 __device__ __forceinline__ void chunk_partial_streamed(const T* p, int n, float* scratch,
                                                        float& m, float& s) {
   constexpr int ITEMS = kOnlineVals / VEC;
   auto item = [&](int i, float* f) {
     const int c = (i * kOnlineThreads + static_cast<int>(threadIdx.x)) * VEC;
-    if (c < n) {
+    if (ACCESS == tk::Access::kAny || c + VEC > n) {
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) f[k] = c + k < n ? tk::to_f32(p[c + k]) : -INFINITY;
+    } else if (c < n) {
       tk::load_vec<T, VEC>(p + c, f);
     } else {
 #pragma unroll
@@ -269,7 +295,7 @@ __global__ __launch_bounds__(256) void online_clear_kernel(uint64_t* __restrict_
 
 // Five waves per SIMD (96 registers) where the chunk fits without spills (float32 and bfloat16
 // 16-byte vectors: f32 64 x 1048576 0.1022 vs 0.1033 ms at four).
-template <typename T, int VEC>
+template <typename T, int VEC, tk::Access ACCESS>
 __global__ __launch_bounds__(kOnlineThreads)
 __attribute__((amdgpu_waves_per_eu(VEC == 1 ? 3 : __is_same(T, _Float16) ? 4 : 5))) void
 softmax_online_single_read_kernel(
@@ -283,7 +309,7 @@ softmax_online_single_read_kernel(
   float v[kOnlineVals];
   {
     const int c0 = chunk * kOnlineChunk;
-    load_chunk<T, VEC, tk::kCpolStream>(xr + c0, min(kOnlineChunk, cols - c0), threadIdx.x, v);
+    load_chunk<T, VEC, ACCESS, tk::kCpolStream>(xr + c0, min(kOnlineChunk, cols - c0), threadIdx.x, v);
   }
   float m, s;
   chunk_partial(v, scratch, m, s);
@@ -318,7 +344,7 @@ softmax_online_single_read_kernel(
     for (int j = 0; j < chunks; ++j) {
       const int c0 = j * kOnlineChunk;
       float mk, sk;
-      chunk_partial_streamed<T, VEC>(xr + c0, min(kOnlineChunk, cols - c0), scratch, mk, sk);
+      chunk_partial_streamed<T, VEC, ACCESS>(xr + c0, min(kOnlineChunk, cols - c0), scratch, mk, sk);
       if (threadIdx.x == 0) {
         fallback[2 * j] = mk;
         fallback[2 * j + 1] = sk;
@@ -338,10 +364,7 @@ softmax_online_single_read_kernel(
   const int c0 = chunk * kOnlineChunk;
   const int n = min(kOnlineChunk, cols - c0);
   T* yr = y + row * y_stride + c0;
-  if constexpr (VEC * sizeof(T) == 16)
-    tk::store_row_buf<T, VEC, kOnlineThreads, kOnlineVals, tk::kCpolStream>(yr, n, threadIdx.x, v);
-  else
-    tk::store_row<T, VEC, kOnlineThreads, kOnlineVals>(yr, n, threadIdx.x, v);
+  store_chunk<T, VEC, ACCESS>(yr, n, threadIdx.x, v);
 }
 
 }  // namespace
@@ -364,6 +387,7 @@ extern "C" int tk_softmax_online_fwd(int dtype, const void* x, void* y, float* p
   const int vec = 16 / es;
   const bool vector_ok = tk::aligned16(x) && tk::aligned16(y) && cols % vec == 0 &&
                          (x_row_stride * es) % 16 == 0 && (y_row_stride * es) % 16 == 0;
+  const tk::Access access = tk::row_access(dtype, cols, vector_ok);
   const dim3 grid(static_cast<unsigned>(rows * chunks));
   const dim3 block(kOnlineThreads);
   hipStream_t s = tk::as_stream(stream);
@@ -379,18 +403,18 @@ extern "C" int tk_softmax_online_fwd(int dtype, const void* x, void* y, float* p
     hipLaunchKernelGGL(online_clear_kernel, dim3(clear_blocks), dim3(256), 0, s,
                        reinterpret_cast<uint64_t*>(partials), words);
     TK_DISPATCH_DTYPE(dtype, T,
-      TK_DISPATCH_VEC(T, vector_ok,
-        hipLaunchKernelGGL((softmax_online_single_read_kernel<T, VEC>), grid, block, 0, s,
+      TK_DISPATCH_ACCESS(T, access,
+        hipLaunchKernelGGL((softmax_online_single_read_kernel<T, VEC, ACCESS>), grid, block, 0, s,
                            static_cast<const T*>(x), static_cast<T*>(y), partials, (int)cols,
                            (int)chunks, x_row_stride, y_row_stride, polls)));
     return tk::check_launch("online softmax");
   }
   TK_DISPATCH_DTYPE(dtype, T,
-    TK_DISPATCH_VEC(T, vector_ok,
-      hipLaunchKernelGGL((softmax_online_partial_kernel<T, VEC>), grid, block, 0, s,
+    TK_DISPATCH_ACCESS(T, access,
+      hipLaunchKernelGGL((softmax_online_partial_kernel<T, VEC, ACCESS>), grid, block, 0, s,
                          static_cast<const T*>(x), partials, (int)cols, (int)chunks,
                          x_row_stride);
-      hipLaunchKernelGGL((softmax_online_apply_kernel<T, VEC>), grid, block, 0, s,
+      hipLaunchKernelGGL((softmax_online_apply_kernel<T, VEC, ACCESS>), grid, block, 0, s,
                          static_cast<const T*>(x), static_cast<T*>(y), partials, (int)cols,
                          (int)chunks, x_row_stride, y_row_stride)));
   return tk::check_launch("online softmax");
@@ -412,22 +436,35 @@ extern "C" int tk_softmax_fwd(int dtype, const void* x, void* y, int64_t rows, i
   const int vec = 16 / es;
   const bool vector_ok = tk::aligned16(x) && tk::aligned16(y) && cols % vec == 0 &&
                          (x_row_stride * es) % 16 == 0 && (y_row_stride * es) % 16 == 0;
+  tk::Access access = tk::row_access(dtype, cols, vector_ok);
+  // Rows of 1024 threads go through aligned vectors on shifted rows when every x row starts at
+  // the same place between two 16-byte boundaries as its y row (contiguous tensors do): bf16
+  // 2048 x 32001 58.7 us against 66.6 us with vectors at any boundary, 2048 x 50257 95 against
+  // 120. Narrower rows pay more for the element stores at their ends: fp16 16384 x 1001 15.5
+  // against 12.0 us, f32 4096 x 4097 25.1 against 23.3.
+  tk::RowShape shifted;
+  if (access == tk::Access::kAny &&
+      (reinterpret_cast<uintptr_t>(x) - reinterpret_cast<uintptr_t>(y)) % 16 == 0 &&
+      reinterpret_cast<uintptr_t>(x) % es == 0 && ((x_row_stride - y_row_stride) * es) % 16 == 0 &&
+      tk::pick_row_shape(cols + vec - 1, &shifted) && shifted.rt == 1024) {
+    access = tk::Access::kShift;
+    shape = shifted;
+  }
   // Two single-wave rows per wave once that still leaves two waves per SIMD (4096 rows).
   const bool pair = shape.rt == 64 && rows >= 4096;
   const dim3 grid(static_cast<unsigned>(tk::cdiv(rows, pair ? 2 : 1)));
   const dim3 block(shape.rt);
   hipStream_t s = tk::as_stream(stream);
   TK_DISPATCH_DTYPE(dtype, T,
-    TK_DISPATCH_VEC(T, vector_ok,
-      TK_DISPATCH_ROW_SHAPE(shape,
+    TK_DISPATCH_ROWS(T, access, shape,
         constexpr int P2 = RT == 64 ? 2 : 1;
         if (pair)
-          hipLaunchKernelGGL((softmax_fwd_kernel<T, VEC, RT, VALS, P2>), grid, block, 0, s,
+          hipLaunchKernelGGL((softmax_fwd_kernel<T, VEC, ACCESS, RT, VALS, P2>), grid, block, 0, s,
                              static_cast<const T*>(x), static_cast<T*>(y), (int)rows, (int)cols,
                              x_row_stride, y_row_stride);
         else
-          hipLaunchKernelGGL((softmax_fwd_kernel<T, VEC, RT, VALS, 1>), grid, block, 0, s,
+          hipLaunchKernelGGL((softmax_fwd_kernel<T, VEC, ACCESS, RT, VALS, 1>), grid, block, 0, s,
                              static_cast<const T*>(x), static_cast<T*>(y), (int)rows, (int)cols,
-                             x_row_stride, y_row_stride))));
+                             x_row_stride, y_row_stride)));
   return tk::check_launch("softmax");
 }
