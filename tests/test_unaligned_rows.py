@@ -73,3 +73,48 @@ def test_online_softmax_of_short_last_chunks(cols, monkeypatch) -> None:
     assert_close(got, torch.softmax(x.double(), dim=-1))
     monkeypatch.setenv("TKLAB_ONLINE_SOFTMAX_POLLS", "0")
     assert bits_equal(online_softmax(x), got)
+
+
+def _norm_step(x, r, w, ds, dy):
+    """Forward and backward through the private launchers into NaN-surrounded odd rows."""
+    from tklab.kernels import residual_rms_norm as rrn
+    from tklab.kernels import rms_norm as rn
+
+    rows, cols = x.shape
+    s, y = _odd_rows(rows, cols, x.dtype, 0), _odd_rows(rows, cols, x.dtype, 0, offset=5)
+    rstd = torch.empty(rows, device="cuda")
+    rrn._launch_forward(x, r, w, s, y, rstd, eps=1e-6, store_residual=True, store_stats=True)
+    dx, dw = rn._launch_backward(dy, s, w, rstd, incoming_dx=ds)
+    assert torch.isnan(_tail(s[:-1], cols)).all() and torch.isnan(_tail(y[:-1], cols)).all()
+    return s, y, rstd, dx, dw
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize(("rows", "cols"), [(1, 3), (2, 8), (7, 9), (300, 65), (1000, 257), (513, 1023),
+                                            (300, 1025), (260, 4097), (771, 2049), (3, 8193),
+                                            (257, 16383), (2, 12345), (600, 1024)])
+def test_residual_rms_norm(dtype, rows, cols) -> None:
+    if cols * torch.empty((), dtype=dtype).element_size() > 65536:
+        pytest.skip("row past the fused limit")
+    x, r, ds, dy = (_odd_rows(rows, cols, dtype, seed=i) for i in range(1, 5))
+    w = _odd_rows(2, cols, dtype, seed=9)[0]
+    s, y, rstd, dx, dw = _norm_step(x, r, w, ds, dy)
+    s64 = s.double()
+    assert bits_equal(s, (x.float() + r.float()).to(dtype))
+    rstd64 = torch.rsqrt(s64.square().mean(-1) + 1e-6)
+    torch.testing.assert_close(rstd.double(), rstd64, rtol=1e-5, atol=0)
+    unit, g = s64 * rstd64[:, None], dy.double() * w.double()
+    assert_close(y, unit * w.double())
+    assert_close(dx, rstd64[:, None] * (g - unit * (g * unit).mean(-1, keepdim=True)) + ds.double())
+    want = (dy.double() * unit).sum(0)
+    error = (dw.double() - want).norm() / want.norm()
+    assert error < (1e-5 if dtype == torch.float32 else 1e-2), error
+    if cols % 8 == 0:  # the same vectors as on aligned rows
+        aligned = [t.contiguous().clone() for t in (x, r, w, ds, dy)]
+        from tklab.kernels.residual_rms_norm import residual_rms_norm
+
+        ax, ar, aw = (t.requires_grad_() for t in aligned[:3])
+        as_, ay = residual_rms_norm(ax, ar, aw, 1e-6)
+        adx, _, adw = torch.autograd.grad((as_, ay), (ax, ar, aw), aligned[3:])
+        for got, same in ((s, as_), (y, ay), (dx, adx), (dw, adw)):
+            assert bits_equal(got, same)

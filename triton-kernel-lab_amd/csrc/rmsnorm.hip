@@ -26,7 +26,11 @@ namespace {
 
 constexpr int kNormBlock = 256;
 
-template <typename T, int VEC, int RT, int VALS>
+// Rows at any element boundary (odd widths) keep the 16-byte vectors, here and in the backward
+// stage 1 with its pipeline (RawRow::load_any). With one element per access the residual step
+// (forward, stages 1 and 2) ran bf16 16384 x 4095 in 1135 us; now 239 us (4096 columns: 174),
+// fp16 2000 x 5043 238 -> 164 us (the host's time), f32 16384 x 2001 237 -> 215 us.
+template <typename T, int VEC, tk::Access ACCESS, int RT, int VALS>
 __global__ __launch_bounds__(RT >= kNormBlock ? RT : kNormBlock) void rmsnorm_fwd_kernel(
     const T* __restrict__ x, const T* __restrict__ residual, const T* __restrict__ weight,
     T* __restrict__ residual_sum, T* __restrict__ y, float* __restrict__ rstd_out, int rows,
@@ -36,7 +40,7 @@ __global__ __launch_bounds__(RT >= kNormBlock ? RT : kNormBlock) void rmsnorm_fw
   __shared__ float scratch[RT / 64];
   // 16-byte rows go through buffer accesses with per-stream cache policies: the
   // inputs are streamed (non-temporal), the outputs stored with sc1.
-  constexpr bool kBuf = VEC * sizeof(T) == 16;
+  constexpr bool kBuf = ACCESS == tk::Access::kAligned, kAny = ACCESS == tk::Access::kAny;
   const int lane = threadIdx.x % RT;
   // A wave's threads share one row (RT >= 64); readfirstlane makes that visible to
   // the compiler, so the row's buffer resource lives in scalar registers.
@@ -47,22 +51,32 @@ __global__ __launch_bounds__(RT >= kNormBlock ? RT : kNormBlock) void rmsnorm_fw
   Row sv;
   if constexpr (kBuf)
     sv.template load_buf<tk::kCpolStream>(x + row * x_stride, cols, lane);
+  else if constexpr (kAny)
+    sv.load_any(x + row * x_stride, cols, lane);
   else
     sv.load(x + row * x_stride, cols, lane);
   if (residual != nullptr) {
     Row rv;
     if constexpr (kBuf)
       rv.template load_buf<tk::kCpolStream>(residual + row * r_stride, cols, lane);
+    else if constexpr (kAny)
+      rv.load_any(residual + row * r_stride, cols, lane);
     else
       rv.load(residual + row * r_stride, cols, lane);
+    if constexpr (kAny) rv.fix_any(cols, lane);
+    if constexpr (kAny) sv.fix_any(cols, lane);
 #pragma unroll
     for (int e = 0; e < VALS; ++e) sv.set(e, sv.get(e) + rv.get(e));
     if (residual_sum != nullptr) {
       if constexpr (kBuf)
         sv.template store_buf<tk::kCpolSc1>(residual_sum + row * s_stride, cols, lane);
+      else if constexpr (kAny)
+        sv.store_any(residual_sum + row * s_stride, cols, lane);
       else
         sv.store(residual_sum + row * s_stride, cols, lane);
     }
+  } else if constexpr (kAny) {
+    sv.fix_any(cols, lane);
   }
 
   float ss = 0.f;
@@ -75,11 +89,18 @@ __global__ __launch_bounds__(RT >= kNormBlock ? RT : kNormBlock) void rmsnorm_fw
   // rstd and the weight itself (the row-scaled GEMM).
   if (y != nullptr) {
     Row wv;
-    wv.load(weight, cols, lane);
+    if constexpr (kAny) {
+      wv.load_any(weight, cols, lane);
+      wv.fix_any(cols, lane);
+    } else {
+      wv.load(weight, cols, lane);
+    }
 #pragma unroll
     for (int e = 0; e < VALS; ++e) wv.set(e, sv.get(e) * rstd * wv.get(e));
     if constexpr (kBuf)
       wv.template store_buf<tk::kCpolSc1>(y + row * y_stride, cols, lane);
+    else if constexpr (kAny)
+      wv.store_any(y + row * y_stride, cols, lane);
     else
       wv.store(y + row * y_stride, cols, lane);
   }
@@ -125,13 +146,29 @@ __device__ __forceinline__ void load_rowset_buf(RowSet<Row>& s, const RowPtrs<T>
   s.r = rstd[row];
 }
 
+// The same at any element boundary (rows are clamped to the group's last one instead of read with
+// no extent); stage1_row puts the elements in place.
+template <typename T, typename Row>
+__device__ __forceinline__ void load_rowset_any(RowSet<Row>& s, const RowPtrs<T>& p, int64_t row,
+                                                int cols, int lane, const float* rstd) {
+  s.x.load_any(p.x + row * p.xs, cols, lane);
+  s.dy.load_any(p.dy + row * p.dys, cols, lane);
+  if (p.inc != nullptr) s.inc.load_any(p.inc + row * p.incs, cols, lane);
+  s.r = rstd[row];
+}
+
 // dx of one row and its dweight contribution: x_hat = x*rstd, g = w*dy,
 // dx = rstd*(g - x_hat*mean(g*x_hat)) (+ incoming), acc += dy*x_hat. Every thread of the
 // row group calls it (group_allreduce holds block barriers for multi-wave rows).
-template <typename T, int VEC, int RT, int VALS, bool ACC_LDS, typename Row>
+template <typename T, int VEC, tk::Access ACCESS, int RT, int VALS, bool ACC_LDS, typename Row>
 __device__ __forceinline__ void stage1_row(RowSet<Row>& s, const Row& wv, const RowPtrs<T>& p,
                                            int64_t row, int cols, int lane, float* acc,
                                            float* fold, float* scratch) {
+  if constexpr (ACCESS == tk::Access::kAny) {
+    s.x.fix_any(cols, lane);
+    s.dy.fix_any(cols, lane);
+    if (p.inc != nullptr) s.inc.fix_any(cols, lane);
+  }
   float dot = 0.f;
 #pragma unroll
   for (int e = 0; e < VALS; ++e) {
@@ -153,8 +190,10 @@ __device__ __forceinline__ void stage1_row(RowSet<Row>& s, const Row& wv, const 
     if (p.inc != nullptr) v += s.inc.get(e);
     s.x.set(e, v);
   }
-  if constexpr (VEC * sizeof(T) == 16)
+  if constexpr (ACCESS == tk::Access::kAligned)
     s.x.template store_buf<tk::kCpolStream>(p.dx + row * p.dxs, cols, lane);
+  else if constexpr (ACCESS == tk::Access::kAny)
+    s.x.store_any(p.dx + row * p.dxs, cols, lane);
   else
     s.x.store(p.dx + row * p.dxs, cols, lane);
 }
@@ -164,7 +203,7 @@ __device__ __forceinline__ void stage1_row(RowSet<Row>& s, const Row& wv, const 
 template <int RT>
 constexpr int bwd_block() { return RT == 64 ? 256 : RT; }
 
-template <typename T, int VEC, int RT, int VALS>
+template <typename T, int VEC, tk::Access ACCESS, int RT, int VALS>
 __global__ __launch_bounds__(bwd_block<RT>()) void rmsnorm_bwd_stage1_kernel(
     T* __restrict__ dx, const T* __restrict__ dy, const T* __restrict__ incoming,
     float* __restrict__ partial, const T* __restrict__ x, const T* __restrict__ weight,
@@ -206,13 +245,19 @@ __global__ __launch_bounds__(bwd_block<RT>()) void rmsnorm_bwd_stage1_kernel(
 
   // The weight row is loaded once, before any row: a load issued after the prefetches
   // would make its wait (in-order vmcnt) wait for them too.
+  constexpr bool kAny = ACCESS == tk::Access::kAny;
   Row wv;
-  wv.load(weight, cols, lane);
+  if constexpr (kAny) {
+    wv.load_any(weight, cols, lane);
+    wv.fix_any(cols, lane);
+  } else {
+    wv.load(weight, cols, lane);
+  }
   const RowPtrs<T> ptr{x, dy, incoming, dx, x_stride, dy_stride, inc_stride, dx_stride};
   if (group_rows == 0) {
     // A group past the last row owns no rows (the entry points launch min(G, rows)
     // groups, so none does); it would only write a zero partial row.
-  } else if constexpr (RT < 1024 && VEC * sizeof(T) == 16) {
+  } else if constexpr (RT < 1024 && ACCESS != tk::Access::kScalar) {
     // Software pipeline, unrolled by three so the three row buffers rotate roles
     // without register copies (a copy would wait for the load still in flight): the
     // loads of the next two rows of this slot overlap the current row's reduction.
@@ -222,20 +267,26 @@ __global__ __launch_bounds__(bwd_block<RT>()) void rmsnorm_bwd_stage1_kernel(
     RowSet<Row> ra, rb, rc;
     const int last = max(group_rows - 1, 0);
     auto rowk = [&](int k) { return row_of(min(k, last)); };
-    auto extent = [&](int k) { return k < group_rows ? cols : 0; };
+    auto extent = [&](int k) { return kAny || k < group_rows ? cols : 0; };
+    auto load = [&](RowSet<Row>& s, int k) {
+      if constexpr (kAny)
+        load_rowset_any<T>(s, ptr, rowk(k), extent(k), lane, rstd);
+      else
+        load_rowset_buf<T>(s, ptr, rowk(k), extent(k), lane, rstd);
+    };
     const int k0 = slot;
-    load_rowset_buf<T>(ra, ptr, rowk(k0), extent(k0), lane, rstd);
-    load_rowset_buf<T>(rb, ptr, rowk(k0 + SLOTS), extent(k0 + SLOTS), lane, rstd);
+    load(ra, k0);
+    load(rb, k0 + SLOTS);
     for (int k = k0; k < group_rows; k += 3 * SLOTS) {
-      load_rowset_buf<T>(rc, ptr, rowk(k + 2 * SLOTS), extent(k + 2 * SLOTS), lane, rstd);
-      stage1_row<T, VEC, RT, VALS, ACC_LDS>(ra, wv, ptr, row_of(k), cols, lane, acc, fold, scratch);
+      load(rc, k + 2 * SLOTS);
+      stage1_row<T, VEC, ACCESS, RT, VALS, ACC_LDS>(ra, wv, ptr, row_of(k), cols, lane, acc, fold, scratch);
       if (k + SLOTS >= group_rows) break;
-      load_rowset_buf<T>(ra, ptr, rowk(k + 3 * SLOTS), extent(k + 3 * SLOTS), lane, rstd);
-      stage1_row<T, VEC, RT, VALS, ACC_LDS>(rb, wv, ptr, row_of(k + SLOTS), cols, lane, acc, fold,
+      load(ra, k + 3 * SLOTS);
+      stage1_row<T, VEC, ACCESS, RT, VALS, ACC_LDS>(rb, wv, ptr, row_of(k + SLOTS), cols, lane, acc, fold,
                                             scratch);
       if (k + 2 * SLOTS >= group_rows) break;
-      load_rowset_buf<T>(rb, ptr, rowk(k + 4 * SLOTS), extent(k + 4 * SLOTS), lane, rstd);
-      stage1_row<T, VEC, RT, VALS, ACC_LDS>(rc, wv, ptr, row_of(k + 2 * SLOTS), cols, lane, acc,
+      load(rb, k + 4 * SLOTS);
+      stage1_row<T, VEC, ACCESS, RT, VALS, ACC_LDS>(rc, wv, ptr, row_of(k + 2 * SLOTS), cols, lane, acc,
                                             fold, scratch);
     }
   } else {
@@ -243,8 +294,11 @@ __global__ __launch_bounds__(bwd_block<RT>()) void rmsnorm_bwd_stage1_kernel(
     // one row at a time.
     RowSet<Row> ra;
     for (int k = slot; k < group_rows; k += SLOTS) {
-      load_rowset<T>(ra, ptr, row_of(k), cols, lane, rstd);
-      stage1_row<T, VEC, RT, VALS, ACC_LDS>(ra, wv, ptr, row_of(k), cols, lane, acc, fold, scratch);
+      if constexpr (kAny)
+        load_rowset_any<T>(ra, ptr, row_of(k), cols, lane, rstd);
+      else
+        load_rowset<T>(ra, ptr, row_of(k), cols, lane, rstd);
+      stage1_row<T, VEC, ACCESS, RT, VALS, ACC_LDS>(ra, wv, ptr, row_of(k), cols, lane, acc, fold, scratch);
     }
   }
 
@@ -314,14 +368,12 @@ bool rows_vector_ok(int dtype, int64_t cols, std::initializer_list<const void*> 
   return true;
 }
 
-int check_rows(const char* what, int dtype, int64_t rows, int64_t cols, bool vector_ok,
-               tk::RowShape* shape) {
+int check_rows(const char* what, int dtype, int64_t rows, int64_t cols, tk::RowShape* shape) {
   if (!tk::valid_dtype(dtype)) return tk::fail("%s: unsupported dtype code %d", what, dtype);
   if (rows <= 0 || cols <= 0) return tk::fail("%s: empty problem", what);
   if (rows > INT32_MAX) return tk::fail("%s: too many rows", what);
-  // At most 32 registers per row tensor per thread: 64 packed 16-bit values,
-  // 32 float32 values, or 32 unpacked values on the unaligned scalar path.
-  const int max_vals = vector_ok ? 128 / tk::elem_size(dtype) : 32;
+  // At most 32 registers per row tensor per thread: 64 packed 16-bit or 32 float32 values.
+  const int max_vals = 128 / tk::elem_size(dtype);
   if (cols * tk::elem_size(dtype) > 65536 || !tk::pick_row_shape(cols, shape, max_vals))
     return tk::fail("%s: feature row exceeds the 65536-byte fused limit", what);
   return 0;
@@ -346,7 +398,8 @@ extern "C" int tk_rmsnorm_fwd(int dtype, const void* x, const void* residual, co
       {x_row_stride, residual ? residual_row_stride : 0, residual_sum ? residual_sum_row_stride : 0,
        y_row_stride});
   tk::RowShape shape;
-  if (check_rows("rmsnorm_fwd", dtype, rows, cols, vector_ok, &shape)) return 1;
+  if (check_rows("rmsnorm_fwd", dtype, rows, cols, &shape)) return 1;
+  const tk::Access access = tk::row_access(dtype, cols, vector_ok);
   // At most 16 values per thread where the row allows (several waves per row): on the
   // bf16 16384 x 4096 residual forward one wave per row (64 values per thread) ran 93 us,
   // four waves per row 88 us. Rows wider than 1024 x 16 keep the wider shape.
@@ -356,13 +409,12 @@ extern "C" int tk_rmsnorm_fwd(int dtype, const void* x, const void* residual, co
   const dim3 block(shape.rt >= kNormBlock ? shape.rt : kNormBlock);
   hipStream_t s = tk::as_stream(stream);
   TK_DISPATCH_DTYPE(dtype, T,
-    TK_DISPATCH_VEC(T, vector_ok,
-      TK_DISPATCH_ROW_SHAPE(shape,
-        hipLaunchKernelGGL((rmsnorm_fwd_kernel<T, VEC, RT, VALS>), grid, block, 0, s,
+    TK_DISPATCH_NORM_ROWS(T, access, shape,
+        hipLaunchKernelGGL((rmsnorm_fwd_kernel<T, VEC, ACCESS, RT, VALS>), grid, block, 0, s,
                            static_cast<const T*>(x), static_cast<const T*>(residual),
                            static_cast<const T*>(weight), static_cast<T*>(residual_sum),
                            static_cast<T*>(y), rstd, (int)rows, (int)cols, x_row_stride,
-                           residual_row_stride, residual_sum_row_stride, y_row_stride, eps))));
+                           residual_row_stride, residual_sum_row_stride, y_row_stride, eps)));
   return tk::check_launch("rmsnorm_fwd");
 }
 
@@ -386,7 +438,8 @@ extern "C" int tk_rmsnorm_bwd_stage1(int dtype, void* dx, const void* dy, const 
       dtype, cols, {dx, dy, incoming_dx, x, weight},
       {x_row_stride, dy_row_stride, incoming_dx ? incoming_dx_row_stride : 0, dx_row_stride});
   tk::RowShape shape;
-  if (check_rows("rmsnorm_bwd_stage1", dtype, rows, cols, vector_ok, &shape)) return 1;
+  if (check_rows("rmsnorm_bwd_stage1", dtype, rows, cols, &shape)) return 1;
+  const tk::Access access = tk::row_access(dtype, cols, vector_ok);
   // Stage 1 holds three rows of three tensors plus the dweight partials per thread: at
   // most 64 bytes of each row tensor per thread (32 packed 16-bit or 16 float32 values)
   // keeps that in registers without spilling.
@@ -395,14 +448,13 @@ extern "C" int tk_rmsnorm_bwd_stage1(int dtype, void* dx, const void* dy, const 
   hipStream_t s = tk::as_stream(stream);
   int32_t* counts = locks + group_size;
   TK_DISPATCH_DTYPE(dtype, T,
-    TK_DISPATCH_VEC(T, vector_ok,
-      TK_DISPATCH_ROW_SHAPE(shape,
-        hipLaunchKernelGGL((rmsnorm_bwd_stage1_kernel<T, VEC, RT, VALS>), grid,
+    TK_DISPATCH_NORM_ROWS(T, access, shape,
+        hipLaunchKernelGGL((rmsnorm_bwd_stage1_kernel<T, VEC, ACCESS, RT, VALS>), grid,
                            dim3(bwd_block<RT>()), 0, s, static_cast<T*>(dx),
                            static_cast<const T*>(dy), static_cast<const T*>(incoming_dx),
                            partial_dw, static_cast<const T*>(x), static_cast<const T*>(weight),
                            rstd, counts, (int)rows, (int)cols, x_row_stride, dy_row_stride,
-                           incoming_dx_row_stride, dx_row_stride))));
+                           incoming_dx_row_stride, dx_row_stride)));
   return tk::check_launch("rmsnorm_bwd_stage1");
 }
 
@@ -494,7 +546,8 @@ extern "C" int tk_rmsnorm_bwd_noalloc(int dtype, void* dx, void* dw, const void*
       dtype, cols, {dx, dy, incoming_dx, x, weight},
       {x_row_stride, dy_row_stride, incoming_dx ? incoming_dx_row_stride : 0, dx_row_stride});
   tk::RowShape shape;
-  if (check_rows("rmsnorm_bwd_noalloc", dtype, rows, cols, vector_ok, &shape)) return 1;
+  if (check_rows("rmsnorm_bwd_noalloc", dtype, rows, cols, &shape)) return 1;
+  const tk::Access access = tk::row_access(dtype, cols, vector_ok);
   tk::pick_row_shape(cols, &shape, 64 / tk::elem_size(dtype));
   hipStream_t s = tk::as_stream(stream);
   float* partial = nullptr;
@@ -502,15 +555,14 @@ extern "C" int tk_rmsnorm_bwd_noalloc(int dtype, void* dx, void* dw, const void*
   // Stage 1 writes every one of the group_count = min(group_size, rows) partial rows, so
   // the array needs no clearing; stage 2 reads exactly those rows.
   TK_DISPATCH_DTYPE(dtype, T,
-    TK_DISPATCH_VEC(T, vector_ok,
-      TK_DISPATCH_ROW_SHAPE(shape,
-        hipLaunchKernelGGL((rmsnorm_bwd_stage1_kernel<T, VEC, RT, VALS>),
+    TK_DISPATCH_NORM_ROWS(T, access, shape,
+        hipLaunchKernelGGL((rmsnorm_bwd_stage1_kernel<T, VEC, ACCESS, RT, VALS>),
                            dim3(static_cast<unsigned>(group_count)), dim3(bwd_block<RT>()), 0, s,
                            static_cast<T*>(dx), static_cast<const T*>(dy),
                            static_cast<const T*>(incoming_dx), partial, static_cast<const T*>(x),
                            static_cast<const T*>(weight), rstd, nullptr, (int)rows, (int)cols,
                            x_row_stride, dy_row_stride, incoming_dx_row_stride,
-                           dx_row_stride))));
+                           dx_row_stride)));
   if (tk::check_launch("rmsnorm_bwd_noalloc (stage 1)")) return 1;
   TK_DISPATCH_DTYPE(dtype, T,
     hipLaunchKernelGGL((rmsnorm_bwd_stage2_kernel<T>),

@@ -148,7 +148,7 @@ __device__ __forceinline__ u32x4 any_fix(u32x4 v, int cols, int c, int end, uint
 template <typename T, int VEC>
 __device__ __forceinline__ void any_store(T* row, int cols, int c, int end, u32x4 v) {
   if (end <= cols || c + VEC <= cols) {
-    store_any(row + c, v);
+    tk::store_any(row + c, v);
   } else {
     const Vec<T, VEC> e = __builtin_bit_cast(Vec<T, VEC>, v);
 #pragma unroll
@@ -343,6 +343,33 @@ struct RawRow {
     return uint32_t((i * RT + lane) * VEC * int(sizeof(T)));
   }
 
+  // 16-byte variants at any element boundary: load_any issues the loads (of any row with at
+  // least VEC columns), fix_any puts the elements in place and zeroes what lies past the row.
+  __device__ __forceinline__ void load_any(const T* row, int cols, int lane) {
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const u32x4 u = any_load<T, VEC>(row, cols, (i * RT + lane) * VEC);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[i * 4 + j] = u[j];
+    }
+  }
+  __device__ __forceinline__ void fix_any(int cols, int lane) {
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      u32x4 u = {w[i * 4 + 0], w[i * 4 + 1], w[i * 4 + 2], w[i * 4 + 3]};
+      u = any_fix<T, VEC>(u, cols, (i * RT + lane) * VEC, (i + 1) * RT * VEC, 0u);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[i * 4 + j] = u[j];
+    }
+  }
+  __device__ __forceinline__ void store_any(T* row, int cols, int lane) const {
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const u32x4 u = {w[i * 4 + 0], w[i * 4 + 1], w[i * 4 + 2], w[i * 4 + 3]};
+      any_store<T, VEC>(row, cols, (i * RT + lane) * VEC, (i + 1) * RT * VEC, u);
+    }
+  }
+
   __device__ __forceinline__ void store(T* __restrict__ row, int cols, int lane) const {
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
@@ -428,8 +455,8 @@ inline Access row_access(int dtype, int64_t cols, bool aligned) {
   }
 
 // Expands `__VA_ARGS__` with constexpr VEC, ACCESS, RT and VALS bound to `access` and `shape`
-// (scalar rows are narrower than one vector: a single shape; shifted ones take 1024 threads).
-#define TK_DISPATCH_ROWS(T, access, shape, ...)                              \
+// (scalar rows are narrower than one vector: a single shape).
+#define TK_DISPATCH_NORM_ROWS(T, access, shape, ...)                         \
   if ((access) == tk::Access::kScalar) {                                     \
     constexpr tk::Access ACCESS = tk::Access::kScalar;                       \
     constexpr int VEC = 1, RT = 64, VALS = 16;                               \
@@ -438,16 +465,22 @@ inline Access row_access(int dtype, int64_t cols, bool aligned) {
     constexpr tk::Access ACCESS = tk::Access::kAny;                          \
     constexpr int VEC = 16 / int(sizeof(T));                                 \
     TK_DISPATCH_ROW_SHAPE(shape, __VA_ARGS__)                                \
-  } else if ((access) == tk::Access::kShift) {                               \
+  } else {                                                                   \
+    constexpr tk::Access ACCESS = tk::Access::kAligned;                      \
+    constexpr int VEC = 16 / int(sizeof(T));                                 \
+    TK_DISPATCH_ROW_SHAPE(shape, __VA_ARGS__)                                \
+  }
+
+// The same with shifted rows of 1024 threads.
+#define TK_DISPATCH_ROWS(T, access, shape, ...)                              \
+  if ((access) == tk::Access::kShift) {                                      \
     constexpr tk::Access ACCESS = tk::Access::kShift;                        \
     constexpr int VEC = 16 / int(sizeof(T)), RT = 1024;                      \
     if ((shape).vals == 16) { constexpr int VALS = 16; __VA_ARGS__; }        \
     else if ((shape).vals == 32) { constexpr int VALS = 32; __VA_ARGS__; }   \
     else { constexpr int VALS = 64; __VA_ARGS__; }                           \
   } else {                                                                   \
-    constexpr tk::Access ACCESS = tk::Access::kAligned;                      \
-    constexpr int VEC = 16 / int(sizeof(T));                                 \
-    TK_DISPATCH_ROW_SHAPE(shape, __VA_ARGS__)                                \
+    TK_DISPATCH_NORM_ROWS(T, access, shape, __VA_ARGS__)                     \
   }
 
 // Expands `__VA_ARGS__` with constexpr RT and VALS bound to `shape`.
