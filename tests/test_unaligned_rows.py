@@ -118,3 +118,27 @@ def test_residual_rms_norm(dtype, rows, cols) -> None:
         adx, _, adw = torch.autograd.grad((as_, ay), (ax, ar, aw), aligned[3:])
         for got, same in ((s, as_), (y, ay), (dx, adx), (dw, adw)):
             assert bits_equal(got, same)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize(("rows", "cols"), [(1, 1), (1, 3), (1, 9), (3, 5), (7, 503), (8, 503), (179, 503),
+                                            (1025, 1023), (5, 4096), (2, 16385)])
+def test_swiglu_of_any_length(dtype, rows, cols) -> None:
+    """Contiguous problems whose length ends inside a vector: the bits of the same elements in an
+    aligned problem, nothing written past the end."""
+    from tklab.kernels.swiglu import swiglu
+
+    g = torch.Generator("cuda").manual_seed(rows * cols)
+    count = rows * cols
+    padded = -(-count // 64) * 64
+    value, gate, dy = (torch.randn(padded, device="cuda", generator=g).to(dtype) for _ in range(3))
+
+    def step(shape, *tensors):
+        v, gt, d = (t.reshape(shape).detach().clone() for t in tensors)
+        v.requires_grad_(), gt.requires_grad_()
+        y = swiglu(v, gt)
+        return (y, *torch.autograd.grad(y, (v, gt), d))
+
+    whole = step((1, padded), value, gate, dy)
+    for got, want in zip(step((rows, cols), value[:count], gate[:count], dy[:count]), whole):
+        assert bits_equal(got.reshape(-1), want.reshape(-1)[:count])

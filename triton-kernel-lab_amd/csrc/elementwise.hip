@@ -59,11 +59,21 @@ __device__ __forceinline__ ChunkPos chunk_pos(uint32_t i, const tk::FastDiv& per
 
 // ------------------------------------------------------------------ SwiGLU
 
+__device__ __forceinline__ float swiglu_value(float v, float g) { return v * g * stable_sigmoid(g); }
+
+// A contiguous problem whose length is no multiple of VEC is one row of `chunks` vectors and
+// `tail` (< VEC) elements after them, which the first workgroup's threads take one each: bf16
+// 8191 x 14335 forward and backward 478 us one element per access, 294 us so (5.3 TB/s).
+//
 // y = value * gate * sigmoid(gate)  (src/tklab/kernels/swiglu.py:44-58)
 template <typename T, int VEC>
 __global__ __launch_bounds__(kBlock) void swiglu_fwd_kernel(
     const T* __restrict__ value, const T* __restrict__ gate, T* __restrict__ y, uint32_t chunks,
-    tk::FastDiv per_row, int64_t vs, int64_t gs, int64_t ys) {
+    tk::FastDiv per_row, int64_t vs, int64_t gs, int64_t ys, int tail) {
+  if (blockIdx.x == 0 && static_cast<int>(threadIdx.x) < tail) {
+    const int64_t i = int64_t(chunks) * VEC + threadIdx.x;
+    y[i] = tk::from_f32<T>(swiglu_value(tk::to_f32(value[i]), tk::to_f32(gate[i])));
+  }
   // A workgroup pass covers kUnroll * kBlock consecutive chunks (one 4 KiB run per
   // wave and tensor), then the grid strides on.
   const uint32_t stride = gridDim.x * kBlock * kUnroll;
@@ -83,10 +93,18 @@ __global__ __launch_bounds__(kBlock) void swiglu_fwd_kernel(
       if (i >= chunks) break;
       const ChunkPos p = chunk_pos<VEC>(i, per_row);
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) v[u][j] = v[u][j] * g[u][j] * stable_sigmoid(g[u][j]);
+      for (int j = 0; j < VEC; ++j) v[u][j] = swiglu_value(v[u][j], g[u][j]);
       tk::store_vec_stream<T, VEC>(y + p.row * ys + p.col, v[u]);
     }
   }
+}
+
+__device__ __forceinline__ void swiglu_grad(float d, float v, float g, float& dv, float& dg) {
+  const float sg = stable_sigmoid(g);
+  const float silu = g * sg;
+  const float dsilu = sg * (1.0f + g * (1.0f - sg));
+  dv = d * silu;
+  dg = d * v * dsilu;
 }
 
 // dvalue = dy * silu(g); dgate = dy * value * sigmoid(g) * (1 + g * (1 - sigmoid(g)))
@@ -95,7 +113,14 @@ template <typename T, int VEC>
 __global__ __launch_bounds__(kBlock) void swiglu_bwd_kernel(
     const T* __restrict__ dy, const T* __restrict__ value, const T* __restrict__ gate,
     T* __restrict__ dvalue, T* __restrict__ dgate, uint32_t chunks, tk::FastDiv per_row, int64_t dys,
-    int64_t vs, int64_t gs, int64_t dvs, int64_t dgs) {
+    int64_t vs, int64_t gs, int64_t dvs, int64_t dgs, int tail) {
+  if (blockIdx.x == 0 && static_cast<int>(threadIdx.x) < tail) {
+    const int64_t i = int64_t(chunks) * VEC + threadIdx.x;
+    float dv, dg;
+    swiglu_grad(tk::to_f32(dy[i]), tk::to_f32(value[i]), tk::to_f32(gate[i]), dv, dg);
+    dvalue[i] = tk::from_f32<T>(dv);
+    dgate[i] = tk::from_f32<T>(dg);
+  }
   // A workgroup pass covers kUnroll * kBlock consecutive chunks (one 4 KiB run per
   // wave and tensor), then the grid strides on.
   const uint32_t stride = gridDim.x * kBlock * kUnroll;
@@ -117,13 +142,7 @@ __global__ __launch_bounds__(kBlock) void swiglu_bwd_kernel(
       const ChunkPos p = chunk_pos<VEC>(i, per_row);
       float dv[VEC], dg[VEC];
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) {
-        const float sg = stable_sigmoid(g[u][j]);
-        const float silu = g[u][j] * sg;
-        const float dsilu = sg * (1.0f + g[u][j] * (1.0f - sg));
-        dv[j] = d[u][j] * silu;
-        dg[j] = d[u][j] * v[u][j] * dsilu;
-      }
+      for (int j = 0; j < VEC; ++j) swiglu_grad(d[u][j], v[u][j], g[u][j], dv[j], dg[j]);
       tk::store_vec_stream<T, VEC>(dvalue + p.row * dvs + p.col, dv);
       tk::store_vec_stream<T, VEC>(dgate + p.row * dgs + p.col, dg);
     }
@@ -299,6 +318,19 @@ bool vector_ok(int dtype, int64_t width, std::initializer_list<const void*> ptrs
   return true;
 }
 
+// Elements of a one-row problem past its last whole vector, dropped from `cols`, where the rest
+// can be vectors; 0 where nothing is left over or only scalar accesses fit.
+int split_tail(int dtype, int64_t rows, int64_t* cols, std::initializer_list<const void*> ptrs) {
+  if (!tk::valid_dtype(dtype) || rows != 1) return 0;
+  const int vec = 16 / tk::elem_size(dtype);
+  if (*cols < vec) return 0;
+  for (const void* p : ptrs)
+    if (!tk::aligned16(p)) return 0;
+  const int tail = static_cast<int>(*cols % vec);
+  *cols -= tail;
+  return tail;
+}
+
 int check_problem(const char* what, int dtype, int64_t rows, int64_t width, int vec,
                   int64_t* chunks_per_row, int64_t* chunks) {
   if (!tk::valid_dtype(dtype)) return tk::fail("%s: unsupported dtype code %d", what, dtype);
@@ -328,7 +360,9 @@ extern "C" int tk_swiglu_fwd(int dtype, const void* value, const void* gate, voi
     cols = tk::folded_extent(rows, cols);
     rows = 1;
     if (cols < 0) return tk::fail("swiglu_fwd: problem too large");
+    value_row_stride = gate_row_stride = y_row_stride = 0;  // one row
   }
+  const int tail = split_tail(dtype, rows, &cols, {value, gate, y});
   const bool vok = tk::valid_dtype(dtype) &&
                    vector_ok(dtype, cols, {value, gate, y},
                              {value_row_stride, gate_row_stride, y_row_stride});
@@ -343,7 +377,7 @@ extern "C" int tk_swiglu_fwd(int dtype, const void* value, const void* gate, voi
       hipLaunchKernelGGL((swiglu_fwd_kernel<T, VEC>), dim3(g.blocks), dim3(kBlock), 0, s,
                          static_cast<const T*>(value), static_cast<const T*>(gate),
                          static_cast<T*>(y), (int)chunks, div, value_row_stride,
-                         gate_row_stride, y_row_stride)));
+                         gate_row_stride, y_row_stride, tail)));
   return tk::check_launch("swiglu_fwd");
 }
 
@@ -363,7 +397,10 @@ extern "C" int tk_swiglu_bwd(int dtype, const void* dy, const void* value, const
     cols = tk::folded_extent(rows, cols);
     rows = 1;
     if (cols < 0) return tk::fail("swiglu_bwd: problem too large");
+    dy_row_stride = value_row_stride = gate_row_stride = dvalue_row_stride = dgate_row_stride =
+        0;  // one row
   }
+  const int tail = split_tail(dtype, rows, &cols, {dy, value, gate, dvalue, dgate});
   const bool vok = tk::valid_dtype(dtype) &&
                    vector_ok(dtype, cols, {dy, value, gate, dvalue, dgate},
                              {dy_row_stride, value_row_stride, gate_row_stride,
@@ -381,7 +418,7 @@ extern "C" int tk_swiglu_bwd(int dtype, const void* dy, const void* value, const
                          static_cast<const T*>(gate), static_cast<T*>(dvalue),
                          static_cast<T*>(dgate), (int)chunks, div, dy_row_stride,
                          value_row_stride, gate_row_stride, dvalue_row_stride,
-                         dgate_row_stride)));
+                         dgate_row_stride, tail)));
   return tk::check_launch("swiglu_bwd");
 }
 
