@@ -160,13 +160,20 @@ def ptr(tensor: torch.Tensor | None) -> int | None:
 
 
 def stream_of(tensor: torch.Tensor) -> int:
-    """Handle of PyTorch's current stream on ``tensor``'s device."""
-    return torch.cuda.current_stream(tensor.device).cuda_stream
+    """Handle of PyTorch's current stream on ``tensor``'s device.
+
+    The raw handle, without the ``torch.cuda.Stream`` object around it (2-3 us per launch).
+    """
+    return torch._C._cuda_getCurrentRawStream(tensor.get_device())
+
+
+_INT64_ARRAYS = tuple(ctypes.c_int64 * n for n in range(5))
 
 
 def int64_array(values: tuple[int, ...] | list[int]) -> ctypes.Array[ctypes.c_int64]:
     """Pack integers into a C ``int64_t[]``."""
-    return (ctypes.c_int64 * len(values))(*values)
+    n = len(values)
+    return (_INT64_ARRAYS[n] if n < 5 else ctypes.c_int64 * n)(*values)
 
 
 _bound: dict[str, ctypes._CFuncPtr] = {}
@@ -185,9 +192,7 @@ def _function(name: str) -> ctypes._CFuncPtr:
 
 def call(name: str, *args: object) -> None:
     """Invoke ``name`` and raise :class:`HipLibraryError` on a non-zero status."""
-    fn = _function(name)
-    lib = load_library()
-    status = fn(*args)
+    status = (_bound.get(name) or _function(name))(*args)
     if status != 0:
-        message = lib.tk_last_error().decode(errors="replace")
+        message = load_library().tk_last_error().decode(errors="replace")
         raise HipLibraryError(f"{name} failed: {message}")

@@ -28,5 +28,7 @@ def max_relative_offset(tensor: torch.Tensor) -> int:
 
 def assert_int32_addressable(tensor: torch.Tensor, *, name: str) -> None:
     """Raise ``ValueError`` when ``tensor`` cannot be indexed with int32 offsets."""
+    if tensor.is_contiguous() and tensor.numel() <= MAX_INT32_OFFSET + 1:
+        return  # its last element is the farthest one
     if max_relative_offset(tensor) > MAX_INT32_OFFSET:
         raise ValueError(f"{name} strides exceed the signed int32 offset range")

@@ -95,7 +95,7 @@ def _make_output(args: TensorArgs) -> torch.Tensor:
 
 def _strides(t: torch.Tensor) -> Any:
     """(batch, head, sequence) element strides as a C ``int64_t[3]``."""
-    return _hip.int64_array(list(t.stride()[:3]))
+    return _hip.int64_array(t.stride()[:3])
 
 
 def _launch_forward(
@@ -114,16 +114,24 @@ def _launch_forward(
         raise ValueError("attention output metadata must match Q")
     if not output.is_contiguous():
         raise ValueError("attention output must be contiguous")
-    batch, heads, n_ctx, head_dim = q.shape
     if store_lse:
         if (
-            softmax_lse.shape != (batch, heads, n_ctx)
+            softmax_lse.shape != q.shape[:3]
             or softmax_lse.device != q.device
             or softmax_lse.dtype != torch.float32
             or not softmax_lse.is_contiguous()
         ):
             raise ValueError("attention log-sum-exp buffer must be contiguous float32 BxHxN")
         assert_int32_addressable(softmax_lse, name="log-sum-exp buffer")
+    _enqueue_forward(q, k, v, output, softmax_lse if store_lse else None, causal=causal)
+
+
+def _enqueue_forward(
+    q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, output: torch.Tensor,
+    softmax_lse: torch.Tensor | None, *, causal: bool,
+) -> None:
+    """The forward for contiguous tensors already checked."""
+    batch, heads, n_ctx, head_dim = q.shape
     _hip.call(
         "tk_attn_fwd",
         _hip.dtype_code(q.dtype),
@@ -131,7 +139,7 @@ def _launch_forward(
         k.data_ptr(),
         v.data_ptr(),
         output.data_ptr(),
-        softmax_lse.data_ptr() if store_lse else None,
+        _hip.ptr(softmax_lse),
         batch,
         heads,
         n_ctx,
@@ -226,11 +234,10 @@ class _FlashAttentionFunction(torch.autograd.Function):
     def forward(
         ctx: Any, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool
     ) -> torch.Tensor:
-        _validate(q, k, v)
         output = torch.empty_like(q)
         batch, heads, n_ctx, _ = q.shape
         softmax_lse = torch.empty((batch, heads, n_ctx), dtype=torch.float32, device=q.device)
-        _launch_forward(q, k, v, output, softmax_lse, causal=causal, store_lse=True)
+        _enqueue_forward(q, k, v, output, softmax_lse, causal=causal)
         ctx.save_for_backward(q, k, v, output, softmax_lse)
         ctx.causal = causal
         return output
@@ -251,7 +258,7 @@ def _attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: boo
     needs_grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
     if not needs_grad:
         output = torch.empty_like(q)
-        _launch_forward(q, k, v, output, output, causal=causal, store_lse=False)
+        _enqueue_forward(q, k, v, output, None, causal=causal)
         return output
     return cast(torch.Tensor, _FlashAttentionFunction.apply(q, k, v, causal))
 

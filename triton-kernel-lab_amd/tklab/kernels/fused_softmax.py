@@ -39,7 +39,10 @@ def softmax(x: torch.Tensor) -> torch.Tensor:
     """
     _validate(x)
     output = _make_output((x,))
-    _launch((x,), output)
+    if output.stride(1) != 1:
+        raise ValueError("softmax output requires a contiguous final dimension")
+    assert_int32_addressable(output, name="output")
+    _enqueue(x, output)
     return output
 
 
@@ -56,7 +59,10 @@ def online_softmax(x: torch.Tensor) -> torch.Tensor:
     """
     _validate(x, single_pass=False)
     output = _make_output((x,))
-    _launch_online((x,), output)
+    if output.stride(1) != 1:
+        raise ValueError("softmax output requires a contiguous final dimension")
+    assert_int32_addressable(output, name="output")
+    _enqueue_online(x, output)
     return output
 
 
@@ -69,6 +75,11 @@ def _launch_online(args: TensorArgs, output: torch.Tensor) -> None:
     if output.stride(1) != 1:
         raise ValueError("softmax output requires a contiguous final dimension")
     assert_int32_addressable(output, name="output")
+    _enqueue_online(x, output)
+
+
+def _enqueue_online(x: torch.Tensor, output: torch.Tensor) -> None:
+    """The online softmax for tensors already checked."""
     rows, columns = x.shape
     chunks = -(-columns // ONLINE_CHUNK_COLUMNS)
     partials = torch.empty(2 * rows * chunks, device=x.device, dtype=torch.float32)
@@ -129,6 +140,11 @@ def _launch(args: TensorArgs, output: torch.Tensor) -> None:
     if output.stride(1) != 1:
         raise ValueError("softmax output requires a contiguous final dimension")
     assert_int32_addressable(output, name="output")
+    _enqueue(x, output)
+
+
+def _enqueue(x: torch.Tensor, output: torch.Tensor) -> None:
+    """The single-pass softmax for tensors already checked."""
     rows, columns = x.shape
     _hip.call(
         "tk_softmax_fwd",

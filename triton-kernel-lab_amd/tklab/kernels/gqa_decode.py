@@ -59,8 +59,8 @@ def gqa_decode(
     batch, q_heads, head_dim = q.shape
     out = torch.empty((batch, q_heads, head_dim), device=q.device, dtype=q.dtype)
     lse = torch.empty((batch, q_heads), device=q.device, dtype=torch.float32)
-    _launch(q, k_cache, v_cache, cache_seqlens, out, lse,
-            scale=head_dim ** -0.5 if scale is None else scale)
+    _enqueue(q, k_cache, v_cache, cache_seqlens, out, lse,
+             scale=head_dim ** -0.5 if scale is None else scale)
     return (out, lse) if return_lse else out
 
 
@@ -85,7 +85,6 @@ def _launch(
     """Run the decode into preallocated ``out`` (and ``lse`` when given)."""
     _validate(q, k_cache, v_cache, cache_seqlens)
     batch, q_heads, head_dim = q.shape
-    kv_heads, max_len = k_cache.shape[1], k_cache.shape[2]
     if out.shape != q.shape or out.dtype != q.dtype or out.device != q.device:
         raise ValueError("output metadata must match q")
     if out.stride(-1) != 1 or out.data_ptr() % 16 or any(s % 8 for s in out.stride()[:2]):
@@ -93,6 +92,22 @@ def _launch(
     if lse is not None and (lse.shape != (batch, q_heads) or lse.dtype != torch.float32
                             or not lse.is_contiguous()):
         raise ValueError("lse must be a contiguous float32 [batch, q_heads] tensor")
+    _enqueue(q, k_cache, v_cache, cache_seqlens, out, lse, scale=scale)
+
+
+def _enqueue(
+    q: torch.Tensor,
+    k_cache: torch.Tensor,
+    v_cache: torch.Tensor,
+    cache_seqlens: torch.Tensor | None,
+    out: torch.Tensor,
+    lse: torch.Tensor | None,
+    *,
+    scale: float,
+) -> None:
+    """The decode launches for tensors already checked."""
+    batch, q_heads, head_dim = q.shape
+    kv_heads, max_len = k_cache.shape[1], k_cache.shape[2]
     split = split_length(batch, kv_heads, max_len)
     splits = -(-max_len // split)
     partials = torch.empty((batch, q_heads, splits, head_dim + 4), device=q.device,
@@ -113,10 +128,10 @@ def _launch(
         max_len,
         head_dim,
         split,
-        _hip.int64_array(list(q.stride()[:2])),
-        _hip.int64_array(list(k_cache.stride()[:3])),
-        _hip.int64_array(list(v_cache.stride()[:3])),
-        _hip.int64_array(list(out.stride()[:2])),
+        _hip.int64_array(q.stride()[:2]),
+        _hip.int64_array(k_cache.stride()[:3]),
+        _hip.int64_array(v_cache.stride()[:3]),
+        _hip.int64_array(out.stride()[:2]),
         float(scale),
         _hip.stream_of(q),
     )

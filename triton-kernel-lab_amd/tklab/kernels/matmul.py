@@ -150,28 +150,19 @@ def _launch_factory(*, fp16_accumulate: bool) -> LaunchFn:
             raise ValueError("output metadata must match the inputs")
         if not output.is_contiguous():
             raise ValueError("matmul output must be contiguous")
-        m, k = a.shape
-        n = b.shape[1]
-        _hip.call(
-            "tk_gemm",
-            _hip.dtype_code(a.dtype),
-            a.data_ptr(),
-            b.data_ptr(),
-            output.data_ptr(),
-            m,
-            n,
-            k,
-            a.stride(0),
-            a.stride(1),
-            b.stride(0),
-            b.stride(1),
-            output.stride(0),
-            output.stride(1),
-            int(fp16_accumulate),
-            _hip.stream_of(a),
-        )
+        _enqueue(a, b, output, fp16_accumulate=fp16_accumulate)
 
     return launch
+
+
+def _enqueue(a: torch.Tensor, b: torch.Tensor, output: torch.Tensor, *, fp16_accumulate: bool) -> None:
+    """``output = a @ b`` for operands and an output already checked."""
+    m, k = a.shape
+    _hip.call(
+        "tk_gemm", _hip.dtype_code(a.dtype), a.data_ptr(), b.data_ptr(), output.data_ptr(), m,
+        b.shape[1], k, *a.stride(), *b.stride(), *output.stride(), int(fp16_accumulate),
+        _hip.stream_of(a),
+    )
 
 
 _launch_fp32acc = _launch_factory(fp16_accumulate=False)
@@ -182,7 +173,7 @@ def matmul_fp32acc(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """``a @ b`` with float32 MFMA accumulation."""
     _validate(a, b)
     output = _make_output((a, b))
-    _launch_fp32acc((a, b), output)
+    _enqueue(a, b, output, fp16_accumulate=False)
     return output
 
 
@@ -190,7 +181,7 @@ def matmul_fp16acc(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """Registry-compatible FP16-accumulate entry point (runs the FP32-accumulate kernel)."""
     _validate(a, b)
     output = _make_output((a, b))
-    _launch_fp16acc((a, b), output)
+    _enqueue(a, b, output, fp16_accumulate=True)
     return output
 
 

@@ -74,26 +74,43 @@ def _launch_forward(
     _validate_output(output, x, name="output")
     if store_residual:
         _validate_output(residual_sum, x, name="residual_sum")
-    rows, columns = x.shape
     if store_stats:
-        if rstd.shape != (rows,) or rstd.device != x.device:
+        if rstd.shape != (x.shape[0],) or rstd.device != x.device:
             raise ValueError("rstd must contain one value per input row")
         if rstd.dtype != torch.float32:
             raise ValueError("rstd must use float32")
+    _enqueue_forward(
+        x, residual, weight, residual_sum if store_residual else None, output,
+        rstd if store_stats else None, eps=eps,
+    )
+
+
+def _enqueue_forward(
+    x: torch.Tensor,
+    residual: torch.Tensor,
+    weight: torch.Tensor,
+    residual_sum: torch.Tensor | None,
+    output: torch.Tensor,
+    rstd: torch.Tensor | None,
+    *,
+    eps: float,
+) -> None:
+    """The fused add + norm for tensors already checked."""
+    rows, columns = x.shape
     _hip.call(
         "tk_rmsnorm_fwd",
         _hip.dtype_code(x.dtype),
         x.data_ptr(),
         residual.data_ptr(),
         weight.data_ptr(),
-        residual_sum.data_ptr() if store_residual else None,
+        _hip.ptr(residual_sum),
         output.data_ptr(),
-        rstd.data_ptr() if store_stats else None,
+        _hip.ptr(rstd),
         rows,
         columns,
         x.stride(0),
         residual.stride(0),
-        residual_sum.stride(0) if store_residual else 0,
+        0 if residual_sum is None else residual_sum.stride(0),
         output.stride(0),
         eps,
         _hip.stream_of(x),
@@ -108,15 +125,12 @@ class _ResidualRMSNormFunction(torch.autograd.Function):
         ctx: Any, x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float
     ) -> tuple[torch.Tensor, torch.Tensor]:
         """Return ``(residual_sum, normalized)`` and save the sum, weight and rstd."""
-        _validate_inputs(x, residual, weight)
         ctx.set_materialize_grads(False)
         residual_sum = torch.empty(x.shape, dtype=x.dtype, device=x.device)
         output = torch.empty_like(residual_sum)
         rstd = torch.empty(x.shape[0], dtype=torch.float32, device=x.device)
-        _launch_forward(
-            x, residual, weight, residual_sum, output, rstd,
-            eps=eps, store_residual=True, store_stats=True,
-        )
+        assert_int32_addressable(output, name="output")  # larger than broadcast inputs
+        _enqueue_forward(x, residual, weight, residual_sum, output, rstd, eps=eps)
         ctx.save_for_backward(residual_sum, weight, rstd)
         return residual_sum, output
 
@@ -158,10 +172,8 @@ def residual_rms_norm(
     if not needs_grad:
         residual_sum = torch.empty(x.shape, dtype=x.dtype, device=x.device)
         output = torch.empty_like(residual_sum)
-        _launch_forward(
-            x, residual, weight, residual_sum, output, output,
-            eps=eps, store_residual=True, store_stats=False,
-        )
+        assert_int32_addressable(output, name="output")
+        _enqueue_forward(x, residual, weight, residual_sum, output, None, eps=eps)
         return residual_sum, output
     result = _ResidualRMSNormFunction.apply(x, residual, weight, eps)
     return cast(tuple[torch.Tensor, torch.Tensor], result)

@@ -111,14 +111,22 @@ def _launch_forward(
     if output.stride(1) != 1:
         raise ValueError("rms_norm output requires a contiguous final dimension")
     assert_int32_addressable(output, name="output")
-    rows, columns = x.shape
     if store_stats:
-        if rstd.shape != (rows,):
+        if rstd.shape != (x.shape[0],):
             raise ValueError("rstd must contain one float32 value per row")
         if rstd.dtype != torch.float32:
             raise ValueError("rstd must use float32")
         if rstd.device != x.device:
             raise ValueError("rstd must be on the input device")
+    _enqueue_forward(x, weight, output, rstd if store_stats else None, eps=eps)
+
+
+def _enqueue_forward(
+    x: torch.Tensor, weight: torch.Tensor, output: torch.Tensor, rstd: torch.Tensor | None,
+    *, eps: float,
+) -> None:
+    """The forward for tensors already checked."""
+    rows, columns = x.shape
     _hip.call(
         "tk_rmsnorm_fwd",
         _hip.dtype_code(x.dtype),
@@ -127,7 +135,7 @@ def _launch_forward(
         weight.data_ptr(),
         None,
         output.data_ptr(),
-        rstd.data_ptr() if store_stats else None,
+        _hip.ptr(rstd),
         rows,
         columns,
         x.stride(0),
@@ -144,8 +152,13 @@ def _make_backward_buffers(
     weight: torch.Tensor,
     *,
     group_size: int | None = None,
+    zero_locks: bool = True,
 ) -> _BackwardBuffers:
-    """Allocate dx, dw, the float32 partial rows and the zeroed lock/count words."""
+    """Allocate dx, dw, the float32 partial rows and the lock/count words.
+
+    The words are zeroed for callers that look at them: the kernels read neither half and write
+    the active groups' counts, so the autograd path leaves out that fill and its launch.
+    """
     rows, columns = x.shape
     block_size, num_warps = block_size_and_warps(columns, x.element_size())
     selected = group_size_m(columns) if group_size is None else group_size
@@ -155,7 +168,9 @@ def _make_backward_buffers(
         dx=torch.empty(x.shape, dtype=x.dtype, device=x.device),
         partial_dw=torch.empty((selected, columns), dtype=torch.float32, device=x.device),
         dw=torch.empty_like(weight),
-        locks=torch.zeros(2 * selected, dtype=torch.int32, device=x.device),
+        locks=(torch.zeros if zero_locks else torch.empty)(
+            2 * selected, dtype=torch.int32, device=x.device
+        ),
         group_size=selected,
         group_count=min(selected, rows),
         block_size=block_size,
@@ -234,7 +249,7 @@ def _launch_backward(
             incoming_dx = incoming_dx.contiguous()
         assert_int32_addressable(incoming_dx, name="incoming input gradient")
     check_deterministic_mode("RMSNorm")
-    buffers = _make_backward_buffers(x, weight)
+    buffers = _make_backward_buffers(x, weight, zero_locks=False)
     _launch_backward_stage1(dy, x, weight, rstd, buffers, incoming_dx=incoming_dx)
     _launch_backward_stage2(buffers, x.shape[1])
     return buffers.dx, buffers.dw
@@ -246,10 +261,10 @@ class _RMSNormFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx: Any, x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
         """Forward with float32 rstd saved for backward."""
-        _validate(x, weight)
         output = torch.empty(x.shape, dtype=x.dtype, device=x.device)
         rstd = torch.empty(x.shape[0], dtype=torch.float32, device=x.device)
-        _launch_forward(x, weight, output, rstd, eps=eps, store_stats=True)
+        assert_int32_addressable(output, name="output")  # larger than a broadcast input
+        _enqueue_forward(x, weight, output, rstd, eps=eps)
         ctx.save_for_backward(x, weight, rstd)
         return output
 
@@ -273,7 +288,8 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = EPS) -> torch.T
     needs_grad = torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)
     if not needs_grad:
         output = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-        _launch_forward(x, weight, output, output, eps=eps, store_stats=False)
+        assert_int32_addressable(output, name="output")
+        _enqueue_forward(x, weight, output, None, eps=eps)
         return output
     return cast(torch.Tensor, _RMSNormFunction.apply(x, weight, eps))
 

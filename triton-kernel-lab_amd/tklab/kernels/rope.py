@@ -63,6 +63,13 @@ def _launch_forward(
     """Forward into a supplied output."""
     _validate_inputs(x, cos, sin)
     _validate_output(output, x, name="output")
+    _enqueue_forward(x, cos, sin, output)
+
+
+def _enqueue_forward(
+    x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, output: torch.Tensor
+) -> None:
+    """The forward for tensors already checked."""
     rows, columns = x.shape
     _hip.call(
         "tk_rope_fwd",
@@ -146,7 +153,8 @@ class _RoPEFunction(torch.autograd.Function):
         """Forward and save (x, cos, sin)."""
         _validate_inputs(x, cos, sin)
         output = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-        _launch_forward(x, cos, sin, output)
+        assert_int32_addressable(output, name="output")  # larger than a broadcast input
+        _enqueue_forward(x, cos, sin, output)
         ctx.save_for_backward(x, cos, sin)
         return output
 

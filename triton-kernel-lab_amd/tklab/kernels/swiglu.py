@@ -63,6 +63,11 @@ def _launch_forward(value: torch.Tensor, gate: torch.Tensor, output: torch.Tenso
     """Forward into a supplied output."""
     _validate_inputs(value, gate)
     _validate_output(output, value, name="output")
+    _enqueue_forward(value, gate, output)
+
+
+def _enqueue_forward(value: torch.Tensor, gate: torch.Tensor, output: torch.Tensor) -> None:
+    """The forward for tensors already checked."""
     rows, columns = value.shape
     _hip.call(
         "tk_swiglu_fwd",
@@ -131,7 +136,8 @@ class _SwiGLUFunction(torch.autograd.Function):
         """Forward and save (value, gate)."""
         _validate_inputs(value, gate)
         output = torch.empty(value.shape, dtype=value.dtype, device=value.device)
-        _launch_forward(value, gate, output)
+        assert_int32_addressable(output, name="output")  # larger than broadcast inputs
+        _enqueue_forward(value, gate, output)
         ctx.save_for_backward(value, gate)
         return output
 
