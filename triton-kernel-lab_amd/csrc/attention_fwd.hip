@@ -45,6 +45,8 @@
 #include "attention.hpp"
 #include "attention_dma.hpp"
 
+#include <type_traits>
+
 namespace {
 
 using namespace tk_attn;
@@ -708,11 +710,335 @@ attn_fwd_dma_kernel(FwdArgs<T> kernel_arg) {
   }  // tiles
 }
 
+// ------------------------------------------------------------------ short problems
+//
+// The same forward for problems whose 256-query workgroups leave CUs idle, where the time is one
+// workgroup's serial walk over its key blocks: a block costs a wave its MFMAs plus its
+// exponentials, one after the other. Here a wave owns 16 queries (half the work per block) and a
+// workgroup 64 (four waves, two workgroups per CU), so four times as many workgroups walk
+// blocks half as long. There is no ping-pong: each wave reads K, forms S, takes its softmax
+// while the V fragments of the block's first half arrive, and multiplies. Twice the LDS reads per
+// MFMA make it slower than the 256-query kernel once that fills the chip (small_applies).
+//
+// Every query sees the same operations in the same order as in the 256-query kernel, so the
+// results are bitwise the same.
+template <int D>
+struct SmallGeo {
+  using G = Geo<D>;
+  static constexpr int BM = 64, WAVES = 4, THREADS = 256;
+  static constexpr int STAGES = D == 64 ? 4 : 2;  // 64 KiB: two workgroups per CU
+  static constexpr int DMA_PER_OP = G::OPB / 1024 / WAVES;
+  static constexpr int DPB = 2 * DMA_PER_OP;
+};
+
+// A wave's share of the DMA of one key/value block, into its part `at` of the stage.
+template <int D>
+__device__ __forceinline__ void small_dma(__amdgpu_buffer_rsrc_t rk, __amdgpu_buffer_rsrc_t rv,
+                                          char* at, const uint32_t* k_src, const uint32_t* v_src,
+                                          uint32_t k_off, uint32_t v_off) {
+#pragma unroll
+  for (int x = 0; x < SmallGeo<D>::DMA_PER_OP; ++x) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_void*)(at + x * 1024), 16, k_src[x], k_off,
+                                             0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_void*)(at + Geo<D>::OPB + x * 1024), 16,
+                                             v_src[x], v_off, 0, 0);
+  }
+}
+
+template <typename T, int D, bool CAUSAL>
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2))) void
+attn_fwd_small_kernel(FwdArgs<T> args) {
+  using G = Geo<D>;
+  using S = SmallGeo<D>;
+  constexpr int BN = G::BN, KS = G::KS, FT = G::FT, RB = G::RB, OPB = G::OPB, STB = G::STB,
+                STAGES = S::STAGES;
+  __shared__ __attribute__((aligned(1024))) char lds[STAGES * STB];
+  const Shape& s = args.s;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_void*)lds;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, g = lane >> 4;
+
+  // Tiles: heaviest (last) query blocks first over all heads; with heads a multiple of 8 each
+  // XCD keeps its own heads. Varlen: the heavy-first schedule over every sequence's blocks.
+  int b, h, qb, start = 0, N = s.seq;
+  uint32_t k_bytes = s.k_bytes, v_bytes = s.v_bytes;
+  if (s.cu != nullptr) {
+    h = varlen_head(blockIdx.x, s.heads);
+    VarlenTile vt;
+    if (!varlen_tile(s.cu, s.batch, s.total, s.seq, S::BM, blockIdx.x / s.heads, vt)) return;
+    b = vt.b;
+    qb = vt.level;
+    const VarlenRows rows = varlen_rows(s.cu, b, s.total, s.seq);
+    start = rows.start;
+    N = rows.n;
+    if (qb * S::BM >= N) return;
+    k_bytes = uint32_t(((N - 1) * s.k[2] + D) * 2);
+    v_bytes = uint32_t(((N - 1) * s.v[2] + D) * 2);
+  } else {
+    const int heads = s.tiles / s.q_blocks;
+    int bh, rank;
+    if (heads % 8 == 0) {
+      const int per = heads / 8, i = blockIdx.x / 8;
+      bh = (blockIdx.x % 8) * per + i % per;
+      rank = i / per;
+    } else {
+      bh = blockIdx.x % heads;
+      rank = blockIdx.x / heads;
+    }
+    qb = s.q_blocks - 1 - rank;
+    b = bh / s.heads;
+    h = bh % s.heads;
+  }
+  const int kvh = h / s.group;
+  const T* Qh = args.Q + b * s.q[0] + h * s.q[1] + int64_t(start) * s.q[2];
+  const T* Kh = args.K + b * s.k[0] + kvh * s.k[1] + int64_t(start) * s.k[2];
+  const T* Vh = args.V + b * s.v[0] + kvh * s.v[1] + int64_t(start) * s.v[2];
+  const int q0 = qb * S::BM;
+  const int wq0 = q0 + wave * 16;
+  const __amdgpu_buffer_rsrc_t rk =
+      __builtin_amdgcn_make_buffer_rsrc((void*)Kh, (short)0, k_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rv =
+      __builtin_amdgcn_make_buffer_rsrc((void*)Vh, (short)0, v_bytes, 0x00020000);
+  uint32_t k_src[S::DMA_PER_OP], v_src[S::DMA_PER_OP];
+#pragma unroll
+  for (int x = 0; x < S::DMA_PER_OP; ++x) {
+    const int row = (wave * S::DMA_PER_OP + x) * G::ROWS_PER_DMA + lane / G::SLOTS;
+    const int slot = lane % G::SLOTS;
+    k_src[x] = uint32_t(row * s.k[2] + (slot ^ G::kswz(row)) * 8) * 2u;
+    v_src[x] = uint32_t(row * s.v[2] + ((slot >> 1) ^ G::vswz(row)) * 16 + (slot & 1) * 8) * 2u;
+  }
+  const int kv_end = CAUSAL ? min(N, q0 + S::BM) : N;
+  const int blocks = (kv_end + BN - 1) / BN;
+  const uint32_t k_blk = uint32_t(BN * s.k[2]) * 2u, v_blk = uint32_t(BN * s.v[2]) * 2u;
+  // Blocks past the end reload the last one into a stage that is never read.
+  auto load = [&](int blk, int stage) {
+    blk = min(blk, blocks - 1);
+    small_dma<D>(rk, rv, lds + stage * STB + wave * S::DMA_PER_OP * 1024, k_src, v_src,
+                 blk * k_blk, blk * v_blk);
+  };
+#pragma unroll
+  for (int blk = 0; blk < STAGES - 1; ++blk) load(blk, blk);
+
+  // Q fragments, rotated if asked, as in the 256-query kernel.
+  const int query = wq0 + c;
+  i32x4 qf[KS];
+#pragma unroll
+  for (int kk = 0; kk < KS; ++kk)
+    qf[kk] = query < N ? *reinterpret_cast<const i32x4*>(Qh + query * s.q[2] + kk * 32 + g * 8)
+                       : i32x4{0, 0, 0, 0};
+  if (s.rope_cos != nullptr) {
+    const int64_t at = int64_t(query) * s.rope_stride + g * 8;
+    const T* cr = static_cast<const T*>(s.rope_cos) + at;
+    const T* sr = static_cast<const T*>(s.rope_sin) + at;
+#pragma unroll
+    for (int kk = 0; kk < KS / 2; ++kk) {
+      const i32x4 cv = query < N ? *reinterpret_cast<const i32x4*>(cr + kk * 32) : i32x4{0, 0, 0, 0};
+      const i32x4 sv = query < N ? *reinterpret_cast<const i32x4*>(sr + kk * 32) : i32x4{0, 0, 0, 0};
+      rope_fragment<T>(qf[kk], qf[kk + KS / 2], cv, sv);
+    }
+  }
+  uint32_t ka[KS], va[FT];
+#pragma unroll
+  for (int kk = 0; kk < KS; ++kk) ka[kk] = c * RB + (((4 * kk + g) ^ G::kswz(c)) * 16);
+  {
+    const int row = 4 * g + (c >> 2), q = c & 3;
+#pragma unroll
+    for (int ft = 0; ft < FT; ++ft) va[ft] = OPB + row * RB + ((ft ^ G::vswz(row)) * 32) + q * 8;
+  }
+
+  f32x4 acc[FT];
+#pragma unroll
+  for (int ft = 0; ft < FT; ++ft) acc[ft] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = kNegInf, l_part = 0.f;
+  const float sl2 = s.scale_log2;
+  int stage = 0, fill = STAGES - 1;
+  for (int j = 0; j < blocks; ++j) {
+    // Block j has landed in every wave's share, and every wave has read block j - 1, whose stage
+    // takes block j + STAGES - 1.
+    wait_vmcnt<(STAGES - 2) * S::DPB>();
+    barrier_no_fence();
+    const uint32_t base = lds_base + stage * STB;
+    i32x4 kf[KS][4];
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) {
+      kf[kk][0] = lds_read_b128<0>(base + ka[kk]);
+      kf[kk][1] = lds_read_b128<16 * RB>(base + ka[kk]);
+      kf[kk][2] = lds_read_b128<32 * RB>(base + ka[kk]);
+      kf[kk][3] = lds_read_b128<48 * RB>(base + ka[kk]);
+    }
+    load(j + STAGES - 1, fill);
+    f32x4 st[4];
+    auto score = [&](auto step) {
+      constexpr int kk = decltype(step)::value;
+      wait_lgkm<4 * (KS - 1 - kk) < 15 ? 4 * (KS - 1 - kk) : 15>();
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) pin(kf[kk][kt]);
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+        st[kt] = Mma16<T>::run(kf[kk][kt], qf[kk], kk == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : st[kt]);
+    };
+    score(std::integral_constant<int, 0>{});
+    score(std::integral_constant<int, 1>{});
+    if constexpr (KS == 4) {
+      score(std::integral_constant<int, 2>{});
+      score(std::integral_constant<int, 3>{});
+    }
+    // The first 32 keys' V fragments arrive during the softmax.
+    i32x4 v0[FT], v1[FT];
+#pragma unroll
+    for (int ft = 0; ft < FT; ++ft) v0[ft] = read_v16<0, RB>(base + va[ft]);
+
+    const int n0 = j * BN;
+    if (n0 + BN > N || (CAUSAL && n0 + BN - 1 > wq0)) {
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) {
+        const int k0 = n0 + 16 * kt + 4 * g;
+        int lim = N - 1 - k0;
+        if (CAUSAL) lim = min(lim, query - k0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (r > lim) st[kt][r] = kNegInf;
+      }
+    }
+    i32x4 pf[2];
+    if constexpr (D == 128) {
+      f32x4 p[4];
+      float sum;
+      auto exps = [&]() {
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            p[kt][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kt][r], sl2, -m_run));
+        sum = p[0][0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) sum += p[i / 4][i % 4];
+      };
+      exps();
+      constexpr float kLazyLimit = 256.f;  // 2^kLazyRescale
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(sum <= kLazyLimit)) != 0, 0)) {
+        float mx = kNegInf;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[i / 4][i % 4]);
+        const float bm = max_over_column(mx) * sl2;
+        const bool move = bm > m_run + kLazyRescale;
+        if (__builtin_amdgcn_ballot_w64(move)) {
+          const float m_new = move ? bm : m_run;
+          const float alpha = move ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
+          l_part *= alpha;
+#pragma unroll
+          for (int ft = 0; ft < FT; ++ft) acc[ft] *= alpha;
+          m_run = m_new;
+          exps();
+        }
+      }
+      l_part += sum;
+      pf[0] = acc_frag2<T>(p[0], p[1]);
+      pf[1] = acc_frag2<T>(p[2], p[3]);
+    } else {
+      float mx = kNegInf;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[i / 4][i % 4]);
+      bool move = mx * sl2 > m_run + kLazyRescale;
+      float m_new = m_run;
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(move) != 0, 0)) {
+        const float bm = max_over_column(mx) * sl2;
+        move = bm > m_run + kLazyRescale;
+        m_new = move ? bm : m_run;
+      }
+      float sum = 0.f;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kt][r], sl2, -m_new));
+          st[kt][r] = pv;
+          sum += pv;
+        }
+      if (__builtin_amdgcn_ballot_w64(move)) {
+        const float alpha = move ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
+        l_part *= alpha;
+#pragma unroll
+        for (int ft = 0; ft < FT; ++ft) acc[ft] *= alpha;
+      }
+      l_part += sum;
+      m_run = m_new;
+      pf[0] = acc_frag2<T>(st[0], st[1]);
+      pf[1] = acc_frag2<T>(st[2], st[3]);
+    }
+    wait_lgkm<0>();
+#pragma unroll
+    for (int ft = 0; ft < FT; ++ft) pin(v0[ft]);
+#pragma unroll
+    for (int ft = 0; ft < FT; ++ft) v1[ft] = read_v16<32, RB>(base + va[ft]);
+#pragma unroll
+    for (int ft = 0; ft < FT; ++ft) acc[ft] = Mma16<T>::run(v0[ft], pf[0], acc[ft]);
+    wait_lgkm<0>();
+#pragma unroll
+    for (int ft = 0; ft < FT; ++ft) pin(v1[ft]);
+#pragma unroll
+    for (int ft = 0; ft < FT; ++ft) acc[ft] = Mma16<T>::run(v1[ft], pf[1], acc[ft]);
+    fill = stage;
+    stage = stage == STAGES - 1 ? 0 : stage + 1;
+  }
+  // No DMA may still write the ring, which stages the O rows (16 per wave) now.
+  wait_vmcnt<0>();
+  __syncthreads();
+
+  const float l = sum_over_column(l_part);
+  const float inv = 1.0f / l;
+  char* const orows = lds + wave * (16 * RB);
+#pragma unroll
+  for (int ft = 0; ft < FT; ++ft) {
+    uint2 u;
+    u.x = pack2<T>(acc[ft][0] * inv, acc[ft][1] * inv);
+    u.y = pack2<T>(acc[ft][2] * inv, acc[ft][3] * inv);
+    *reinterpret_cast<uint2*>(orows + c * RB + (((2 * ft + (g >> 1)) ^ G::oswz(c)) * 16) +
+                              (g & 1) * 8) = u;
+  }
+  T* const Oh = args.O + b * s.o[0] + h * s.o[1] + int64_t(start) * s.o[2];
+  constexpr int LPR = RB / 16, RPI = 64 / LPR;  // lanes per row, rows per instruction
+#pragma unroll
+  for (int p = 0; p < 16 / RPI; ++p) {
+    const int r = p * RPI + lane / LPR, q = lane % LPR;
+    const i32x4 v = *reinterpret_cast<const i32x4*>(orows + r * RB + ((q ^ G::oswz(r)) * 16));
+    if (wq0 + r < N)
+      __builtin_nontemporal_store(v, reinterpret_cast<i32x4*>(Oh + (wq0 + r) * s.o[2] + q * 8));
+  }
+  if (query < N && args.lse != nullptr && g == 0) {
+    const int64_t at = s.cu != nullptr ? int64_t(h) * s.total + start + query
+                                       : (int64_t(b) * s.heads + h) * N + query;
+    args.lse[at] = m_run + __log2f(l);
+  }
+}
+
+// Whether the 64-query kernel takes a problem of `tiles` 64-query tiles (512 are resident at once).
+// 256-query against 64-query kernel in us, bf16, one sequence of N for each of H heads:
+//   causal D64:  H16 N1024 (256 tiles) 23.2 / 12.1, H16 N4096 (1024) 76.7 / 56.4, H16 N8192 (2048)
+//                246 / 195, H256 N512 (2048) 25.7 / 27.0, H64 N4096 (4096) 207 / 207
+//   causal D128: H16 N1024 39.9 / 15.7, H8 N8192 (1024) 180 / 169, H32 N4096 (2048) 121 / 170
+//   full D64:    H32 N1024 (512) 23.8 / 17.1, H16 N4096 (1024) 80 / 100
+//   full D128:   H4 N8192 (512) 168 / 160, H32 N2048 (1024) 61 / 91
+// Causal workgroups end at different times and refill the slots, so they stand more tiles.
+inline bool small_applies(int64_t tiles, int64_t seq, int64_t head_dim, bool causal) {
+  return tiles <= (!causal ? 512 : head_dim == 64 && seq > 512 ? 2048 : 1024);
+}
+
 // Causal head_dim 128, equal lengths: `items` workgroups (paired_items); otherwise one
 // workgroup per query block.
 template <typename T, int D>
-void launch(bool causal, int64_t items, hipStream_t st, const void* q, const void* k,
+void launch(bool small, bool causal, int64_t items, hipStream_t st, const void* q, const void* k,
             const void* v, void* o, float* lse, const Shape& s) {
+  if (small) {
+    const dim3 grid(static_cast<unsigned>(s.tiles)), block(SmallGeo<D>::THREADS);
+    const FwdArgs<T> a{(const T*)q, (const T*)k, (const T*)v, (T*)o, lse, s};
+    if (causal)
+      hipLaunchKernelGGL((attn_fwd_small_kernel<T, D, true>), grid, block, 0, st, a);
+    else
+      hipLaunchKernelGGL((attn_fwd_small_kernel<T, D, false>), grid, block, 0, st, a);
+    return;
+  }
   const int64_t n = kPaired<D> && causal && s.cu == nullptr ? items : int64_t(s.tiles);
   const dim3 grid(static_cast<unsigned>(n));
   const FwdArgs<T> a{(const T*)q, (const T*)k, (const T*)v, (T*)o, lse, s};
@@ -762,19 +1088,24 @@ void attn_fwd_dma_launch(int dtype, const void* q, const void* k, const void* v,
   }
   s.scale_log2 = sm_scale * 1.4426950408889634f;
   s.batch = (int)batch;
-  s.q_blocks = (int)cdiv(seq, 256);
-  s.tiles = cu_seqlens != nullptr ? (int)(varlen_tiles(batch, total, seq, 256) * heads)
-                                  : (int)(s.q_blocks * batch * heads);
+  auto tiles_of = [&](int64_t rows) {
+    return (cu_seqlens != nullptr ? varlen_tiles(batch, total, seq, rows) : batch * cdiv(seq, rows)) *
+           heads;
+  };
+  const bool small = small_applies(tiles_of(64), seq, head_dim, causal);
+  const int64_t rows = small ? 64 : 256;
+  s.q_blocks = (int)cdiv(seq, rows);
+  s.tiles = (int)tiles_of(rows);
   s.k_bytes = (uint32_t)head_extent_bytes(seq, head_dim, k_strides[2]);
   s.v_bytes = (uint32_t)head_extent_bytes(seq, head_dim, v_strides[2]);
   const int64_t items = cu_seqlens == nullptr ? paired_items(batch * heads, s.q_blocks)
                                               : int64_t(s.tiles);
   if (dtype == TK_DTYPE_F16) {
-    if (head_dim == 64) launch<_Float16, 64>(causal, items, stream, q, k, v, o, lse, s);
-    else launch<_Float16, 128>(causal, items, stream, q, k, v, o, lse, s);
+    if (head_dim == 64) launch<_Float16, 64>(small, causal, items, stream, q, k, v, o, lse, s);
+    else launch<_Float16, 128>(small, causal, items, stream, q, k, v, o, lse, s);
   } else {
-    if (head_dim == 64) launch<__bf16, 64>(causal, items, stream, q, k, v, o, lse, s);
-    else launch<__bf16, 128>(causal, items, stream, q, k, v, o, lse, s);
+    if (head_dim == 64) launch<__bf16, 64>(small, causal, items, stream, q, k, v, o, lse, s);
+    else launch<__bf16, 128>(small, causal, items, stream, q, k, v, o, lse, s);
   }
 }
 

@@ -53,7 +53,8 @@ _DTYPES = (torch.float16, torch.bfloat16)
 _LOG2_E = 1.4426950408889634
 
 # Tile configuration of csrc/attention.hip (forward / backward).
-# csrc/attention_fwd.hip (Geo<D>: BM, BN, WAVES, STAGES): 256 queries per workgroup as eight
+# csrc/attention_fwd.hip (Geo<D>: BM, BN, WAVES, STAGES; problems that cannot fill the chip with these
+# take 64 queries per workgroup, SmallGeo<D>, with the same results): 256 queries per workgroup as eight
 # wave64s of 32, key blocks of 64, a 4-stage buffer->LDS K/V ring, v_mfma_f32_16x16x32.
 # "num_warps" counts wave64s.
 FORWARD_TILE = {"hip_kernel": "attn_fwd_dma_kernel", "block_m": 256, "block_n": 64, "num_warps": 8,
