@@ -710,23 +710,29 @@ attn_fwd_dma_kernel(FwdArgs<T> kernel_arg) {
   }  // tiles
 }
 
-// ------------------------------------------------------------------ short problems
+// ------------------------------------------------------------------ small workgroups
 //
 // The same forward for problems whose 256-query workgroups leave CUs idle, where the time is one
 // workgroup's serial walk over its key blocks: a block costs a wave its MFMAs plus its
-// exponentials, one after the other. Here a wave owns 16 queries (half the work per block) and a
-// workgroup 64 (four waves, two workgroups per CU), so four times as many workgroups walk
-// blocks half as long. There is no ping-pong: each wave reads K, forms S, takes its softmax
-// while the V fragments of the block's first half arrive, and multiplies. Twice the LDS reads per
-// MFMA make it slower than the 256-query kernel once that fills the chip (small_applies).
+// exponentials, one after the other. Here a wave owns 16 QT queries (QT 1 or 2) and a workgroup
+// has four waves, several workgroups per CU. QT = 1: four times as many workgroups walk
+// blocks half as long; twice the LDS reads per MFMA make it the slower kernel once the chip is
+// full. QT = 2 reads as much per MFMA as the 256-query kernel; workgroups that are not in step
+// with each other take the place of its ping-pong, and their prologues and epilogues overlap,
+// which pays wherever workgroups are short (ragged batches, causal head_dim 64). Each wave
+// reads K, forms S, takes its softmax while the V fragments of the block's first half arrive,
+// and multiplies.
 //
 // Every query sees the same operations in the same order as in the 256-query kernel, so the
 // results are bitwise the same.
-template <int D>
+template <int D, int QT>
 struct SmallGeo {
   using G = Geo<D>;
-  static constexpr int BM = 64, WAVES = 4, THREADS = 256;
-  static constexpr int STAGES = D == 64 ? 4 : 2;  // 64 KiB: two workgroups per CU
+  static constexpr int QW = 16 * QT;  // queries per wave
+  static constexpr int BM = 4 * QW, WAVES = 4, THREADS = 256;
+  // 48 KiB at head_dim 64 (three workgroups per CU; four stages and two workgroups ran causal
+  // H32 N2048 in 31.8 us against 29.2), 64 KiB at 128 (two).
+  static constexpr int STAGES = D == 64 ? 3 : 2;
   static constexpr int DMA_PER_OP = G::OPB / 1024 / WAVES;
   static constexpr int DPB = 2 * DMA_PER_OP;
 };
@@ -737,7 +743,7 @@ __device__ __forceinline__ void small_dma(__amdgpu_buffer_rsrc_t rk, __amdgpu_bu
                                           char* at, const uint32_t* k_src, const uint32_t* v_src,
                                           uint32_t k_off, uint32_t v_off) {
 #pragma unroll
-  for (int x = 0; x < SmallGeo<D>::DMA_PER_OP; ++x) {
+  for (int x = 0; x < SmallGeo<D, 1>::DMA_PER_OP; ++x) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_void*)(at + x * 1024), 16, k_src[x], k_off,
                                              0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_void*)(at + Geo<D>::OPB + x * 1024), 16,
@@ -745,11 +751,11 @@ __device__ __forceinline__ void small_dma(__amdgpu_buffer_rsrc_t rk, __amdgpu_bu
   }
 }
 
-template <typename T, int D, bool CAUSAL>
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2))) void
+template <typename T, int D, int QT, bool CAUSAL>
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(D == 64 ? 3 : 2))) void
 attn_fwd_small_kernel(FwdArgs<T> args) {
   using G = Geo<D>;
-  using S = SmallGeo<D>;
+  using S = SmallGeo<D, QT>;
   constexpr int BN = G::BN, KS = G::KS, FT = G::FT, RB = G::RB, OPB = G::OPB, STB = G::STB,
                 STAGES = S::STAGES;
   __shared__ __attribute__((aligned(1024))) char lds[STAGES * STB];
@@ -795,7 +801,7 @@ attn_fwd_small_kernel(FwdArgs<T> args) {
   const T* Kh = args.K + b * s.k[0] + kvh * s.k[1] + int64_t(start) * s.k[2];
   const T* Vh = args.V + b * s.v[0] + kvh * s.v[1] + int64_t(start) * s.v[2];
   const int q0 = qb * S::BM;
-  const int wq0 = q0 + wave * 16;
+  const int wq0 = q0 + wave * S::QW;
   const __amdgpu_buffer_rsrc_t rk =
       __builtin_amdgcn_make_buffer_rsrc((void*)Kh, (short)0, k_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rv =
@@ -821,21 +827,25 @@ attn_fwd_small_kernel(FwdArgs<T> args) {
   for (int blk = 0; blk < STAGES - 1; ++blk) load(blk, blk);
 
   // Q fragments, rotated if asked, as in the 256-query kernel.
-  const int query = wq0 + c;
-  i32x4 qf[KS];
+  i32x4 qf[QT][KS];
 #pragma unroll
-  for (int kk = 0; kk < KS; ++kk)
-    qf[kk] = query < N ? *reinterpret_cast<const i32x4*>(Qh + query * s.q[2] + kk * 32 + g * 8)
+  for (int qt = 0; qt < QT; ++qt) {
+    const int query = wq0 + 16 * qt + c;
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk)
+      qf[qt][kk] = query < N
+                       ? *reinterpret_cast<const i32x4*>(Qh + query * s.q[2] + kk * 32 + g * 8)
                        : i32x4{0, 0, 0, 0};
-  if (s.rope_cos != nullptr) {
-    const int64_t at = int64_t(query) * s.rope_stride + g * 8;
-    const T* cr = static_cast<const T*>(s.rope_cos) + at;
-    const T* sr = static_cast<const T*>(s.rope_sin) + at;
+    if (s.rope_cos != nullptr) {
+      const int64_t at = int64_t(query) * s.rope_stride + g * 8;
+      const T* cr = static_cast<const T*>(s.rope_cos) + at;
+      const T* sr = static_cast<const T*>(s.rope_sin) + at;
 #pragma unroll
-    for (int kk = 0; kk < KS / 2; ++kk) {
-      const i32x4 cv = query < N ? *reinterpret_cast<const i32x4*>(cr + kk * 32) : i32x4{0, 0, 0, 0};
-      const i32x4 sv = query < N ? *reinterpret_cast<const i32x4*>(sr + kk * 32) : i32x4{0, 0, 0, 0};
-      rope_fragment<T>(qf[kk], qf[kk + KS / 2], cv, sv);
+      for (int kk = 0; kk < KS / 2; ++kk) {
+        const i32x4 cv = query < N ? *reinterpret_cast<const i32x4*>(cr + kk * 32) : i32x4{0, 0, 0, 0};
+        const i32x4 sv = query < N ? *reinterpret_cast<const i32x4*>(sr + kk * 32) : i32x4{0, 0, 0, 0};
+        rope_fragment<T>(qf[qt][kk], qf[qt][kk + KS / 2], cv, sv);
+      }
     }
   }
   uint32_t ka[KS], va[FT];
@@ -847,13 +857,22 @@ attn_fwd_small_kernel(FwdArgs<T> args) {
     for (int ft = 0; ft < FT; ++ft) va[ft] = OPB + row * RB + ((ft ^ G::vswz(row)) * 32) + q * 8;
   }
 
-  f32x4 acc[FT];
+  f32x4 acc[FT][QT];
 #pragma unroll
-  for (int ft = 0; ft < FT; ++ft) acc[ft] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = kNegInf, l_part = 0.f;
+  for (int ft = 0; ft < FT; ++ft)
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) acc[ft][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run[QT], l_part[QT];
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    m_run[qt] = kNegInf;
+    l_part[qt] = 0.f;
+  }
   const float sl2 = s.scale_log2;
   int stage = 0, fill = STAGES - 1;
-  for (int j = 0; j < blocks; ++j) {
+  // Blocks this wave needs (causal: those that start at or before its last query).
+  const int mine = CAUSAL && QT > 1 ? min(blocks, (wq0 + S::QW - 1) / BN + 1) : blocks;
+  for (int j = 0; j < mine; ++j) {
     // Block j has landed in every wave's share, and every wave has read block j - 1, whose stage
     // takes block j + STAGES - 1.
     wait_vmcnt<(STAGES - 2) * S::DPB>();
@@ -868,7 +887,7 @@ attn_fwd_small_kernel(FwdArgs<T> args) {
       kf[kk][3] = lds_read_b128<48 * RB>(base + ka[kk]);
     }
     load(j + STAGES - 1, fill);
-    f32x4 st[4];
+    f32x4 st[QT][4];
     auto score = [&](auto step) {
       constexpr int kk = decltype(step)::value;
       wait_lgkm<4 * (KS - 1 - kk) < 15 ? 4 * (KS - 1 - kk) : 15>();
@@ -876,7 +895,10 @@ attn_fwd_small_kernel(FwdArgs<T> args) {
       for (int kt = 0; kt < 4; ++kt) pin(kf[kk][kt]);
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)
-        st[kt] = Mma16<T>::run(kf[kk][kt], qf[kk], kk == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : st[kt]);
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt)
+          st[qt][kt] = Mma16<T>::run(kf[kk][kt], qf[qt][kk],
+                                     kk == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : st[qt][kt]);
     };
     score(std::integral_constant<int, 0>{});
     score(std::integral_constant<int, 1>{});
@@ -892,80 +914,85 @@ attn_fwd_small_kernel(FwdArgs<T> args) {
     const int n0 = j * BN;
     if (n0 + BN > N || (CAUSAL && n0 + BN - 1 > wq0)) {
 #pragma unroll
-      for (int kt = 0; kt < 4; ++kt) {
-        const int k0 = n0 + 16 * kt + 4 * g;
-        int lim = N - 1 - k0;
-        if (CAUSAL) lim = min(lim, query - k0);
+      for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (r > lim) st[kt][r] = kNegInf;
-      }
+        for (int kt = 0; kt < 4; ++kt) {
+          const int k0 = n0 + 16 * kt + 4 * g;
+          int lim = N - 1 - k0;
+          if (CAUSAL) lim = min(lim, wq0 + 16 * qt + c - k0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (r > lim) st[qt][kt][r] = kNegInf;
+        }
     }
-    i32x4 pf[2];
-    if constexpr (D == 128) {
-      f32x4 p[4];
-      float sum;
-      auto exps = [&]() {
+    i32x4 pf[QT][2];
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      if constexpr (D == 128) {
+        f32x4 p[4];
+        float sum;
+        auto exps = [&]() {
+#pragma unroll
+          for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              p[kt][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[qt][kt][r], sl2, -m_run[qt]));
+          sum = p[0][0];
+#pragma unroll
+          for (int i = 1; i < 16; ++i) sum += p[i / 4][i % 4];
+        };
+        exps();
+        constexpr float kLazyLimit = 256.f;  // 2^kLazyRescale
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(sum <= kLazyLimit)) != 0, 0)) {
+          float mx = kNegInf;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[qt][i / 4][i % 4]);
+          const float bm = max_over_column(mx) * sl2;
+          const bool move = bm > m_run[qt] + kLazyRescale;
+          if (__builtin_amdgcn_ballot_w64(move)) {
+            const float m_new = move ? bm : m_run[qt];
+            const float alpha = move ? __builtin_amdgcn_exp2f(m_run[qt] - m_new) : 1.f;
+            l_part[qt] *= alpha;
+#pragma unroll
+            for (int ft = 0; ft < FT; ++ft) acc[ft][qt] *= alpha;
+            m_run[qt] = m_new;
+            exps();
+          }
+        }
+        l_part[qt] += sum;
+        pf[qt][0] = acc_frag2<T>(p[0], p[1]);
+        pf[qt][1] = acc_frag2<T>(p[2], p[3]);
+      } else {
+        float mx = kNegInf;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[qt][i / 4][i % 4]);
+        bool move = mx * sl2 > m_run[qt] + kLazyRescale;
+        float m_new = m_run[qt];
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(move) != 0, 0)) {
+          const float bm = max_over_column(mx) * sl2;
+          move = bm > m_run[qt] + kLazyRescale;
+          m_new = move ? bm : m_run[qt];
+        }
+        float sum = 0.f;
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            p[kt][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kt][r], sl2, -m_run));
-        sum = p[0][0];
-#pragma unroll
-        for (int i = 1; i < 16; ++i) sum += p[i / 4][i % 4];
-      };
-      exps();
-      constexpr float kLazyLimit = 256.f;  // 2^kLazyRescale
-      if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(sum <= kLazyLimit)) != 0, 0)) {
-        float mx = kNegInf;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[i / 4][i % 4]);
-        const float bm = max_over_column(mx) * sl2;
-        const bool move = bm > m_run + kLazyRescale;
+          for (int r = 0; r < 4; ++r) {
+            const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(st[qt][kt][r], sl2, -m_new));
+            st[qt][kt][r] = pv;
+            sum += pv;
+          }
         if (__builtin_amdgcn_ballot_w64(move)) {
-          const float m_new = move ? bm : m_run;
-          const float alpha = move ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
-          l_part *= alpha;
+          const float alpha = move ? __builtin_amdgcn_exp2f(m_run[qt] - m_new) : 1.f;
+          l_part[qt] *= alpha;
 #pragma unroll
-          for (int ft = 0; ft < FT; ++ft) acc[ft] *= alpha;
-          m_run = m_new;
-          exps();
+          for (int ft = 0; ft < FT; ++ft) acc[ft][qt] *= alpha;
         }
+        l_part[qt] += sum;
+        m_run[qt] = m_new;
+        pf[qt][0] = acc_frag2<T>(st[qt][0], st[qt][1]);
+        pf[qt][1] = acc_frag2<T>(st[qt][2], st[qt][3]);
       }
-      l_part += sum;
-      pf[0] = acc_frag2<T>(p[0], p[1]);
-      pf[1] = acc_frag2<T>(p[2], p[3]);
-    } else {
-      float mx = kNegInf;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[i / 4][i % 4]);
-      bool move = mx * sl2 > m_run + kLazyRescale;
-      float m_new = m_run;
-      if (__builtin_expect(__builtin_amdgcn_ballot_w64(move) != 0, 0)) {
-        const float bm = max_over_column(mx) * sl2;
-        move = bm > m_run + kLazyRescale;
-        m_new = move ? bm : m_run;
-      }
-      float sum = 0.f;
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kt][r], sl2, -m_new));
-          st[kt][r] = pv;
-          sum += pv;
-        }
-      if (__builtin_amdgcn_ballot_w64(move)) {
-        const float alpha = move ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
-        l_part *= alpha;
-#pragma unroll
-        for (int ft = 0; ft < FT; ++ft) acc[ft] *= alpha;
-      }
-      l_part += sum;
-      m_run = m_new;
-      pf[0] = acc_frag2<T>(st[0], st[1]);
-      pf[1] = acc_frag2<T>(st[2], st[3]);
     }
     wait_lgkm<0>();
 #pragma unroll
@@ -973,12 +1000,24 @@ attn_fwd_small_kernel(FwdArgs<T> args) {
 #pragma unroll
     for (int ft = 0; ft < FT; ++ft) v1[ft] = read_v16<32, RB>(base + va[ft]);
 #pragma unroll
-    for (int ft = 0; ft < FT; ++ft) acc[ft] = Mma16<T>::run(v0[ft], pf[0], acc[ft]);
+    for (int ft = 0; ft < FT; ++ft)
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) acc[ft][qt] = Mma16<T>::run(v0[ft], pf[qt][0], acc[ft][qt]);
     wait_lgkm<0>();
 #pragma unroll
     for (int ft = 0; ft < FT; ++ft) pin(v1[ft]);
 #pragma unroll
-    for (int ft = 0; ft < FT; ++ft) acc[ft] = Mma16<T>::run(v1[ft], pf[1], acc[ft]);
+    for (int ft = 0; ft < FT; ++ft)
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) acc[ft][qt] = Mma16<T>::run(v1[ft], pf[qt][1], acc[ft][qt]);
+    fill = stage;
+    stage = stage == STAGES - 1 ? 0 : stage + 1;
+  }
+  // The barriers and loads of the blocks that only later waves need.
+  for (int j = mine; j < blocks; ++j) {
+    wait_vmcnt<(STAGES - 2) * S::DPB>();
+    barrier_no_fence();
+    load(j + STAGES - 1, fill);
     fill = stage;
     stage = stage == STAGES - 1 ? 0 : stage + 1;
   }
@@ -986,57 +1025,76 @@ attn_fwd_small_kernel(FwdArgs<T> args) {
   wait_vmcnt<0>();
   __syncthreads();
 
-  const float l = sum_over_column(l_part);
-  const float inv = 1.0f / l;
   char* const orows = lds + wave * (16 * RB);
-#pragma unroll
-  for (int ft = 0; ft < FT; ++ft) {
-    uint2 u;
-    u.x = pack2<T>(acc[ft][0] * inv, acc[ft][1] * inv);
-    u.y = pack2<T>(acc[ft][2] * inv, acc[ft][3] * inv);
-    *reinterpret_cast<uint2*>(orows + c * RB + (((2 * ft + (g >> 1)) ^ G::oswz(c)) * 16) +
-                              (g & 1) * 8) = u;
-  }
   T* const Oh = args.O + b * s.o[0] + h * s.o[1] + int64_t(start) * s.o[2];
-  constexpr int LPR = RB / 16, RPI = 64 / LPR;  // lanes per row, rows per instruction
 #pragma unroll
-  for (int p = 0; p < 16 / RPI; ++p) {
-    const int r = p * RPI + lane / LPR, q = lane % LPR;
-    const i32x4 v = *reinterpret_cast<const i32x4*>(orows + r * RB + ((q ^ G::oswz(r)) * 16));
-    if (wq0 + r < N)
-      __builtin_nontemporal_store(v, reinterpret_cast<i32x4*>(Oh + (wq0 + r) * s.o[2] + q * 8));
-  }
-  if (query < N && args.lse != nullptr && g == 0) {
-    const int64_t at = s.cu != nullptr ? int64_t(h) * s.total + start + query
-                                       : (int64_t(b) * s.heads + h) * N + query;
-    args.lse[at] = m_run + __log2f(l);
+  for (int qt = 0; qt < QT; ++qt) {
+    const float l = sum_over_column(l_part[qt]);
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int ft = 0; ft < FT; ++ft) {
+      uint2 u;
+      u.x = pack2<T>(acc[ft][qt][0] * inv, acc[ft][qt][1] * inv);
+      u.y = pack2<T>(acc[ft][qt][2] * inv, acc[ft][qt][3] * inv);
+      *reinterpret_cast<uint2*>(orows + c * RB + (((2 * ft + (g >> 1)) ^ G::oswz(c)) * 16) +
+                                (g & 1) * 8) = u;
+    }
+    constexpr int LPR = RB / 16, RPI = 64 / LPR;  // lanes per row, rows per instruction
+#pragma unroll
+    for (int p = 0; p < 16 / RPI; ++p) {
+      const int r = p * RPI + lane / LPR, q = lane % LPR;
+      const i32x4 v = *reinterpret_cast<const i32x4*>(orows + r * RB + ((q ^ G::oswz(r)) * 16));
+      const int row_query = wq0 + 16 * qt + r;
+      if (row_query < N)
+        __builtin_nontemporal_store(v, reinterpret_cast<i32x4*>(Oh + row_query * s.o[2] + q * 8));
+    }
+    const int query = wq0 + 16 * qt + c;
+    if (query < N && args.lse != nullptr && g == 0) {
+      const int64_t at = s.cu != nullptr ? int64_t(h) * s.total + start + query
+                                         : (int64_t(b) * s.heads + h) * N + query;
+      args.lse[at] = m_run[qt] + __log2f(l);
+    }
   }
 }
 
-// Whether the 64-query kernel takes a problem of `tiles` 64-query tiles (512 are resident at once).
-// 256-query against 64-query kernel in us, bf16, one sequence of N for each of H heads:
-//   causal D64:  H16 N1024 (256 tiles) 23.2 / 12.1, H16 N4096 (1024) 76.7 / 56.4, H16 N8192 (2048)
-//                246 / 195, H256 N512 (2048) 25.7 / 27.0, H64 N4096 (4096) 207 / 207
-//   causal D128: H16 N1024 39.9 / 15.7, H8 N8192 (1024) 180 / 169, H32 N4096 (2048) 121 / 170
-//   full D64:    H32 N1024 (512) 23.8 / 17.1, H16 N4096 (1024) 80 / 100
-//   full D128:   H4 N8192 (512) 168 / 160, H32 N2048 (1024) 61 / 91
-// Causal workgroups end at different times and refill the slots, so they stand more tiles.
-inline bool small_applies(int64_t tiles, int64_t seq, int64_t head_dim, bool causal) {
-  return tiles <= (!causal ? 512 : head_dim == 64 && seq > 512 ? 2048 : 1024);
+// Query tiles per wave of the small-workgroup kernel for a problem of `tiles` 64-query tiles, or 0
+// for the 256-query kernel. 256-query / QT 1 / QT 2 in us, bf16, one sequence of N for H heads:
+//   causal D64:  H16 N1024 (256 tiles) 23.3/12.0/16.8, H16 N4096 (1024) 77/52/57,
+//                H16 N8192 (2048) 244/174/160, H64 N8192 (8192) 635/700/587,
+//                H128 N8192 (16384) 1176/-/1211
+//   causal D128: H32 N1024 (512) 40.7/19.0/24.0, H8 N8192 (1024) 180/167/157,
+//                H256 N512 (2048) 39.9/39.8/34.1, H64 N2048 (2048) 67.9/87.8/74.1
+//   full D64:    H32 N1024 (512) 23.6/16.2/18.3, H64 N1024 (1024) 25.1/27.4/26.3
+//   full D128:   H4 N8192 (512) 179/165/147, H64 N1024 (1024) 33.4/46.8/37.4
+//   varlen D128, H32: causal 15 sequences in 12000 tokens 185/187/168, 32 in 12000 150/138/111,
+//                3 in 12000 (to 6000) 523/717/543; full 15 in 12000 257/321/241, 4 in 8000
+//                348/452/377
+int small_query_tiles(int64_t tiles, int64_t seq, int64_t head_dim, bool causal, bool varlen) {
+  if (tiles <= 512) return 1;
+  if (causal && head_dim == 64) return tiles <= 1024 ? 1 : tiles <= 8192 ? 2 : 0;
+  if (causal) {
+    const bool fits = tiles <= 1024 || (tiles <= 2048 && seq <= 1024);
+    return fits || (varlen && seq <= 4096) ? 2 : 0;
+  }
+  return varlen && head_dim == 128 && seq <= 2048 ? 2 : 0;
 }
 
 // Causal head_dim 128, equal lengths: `items` workgroups (paired_items); otherwise one
 // workgroup per query block.
 template <typename T, int D>
-void launch(bool small, bool causal, int64_t items, hipStream_t st, const void* q, const void* k,
+void launch(int small, bool causal, int64_t items, hipStream_t st, const void* q, const void* k,
             const void* v, void* o, float* lse, const Shape& s) {
   if (small) {
-    const dim3 grid(static_cast<unsigned>(s.tiles)), block(SmallGeo<D>::THREADS);
+    const dim3 grid(static_cast<unsigned>(s.tiles)), block(SmallGeo<D, 1>::THREADS);
     const FwdArgs<T> a{(const T*)q, (const T*)k, (const T*)v, (T*)o, lse, s};
-    if (causal)
-      hipLaunchKernelGGL((attn_fwd_small_kernel<T, D, true>), grid, block, 0, st, a);
+    if (causal && small == 1)
+      hipLaunchKernelGGL((attn_fwd_small_kernel<T, D, 1, true>), grid, block, 0, st, a);
+    else if (causal)
+      hipLaunchKernelGGL((attn_fwd_small_kernel<T, D, 2, true>), grid, block, 0, st, a);
+    else if (small == 1)
+      hipLaunchKernelGGL((attn_fwd_small_kernel<T, D, 1, false>), grid, block, 0, st, a);
     else
-      hipLaunchKernelGGL((attn_fwd_small_kernel<T, D, false>), grid, block, 0, st, a);
+      hipLaunchKernelGGL((attn_fwd_small_kernel<T, D, 2, false>), grid, block, 0, st, a);
     return;
   }
   const int64_t n = kPaired<D> && causal && s.cu == nullptr ? items : int64_t(s.tiles);
@@ -1092,8 +1150,8 @@ void attn_fwd_dma_launch(int dtype, const void* q, const void* k, const void* v,
     return (cu_seqlens != nullptr ? varlen_tiles(batch, total, seq, rows) : batch * cdiv(seq, rows)) *
            heads;
   };
-  const bool small = small_applies(tiles_of(64), seq, head_dim, causal);
-  const int64_t rows = small ? 64 : 256;
+  const int small = small_query_tiles(tiles_of(64), seq, head_dim, causal, cu_seqlens != nullptr);
+  const int64_t rows = small ? 64 * small : 256;
   s.q_blocks = (int)cdiv(seq, rows);
   s.tiles = (int)tiles_of(rows);
   s.k_bytes = (uint32_t)head_extent_bytes(seq, head_dim, k_strides[2]);
