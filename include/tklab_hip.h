@@ -205,6 +205,20 @@ int tk_gemm_rowscale(int dtype, const void* a, const void* b, const float* row_s
                      int64_t stride_bk, int64_t stride_bn, int64_t stride_cm, int64_t stride_cn,
                      void* stream);
 
+/* tk_gemm, tk_gemm_rowscale (row_scale non-null) or tk_gemm_swiglu (b = the gate and b_up the
+ * up weight; at most one of b_up and row_scale) with K cut into `splits` runs of whole 64-wide
+ * tiles, 1 <= splits <= ceil(k / 64): one workgroup each for problems with too few output tiles
+ * to fill the chip. `workspace` (float32, 16-byte aligned, splits * m * n values, twice that
+ * with b_up) holds the runs' sums, which are added in order of K in float32 and rounded once, so
+ * the result is deterministic; all three variants add in the same order. Operands the DMA
+ * kernels do not take run as the unsplit entry points. No reference counterpart
+ * (src/tklab/kernels/matmul.py:72-164 computes each tile in one program). */
+int tk_gemm_splitk(int dtype, const void* a, const void* b, const void* b_up,
+                   const float* row_scale, void* c, float* workspace, int64_t m, int64_t n,
+                   int64_t k, int64_t splits, int64_t stride_am, int64_t stride_ak,
+                   int64_t stride_bk, int64_t stride_bn, int64_t stride_uk, int64_t stride_un,
+                   int64_t stride_cm, int64_t stride_cn, void* stream);
+
 /* Row scaling y[r, c] = round_dtype(x[r, c] * scale[r]) for x, y [rows, cols]
  * (unit column stride) and scale[rows] in the same dtype: folds a normalization
  * weight into the projection that follows it (see tk_gemm_rowscale). Helper of

@@ -312,6 +312,49 @@ extern "C" int tk_gemm(int dtype, const void* a, const void* b, void* c, int64_t
   return tk::check_launch("gemm");
 }
 
+extern "C" int tk_gemm_splitk(int dtype, const void* a, const void* b, const void* b_up,
+                              const float* row_scale, void* c, float* workspace, int64_t m,
+                              int64_t n, int64_t k, int64_t splits, int64_t stride_am,
+                              int64_t stride_ak, int64_t stride_bk, int64_t stride_bn,
+                              int64_t stride_uk, int64_t stride_un, int64_t stride_cm,
+                              int64_t stride_cn, void* stream) {
+  if (dtype != TK_DTYPE_F16 && dtype != TK_DTYPE_BF16)
+    return tk::fail("gemm_splitk: dtype must be float16 or bfloat16");
+  if (a == nullptr || b == nullptr || c == nullptr || workspace == nullptr)
+    return tk::fail("gemm_splitk: null pointer");
+  const int64_t strides[8] = {stride_am, stride_ak, stride_bk, stride_bn,
+                              b_up != nullptr ? stride_uk : 1, b_up != nullptr ? stride_un : 1,
+                              stride_cm, stride_cn};
+  for (int64_t s : strides)
+    if (s <= 0) return tk::fail("gemm_splitk: strides must be positive");
+  if (b_up != nullptr && row_scale != nullptr)
+    return tk::fail("gemm_splitk: either a second weight or row scales");
+  if (m <= 0 || n <= 0 || k <= 0) return tk::fail("gemm_splitk: empty problem");
+  const int64_t kt = tk::cdiv(k, 64);
+  if (splits <= 0 || splits > kt || splits > 65535)
+    return tk::fail("gemm_splitk: splits must be between 1 and the 64-wide tiles of K");
+  const int64_t lim = INT32_MAX;
+  if (m > lim || n > lim || k > lim || tk::extent(m, stride_cm, n, stride_cn) > lim)
+    return tk::fail("gemm_splitk: operand exceeds the int32 offset range");
+  if ((reinterpret_cast<uintptr_t>(workspace) & 15) != 0)
+    return tk::fail("gemm_splitk: workspace must be 16-byte aligned");
+  if (tk::cdiv(m, 64) * tk::cdiv(n, 64) > INT32_MAX || tk::cdiv(m * tk::cdiv(n, 4), 256) > INT32_MAX)
+    return tk::fail("gemm_splitk: too many tiles");
+  // Layouts the DMA kernels do not take run unsplit.
+  if (!tk::gemm_split_launch(dtype, a, b, b_up, row_scale, c, workspace, m, n, k, splits, strides,
+                             tk::as_stream(stream))) {
+    if (b_up != nullptr)
+      return tk_gemm_swiglu(dtype, a, b, b_up, c, m, n, k, stride_am, stride_ak, stride_bk,
+                            stride_bn, stride_uk, stride_un, stride_cm, stride_cn, stream);
+    if (row_scale != nullptr)
+      return tk_gemm_rowscale(dtype, a, b, row_scale, c, m, n, k, stride_am, stride_ak, stride_bk,
+                              stride_bn, stride_cm, stride_cn, stream);
+    return tk_gemm(dtype, a, b, c, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, stride_cm,
+                   stride_cn, 0, stream);
+  }
+  return tk::check_launch("gemm_splitk");
+}
+
 extern "C" int tk_gemm_swiglu(int dtype, const void* a, const void* b_gate, const void* b_up,
                               void* y, int64_t m, int64_t n, int64_t k, int64_t stride_am,
                               int64_t stride_ak, int64_t stride_gk, int64_t stride_gn,

@@ -37,6 +37,13 @@ void gemm_dma_launch(const gemm_dma::Plan& plan, int dtype, const void* a, const
                      int64_t m, int64_t n, int64_t k, int64_t stride_cm, int64_t stride_cn,
                      hipStream_t stream, const float* row_scale = nullptr);
 
+// Enqueues the split-K kernels (gemm_tile_kernels.hpp), plain, row-scaled (row_scale) or SwiGLU
+// (b_up), with `partial` holding splits * m * n float32 sums (twice that for SwiGLU); strides:
+// am, ak, bk, bn, up k, up n, cm, cn. False when the DMA kernels do not handle the problem.
+bool gemm_split_launch(int dtype, const void* a, const void* b, const void* b_up,
+                       const float* row_scale, void* c, float* partial, int64_t m, int64_t n,
+                       int64_t k, int64_t splits, const int64_t* strides, hipStream_t stream);
+
 // Enqueues the SwiGLU-fused DMA kernel: y = swiglu(value = a * b_up, gate = a * b_gate),
 // both weights [K, N] row-major; each must satisfy gemm_dma_applies with `a`.
 void gemm_swiglu_dma_launch(int dtype, const void* a, const void* b_gate, const void* b_up,

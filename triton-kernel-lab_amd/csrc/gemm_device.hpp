@@ -32,6 +32,9 @@ struct Problem {
   int tiles_m, tiles_n;
   uint32_t a_bytes, b_bytes, b2_bytes;
   const float* row_scale;  // kRowScale: C[m, :] = round(row_scale[m] * acc)
+  // Split K: the float32 sums, and how many 64-wide K tiles a workgroup takes.
+  float* partial = nullptr;
+  int split_tiles = 0;
 };
 
 template <int N>

@@ -573,6 +573,56 @@ void gemm_dma_launch(const gemm_dma::Plan& plan, int dtype, const void* a, const
   }
 }
 
+bool gemm_split_launch(int dtype, const void* a, const void* b, const void* b_up,
+                       const float* row_scale, void* c, float* partial, int64_t m, int64_t n,
+                       int64_t k, int64_t splits, const int64_t* strides, hipStream_t stream) {
+  const int64_t sam = strides[0], sak = strides[1], sbk = strides[2], sbn = strides[3];
+  const int64_t suk = strides[4], sun = strides[5];
+  int64_t scm = strides[6], scn = strides[7];
+  gemm_dma::Plan plan;
+  if (!gemm_dma::plan(a, b, m, n, k, sam, sak, sbk, sbn, &plan)) return false;
+  const Variant variant = b_up != nullptr        ? Variant::kSwiGLU
+                          : row_scale != nullptr ? Variant::kRowScale
+                                                 : Variant::kPlain;
+  if (variant != Variant::kPlain &&
+      (plan.layout != Layout::NN || plan.swap ||
+       !gemm_dma_applies(a, b, m, n, k, sam, sak, sbk, sbn) ||
+       (b_up != nullptr && !gemm_dma_applies(a, b_up, m, n, k, sam, sak, suk, sun))))
+    return false;
+  if (plan.swap) {
+    std::swap(a, b);
+    std::swap(m, n);
+    std::swap(scm, scn);
+  }
+  const bool a_rows = plan.layout == Layout::TN, b_wide = plan.layout == Layout::NT;
+  auto bytes = [](int64_t rows, int64_t ld, int64_t cols) {
+    return (uint32_t)(((rows - 1) * ld + cols) * 2);
+  };
+  const int64_t kt = cdiv(k, 64), per = cdiv(kt, splits);
+  Problem p{(int)m,
+            (int)n,
+            (int)k,
+            (int)plan.lda,
+            (int)plan.ldb,
+            (int)(b_up != nullptr ? suk : plan.ldb),
+            scm,
+            scn,
+            (int)cdiv(m, 64),
+            (int)cdiv(n, 64),
+            bytes(a_rows ? k : m, plan.lda, a_rows ? m : k),
+            bytes(b_wide ? n : k, plan.ldb, b_wide ? k : n),
+            b_up != nullptr ? bytes(k, suk, n) : 0u,
+            row_scale,
+            partial,
+            (int)per};
+  const int runs = (int)cdiv(kt, per);  // no run is empty
+  if (dtype == TK_DTYPE_F16)
+    launch_split<_Float16>(variant, plan, a, b, b_up, c, p, runs, stream);
+  else
+    launch_split<__bf16>(variant, plan, a, b, b_up, c, p, runs, stream);
+  return true;
+}
+
 void gemm_swiglu_dma_launch(int dtype, const void* a, const void* b_gate, const void* b_up,
                             void* y, int64_t m, int64_t n, int64_t k, int64_t stride_am,
                             int64_t stride_gk, int64_t stride_uk, int64_t stride_ym,

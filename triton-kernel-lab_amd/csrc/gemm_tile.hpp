@@ -26,5 +26,11 @@ template <typename T>
 void launch_tile(int tile, Variant variant, const Plan& plan, const void* a, const void* b,
                  const void* b2, void* c, const Problem& p, hipStream_t stream);
 
+// Enqueues the split-K kernels: 64 x 64 tiles (64 x 128 for SwiGLU: 64 output columns) of a problem
+// whose tile counts, partial and split_tiles are filled in, `splits` runs of K tiles.
+template <typename T>
+void launch_split(Variant variant, const Plan& plan, const void* a, const void* b, const void* b2,
+                  void* c, const Problem& p, int splits, hipStream_t stream);
+
 }  // namespace gemm_dma
 }  // namespace tk

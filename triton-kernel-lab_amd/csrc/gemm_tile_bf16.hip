@@ -6,6 +6,8 @@ namespace gemm_dma {
 
 template void launch_tile<__bf16>(int, Variant, const Plan&, const void*, const void*, const void*,
                                void*, const Problem&, hipStream_t);
+template void launch_split<__bf16>(Variant, const Plan&, const void*, const void*, const void*,
+                                void*, const Problem&, int, hipStream_t);
 
 }  // namespace gemm_dma
 }  // namespace tk

@@ -112,8 +112,10 @@ __device__ __forceinline__ void unroll(F&& f) {
   }
 }
 
-// kAnyK: K need not be a multiple of 32.
-template <typename T, int BM, int BN, int kStages, Layout kLayout, bool kAnyK, Variant kVariant>
+// kAnyK: K need not be a multiple of 32. kSplit: workgroup (x, y) sums the y-th run of
+// p.split_tiles K tiles into p.partial (gemm_split_kernel).
+template <typename T, int BM, int BN, int kStages, Layout kLayout, bool kAnyK, Variant kVariant,
+          bool kSplit = false>
 __device__ __forceinline__ void gemm_tile(const T* __restrict__ A, const T* __restrict__ B,
                                           const T* __restrict__ B2, T* __restrict__ C,
                                           const Problem& p) {
@@ -149,6 +151,8 @@ __device__ __forceinline__ void gemm_tile(const T* __restrict__ A, const T* __re
   if constexpr (!kAnyK) __builtin_assume(p.k % 32 == 0);
   const int kt = (p.k + kTileK - 1) / kTileK;
   const int kv = p.k - (kt - 1) * kTileK;
+  const int first = kSplit ? int(blockIdx.y) * p.split_tiles : 0;  // K tiles first .. end - 1
+  const int end = kSplit ? min(kt, first + p.split_tiles) : kt;
   // Instruction x of wave w is instruction x * 8 + w of the operand's tile; with SwiGLU the
   // first half of them reads the gate weight.
   uint32_t a_src[kADma], a_last[kADma], b_src[kBDma], b_last[kBDma];
@@ -172,19 +176,19 @@ __device__ __forceinline__ void gemm_tile(const T* __restrict__ A, const T* __re
   // Tiles past the end reload the last one into a stage that is never read, keeping every
   // tile's DMA count constant.
   auto load = [&](int tile, int stage) {
-    const bool end = tile >= kt - 1;
-    tile = min(tile, kt - 1);
+    tile = min(tile, end - 1);
+    const bool last = tile == kt - 1;
     char* at = lds + stage * kStageBytes + wave * 1024;
 #pragma unroll
     for (int x = 0; x < kADma; ++x)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void*)(at + x * 8192), 16,
-                                               end ? a_last[x] : a_src[x], tile * a_step, 0, 0);
+                                               last ? a_last[x] : a_src[x], tile * a_step, 0, 0);
     at += BM * 128;
 #pragma unroll
     for (int x = 0; x < kBDma; ++x) {
       const bool up = kSwiGLU && x >= kBDma / 2;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(up ? rb2 : rb, (lds_void*)(at + x * 8192), 16,
-                                               end ? b_last[x] : b_src[x],
+                                               last ? b_last[x] : b_src[x],
                                                tile * (up ? b2_step : b_step), 0, 0);
     }
   };
@@ -206,11 +210,11 @@ __device__ __forceinline__ void gemm_tile(const T* __restrict__ A, const T* __re
     for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
 #pragma unroll
-  for (int t = 0; t < kStages - 1; ++t) load(t, t);
+  for (int t = 0; t < kStages - 1; ++t) load(first + t, t);
 
   i32x4 a0[MT], b0[NT], a1[MT], b1[NT];
   int stage = 0, fill = kStages - 1;
-  for (int t = 0; t < kt; ++t) {
+  for (int t = first; t < end; ++t) {
     wait_vmcnt<(kStages - 2) * (kADma + kBDma)>();
     barrier_no_fence();
     const uint32_t base = lds_base + stage * kStageBytes;
@@ -237,6 +241,30 @@ __device__ __forceinline__ void gemm_tile(const T* __restrict__ A, const T* __re
     stage = stage == kStages - 1 ? 0 : stage + 1;
   }
   wait_vmcnt<0>();
+  if constexpr (kSplit) {
+    // [split][gate, up][m][n] float32; a lane's four values are consecutive columns.
+    const int64_t plane = int64_t(p.m) * p.n;
+    constexpr int kPlanes = kSwiGLU ? 2 : 1, kTiles = NT / kPlanes;
+    float* out = p.partial + blockIdx.y * kPlanes * plane;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int m = m0 + wm + i * 16 + l16;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int n = n0 + wq * (kOutN / WN) + (j % kTiles) * 16 + lg * 4;
+        float* at = out + (j / kTiles) * plane + int64_t(m) * p.n + n;
+        if (m >= p.m || n >= p.n) continue;
+        if ((p.n & 3) == 0) {
+          *reinterpret_cast<f32x4*>(at) = acc[i][j];
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < p.n) at[e] = acc[i][j][e];
+        }
+      }
+    }
+    return;
+  }
   __syncthreads();
 
   float* scales = reinterpret_cast<float*>(lds + kStaged);
@@ -289,6 +317,65 @@ __global__ __launch_bounds__(kTileThreads) void gemm_kernel(const T* __restrict_
   gemm_tile<T, BM, BN, tile_stages(BM, BN), kLayout, true, Variant::kPlain>(A, B, B, C, p);
 }
 
+// Split K. A problem of few 64 x 64 tiles and a long K leaves most CUs idle while one workgroup
+// walks K, and a CU pulls ~30 GB/s whatever its ring holds (deeper rings, two K tiles per barrier
+// and nt loads changed nothing). Its K is cut into runs of whole K tiles, one workgroup each,
+// whose float32 sums the second kernel adds in order of K and rounds as the unsplit epilogues
+// do. bf16, unsplit -> split, both kernels: 64x4096x14336 84.6 -> 31.9 us (4 runs, 117 MB: 3.8
+// TB/s), 16x2048x8192 37.1 -> 14.4 (8), 16x6144x4096 22.7 -> 16.7 (2), 16x512x8192 27.4 -> 10.6
+// (8), SwiGLU 64x2048x8192 75.5 -> 25.8 (8). The wide tiles stay unsplit: SwiGLU 16x14336x4096
+// 45.8, 2 runs 53.6.
+template <typename T, int BM, int BN, Layout kLayout, Variant kVariant>
+__global__ __launch_bounds__(kTileThreads) void gemm_split_kernel(const T* __restrict__ A,
+                                                                  const T* __restrict__ B,
+                                                                  const T* __restrict__ B2,
+                                                                  Problem p) {
+  gemm_tile<T, BM, BN, tile_stages(BM, BN), kLayout, true, kVariant, true>(A, B, B2, nullptr, p);
+}
+
+// C from the partial sums: one thread per four columns, splits added in order.
+template <typename T, Variant kVariant>
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(T* __restrict__ C, Problem p, int splits) {
+  constexpr int kPlanes = kVariant == Variant::kSwiGLU ? 2 : 1;
+  const int groups = (p.n + 3) / 4;
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= int64_t(p.m) * groups) return;
+  const int m = int(i / groups), n = int(i % groups) * 4;
+  const int64_t plane = int64_t(p.m) * p.n;
+  const int count = min(4, p.n - n);
+  float sum[kPlanes][4];
+#pragma unroll
+  for (int h = 0; h < kPlanes; ++h) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sum[h][e] = 0.f;
+    const float* at = p.partial + h * plane + int64_t(m) * p.n + n;
+#pragma unroll 4
+    for (int s = 0; s < splits; ++s, at += kPlanes * plane) {
+      if ((p.n & 3) == 0) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(at);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[h][e] += v[e];
+      } else {
+        for (int e = 0; e < count; ++e) sum[h][e] += at[e];
+      }
+    }
+  }
+  const float scale = kVariant == Variant::kRowScale ? p.row_scale[m] : 1.f;
+  T* dst = C + m * p.scm + n * p.scn;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (e >= count) break;
+    T v;
+    if constexpr (kVariant == Variant::kSwiGLU)
+      v = swiglu_out<T>(sum[0][e], sum[1][e]);
+    else if constexpr (kVariant == Variant::kRowScale)
+      v = tk::from_f32<T>(sum[0][e] * scale);
+    else
+      v = tk::from_f32<T>(sum[0][e]);
+    dst[e * p.scn] = v;
+  }
+}
+
 template <typename T, int BM, int BN>
 void launch_one(Variant variant, const Plan& plan, const T* a, const T* b, const T* b2, T* c,
                 const Problem& p, hipStream_t stream) {
@@ -330,6 +417,39 @@ void launch_tile(int tile, Variant variant, const Plan& plan, const void* a, con
                  const void* b2, void* c, const Problem& p, hipStream_t stream) {
   launch_index<T, 1>(tile, variant, plan, static_cast<const T*>(a), static_cast<const T*>(b),
                      static_cast<const T*>(b2), static_cast<T*>(c), p, stream);
+}
+
+template <typename T>
+void launch_split(Variant variant, const Plan& plan, const void* a, const void* b, const void* b2,
+                  void* c, const Problem& p, int splits, hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n), static_cast<unsigned>(splits));
+  const dim3 block(kTileThreads);
+  const dim3 reduce(static_cast<unsigned>(cdiv(int64_t(p.m) * cdiv(p.n, 4), 256)));
+  const T* pa = static_cast<const T*>(a);
+  const T* pb = static_cast<const T*>(b);
+  const T* pb2 = static_cast<const T*>(b2);
+  T* pc = static_cast<T*>(c);
+  if (variant == Variant::kSwiGLU)
+    hipLaunchKernelGGL((gemm_split_kernel<T, 64, 128, Layout::NN, Variant::kSwiGLU>), grid, block,
+                       0, stream, pa, pb, pb2, p);
+  else if (plan.layout == Layout::NN)
+    hipLaunchKernelGGL((gemm_split_kernel<T, 64, 64, Layout::NN, Variant::kPlain>), grid, block, 0,
+                       stream, pa, pb, pb, p);
+  else if (plan.layout == Layout::NT)
+    hipLaunchKernelGGL((gemm_split_kernel<T, 64, 64, Layout::NT, Variant::kPlain>), grid, block, 0,
+                       stream, pa, pb, pb, p);
+  else
+    hipLaunchKernelGGL((gemm_split_kernel<T, 64, 64, Layout::TN, Variant::kPlain>), grid, block, 0,
+                       stream, pa, pb, pb, p);
+  if (variant == Variant::kSwiGLU)
+    hipLaunchKernelGGL((gemm_reduce_kernel<T, Variant::kSwiGLU>), reduce, dim3(256), 0, stream, pc,
+                       p, splits);
+  else if (variant == Variant::kRowScale)
+    hipLaunchKernelGGL((gemm_reduce_kernel<T, Variant::kRowScale>), reduce, dim3(256), 0, stream,
+                       pc, p, splits);
+  else
+    hipLaunchKernelGGL((gemm_reduce_kernel<T, Variant::kPlain>), reduce, dim3(256), 0, stream, pc,
+                       p, splits);
 }
 
 }  // namespace gemm_dma

@@ -51,6 +51,7 @@ _SIGNATURES: dict[str, list[object]] = {
     "tk_gemm": [_I32, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I32, _P],
     "tk_gemm_rowscale": [_I32, _P, _P, _P, _P] + [_I64] * 9 + [_P],
     "tk_scale_rows": [_I32, _P, _P, _P, _I64, _I64, _I64, _I64, _P],
+    "tk_gemm_splitk": [_I32, _P, _P, _P, _P, _P, _P] + [_I64] * 12 + [_P],
     "tk_gemm_swiglu": [
         _I32, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P,
     ],

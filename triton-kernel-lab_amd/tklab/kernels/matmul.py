@@ -11,7 +11,8 @@ reports it in the same metadata keys. Operands whose rows are 16-byte aligned an
 multiples of 8 elements long, each row-major or transposed, take buffer->LDS DMA
 kernels (tiles from 64 x 64 to 256 x 256 by problem size, eight wave64s,
 ``v_mfma_f32_16x16x32``): ``gemm_dma_kernel`` for row-major operands with K % 32 == 0 (every registry shape),
-``gemm_kernel`` for transposed ones (a linear layer's gradients) and other K.
+``gemm_kernel`` for transposed ones (a linear layer's gradients) and other K, and
+``gemm_split_kernel`` where few tiles meet a long K (:func:`split_k`).
 Every other layout takes the register-staged ``gemm_kernel`` (64 x 64 to 256 x 128).
 ``matmul_fp16acc`` keeps its registry entry, but gfx950 MFMA
 accumulates f16 products in float32 only, so both entry points run the same
@@ -77,6 +78,43 @@ def _pick_tile(m: int, n: int, k: int, tiles: tuple[tuple[int, int], ...] = _TIL
     return min(tiles, key=cost)
 
 
+def split_k(m: int, n: int, k: int) -> int:
+    """Runs of K for ``tk_gemm_splitk``; 1: one workgroup per output tile walks all of K.
+
+    A workgroup takes ~0.3 us per 64-wide K tile of a 64 x 64 tile; the second kernel and the
+    float32 sums take ~4 us of the device and ~5 of the host. One round of the 256 CUs and runs
+    of at least 16 K tiles were the best or within 8 % of it: 64x4096x14336 (64 tiles) 84.6 us
+    unsplit, 4 runs 31.9, 6 40.1, 8 35.3; 16x512x8192 (8 tiles) 27.4, 8 runs 10.6, 16 12.0. Past
+    128 tiles nothing is left to fill (256x4096x8192: 46.7, 2 runs 49.4). Below the least depth
+    a call is shorter than its host time: with the norm of a QKV projection 1x4096x4096 19.3
+    unsplit, 23.9 split, the product 8x512x3072 11.6 and 14.0; from 96 tiles HBM traffic moves
+    the line: 16x6144x4096 25.6 and 23.9, SwiGLU 8x8192x4096 38.6 and 33.0. The sizes alone
+    decide, so every layout and the fused variants add in the same order. Sums: at most 4 MiB
+    (8 MiB with SwiGLU).
+    """
+    tiles = -(-m // 64) * -(-n // 64)
+    depth = -(-k // 64)
+    if tiles > 128 or depth < (64 if tiles >= 96 else 80):
+        return 1
+    return min(256 // tiles, depth // 16)
+
+
+def enqueue_split(
+    a: torch.Tensor, b: torch.Tensor, out: torch.Tensor, splits: int, *, up: torch.Tensor | None = None,
+    row_scale: torch.Tensor | None = None,
+) -> None:
+    """``tk_gemm_splitk`` on checked operands: ``a @ b``, row-scaled, or SwiGLU with gate ``b``."""
+    (m, k), n = a.shape, b.shape[1]
+    # Float32 sums of the runs, on the stream the kernels run on.
+    sums = torch.empty(splits * m * n * (1 if up is None else 2), device=a.device, dtype=torch.float32)
+    _hip.call(
+        "tk_gemm_splitk", _hip.dtype_code(a.dtype), a.data_ptr(), b.data_ptr(),
+        None if up is None else up.data_ptr(), None if row_scale is None else row_scale.data_ptr(),
+        out.data_ptr(), sums.data_ptr(), m, n, k, splits, *a.stride(), *b.stride(),
+        *(b if up is None else up).stride(), *out.stride(), _hip.stream_of(a),
+    )
+
+
 def _tile_config(tile: tuple[int, int], *, staged: bool = False) -> dict[str, BenchmarkScalar]:
     """Metadata of a tile: K step 64 and a ring that fits the LDS, except the 256 x 256 kernel's."""
     if tile == _TILES[0]:
@@ -96,6 +134,8 @@ def launch_config(a: torch.Tensor, b: torch.Tensor) -> dict[str, BenchmarkScalar
     (m, k), n = a.shape, b.shape[1]
     mma = {"mma_opcode": _MFMA.get(a.dtype, _MFMA[torch.float16])}
     if (_dma_rows(a) or _dma_rows(a.t())) and (_dma_rows(b) or _dma_rows(b.t())):
+        if split_k(m, n, k) > 1:
+            return {**_tile_config((64, 64)), **mma, "hip_kernel": "gemm_split_kernel"}
         plain = _dma_rows(a) and _dma_rows(b) and k % 32 == 0
         swapped = not _dma_rows(a) and not _dma_rows(b)  # computed as C^T = B^T A^T
         tile = _pick_tile(n, m, k) if swapped else _pick_tile(m, n, k)
@@ -139,7 +179,7 @@ def _make_output(args: TensorArgs) -> torch.Tensor:
 
 
 def _launch_factory(*, fp16_accumulate: bool) -> LaunchFn:
-    """Allocation-free launcher for one accumulation mode."""
+    """Launcher for one accumulation mode: allocation-free but for the sums of a split K."""
 
     def launch(args: TensorArgs, output: torch.Tensor) -> None:
         a, b = args
@@ -158,6 +198,10 @@ def _launch_factory(*, fp16_accumulate: bool) -> LaunchFn:
 def _enqueue(a: torch.Tensor, b: torch.Tensor, output: torch.Tensor, *, fp16_accumulate: bool) -> None:
     """``output = a @ b`` for operands and an output already checked."""
     m, k = a.shape
+    splits = split_k(m, b.shape[1], k)
+    if splits > 1:
+        enqueue_split(a, b, output, splits)
+        return
     _hip.call(
         "tk_gemm", _hip.dtype_code(a.dtype), a.data_ptr(), b.data_ptr(), output.data_ptr(), m,
         b.shape[1], k, *a.stride(), *b.stride(), *output.stride(), int(fp16_accumulate),

@@ -70,6 +70,10 @@ def _launch(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, out: torc
         return
     m, k = x.shape
     n = w_gate.shape[1]
+    splits = matmul.split_k(m, n, k)
+    if splits > 1:
+        matmul.enqueue_split(x, w_gate, out, splits, up=w_up)
+        return
     _hip.call(
         "tk_gemm_swiglu",
         _hip.dtype_code(x.dtype),

@@ -141,6 +141,10 @@ def _run(
         eps,
         stream,
     )
+    splits = matmul.split_k(m, n, k)
+    if splits > 1:
+        matmul.enqueue_split(a, folded_weight, out, splits, row_scale=rstd)
+        return s, out
     _hip.call(
         "tk_gemm_rowscale",
         _hip.dtype_code(x.dtype),
