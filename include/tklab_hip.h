@@ -239,6 +239,13 @@ int tk_attn_fwd(int dtype, const void* q, const void* k, const void* v, void* o,
                 const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
                 const int64_t* o_strides, float sm_scale, int causal, void* stream);
 
+/* Query rows per workgroup (64, 128 or 256) of the forward kernel that tk_attn_fwd, _gqa and _rope
+ * (total = 0) and _varlen (seq the longest length, total the packed tokens) launch for heads whose
+ * rows span less than 2 GiB; 0 for sizes they reject. Every choice gives the same bits. A query:
+ * it launches nothing, needs no GPU and sets no error. */
+int tk_attn_fwd_rows(int64_t batch, int64_t heads, int64_t kv_heads, int64_t seq, int64_t head_dim,
+                     int64_t total, int causal);
+
 /* Attention backward preprocess: delta[b][h][i] = sum_d o[i][d] * do[i][d] (float32).
  * o and do share `strides` (batch, head, seq).
  * Replaces `_attn_bwd_preprocess_kernel[...]`, src/tklab/kernels/flash_attention.py:560-569. */

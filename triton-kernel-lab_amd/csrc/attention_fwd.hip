@@ -1057,26 +1057,68 @@ attn_fwd_small_kernel(FwdArgs<T> args) {
   }
 }
 
-// Query tiles per wave of the small-workgroup kernel for a problem of `tiles` 64-query tiles, or 0
-// for the 256-query kernel. 256-query / QT 1 / QT 2 in us, bf16, one sequence of N for H heads:
-//   causal D64:  H16 N1024 (256 tiles) 23.3/12.0/16.8, H16 N4096 (1024) 77/52/57,
-//                H16 N8192 (2048) 244/174/160, H64 N8192 (8192) 635/700/587,
+// Workgroups of `rows` queries a launch has (`total` > 0: a packed batch, where the lengths are on
+// the device and this is an upper bound).
+int64_t fwd_tiles(int64_t batch, int64_t heads, int64_t seq, int64_t total, int64_t rows) {
+  return (total > 0 ? varlen_tiles(batch, total, seq, rows) : batch * tk::cdiv(seq, rows)) * heads;
+}
+
+// What 256-query tiles cost a packed batch over 128-query ones: (query, key) pairs of the whole
+// blocks a sequence needs (causal: up to each tile's last query). Sequences of one length have it
+// exactly; others count half a tile of padding on the mean length.
+double packed_cost_of_256(int64_t batch, int64_t seq, int64_t total, bool causal) {
+  auto cost = [&](double rows) {
+    const double queries = total == batch * seq ? rows * double(tk::cdiv(seq, int64_t(rows)))
+                                                : double(total) / double(batch) + rows / 2;
+    return causal ? queries * (queries + rows) : queries;
+  };
+  return cost(256) / cost(128);
+}
+
+// Query tiles per wave of the small-workgroup kernel, or 0 for the 256-query kernel. A problem
+// has `tiles` 64-query tiles. 256-query / QT 1 / QT 2 in us, bf16, one sequence of N for H heads:
+//   causal D64:  H16 N1024 (256 tiles) 23.2/11.6/16.6, H16 N4096 (1024) 75/49/55,
+//                H16 N8192 (2048) 245/173/158, H64 N8192 (8192) 635/700/587,
 //                H128 N8192 (16384) 1176/-/1211
-//   causal D128: H32 N1024 (512) 40.7/19.0/24.0, H8 N8192 (1024) 180/167/157,
+//   causal D128: H32 N1024 (512) 39.6/17.3/22.0, H8 N8192 (1024) 180/167/158,
 //                H256 N512 (2048) 39.9/39.8/34.1, H64 N2048 (2048) 67.9/87.8/74.1
-//   full D64:    H32 N1024 (512) 23.6/16.2/18.3, H64 N1024 (1024) 25.1/27.4/26.3
-//   full D128:   H4 N8192 (512) 179/165/147, H64 N1024 (1024) 33.4/46.8/37.4
-//   varlen D128, H32: causal 15 sequences in 12000 tokens 185/187/168, 32 in 12000 150/138/111,
-//                3 in 12000 (to 6000) 523/717/543; full 15 in 12000 257/321/241, 4 in 8000
-//                348/452/377
-int small_query_tiles(int64_t tiles, int64_t seq, int64_t head_dim, bool causal, bool varlen) {
-  if (tiles <= 512) return 1;
-  if (causal && head_dim == 64) return tiles <= 1024 ? 1 : tiles <= 8192 ? 2 : 0;
-  if (causal) {
-    const bool fits = tiles <= 1024 || (tiles <= 2048 && seq <= 1024);
-    return fits || (varlen && seq <= 4096) ? 2 : 0;
+//   full D64:    H32 N1024 (512) 22.9/14.8/17.3, H64 N1024 (1024) 25.1/27.4/26.3
+//   full D128:   H16 N1024 (256) 27.5/15.8/21.5, H7 N2048 (224) 47/27/38, H48 N512 (384)
+//                17.6/13.0/13.4, H28 N1024 (448) 27.5/22.3/22.1, H14 N2048 (448) 47.6/40.1/38.5,
+//                H4 N8192 (512) 168/155/138, H64 N1024 (1024) 32.5/45.0/35.9
+// Packed batches: the small workgroups save padding and, with the chip full, read K and V from the
+// caches twice as often. Query heads that share a KV head (`group` of them) share those reads.
+// 256-query / QT 2 in us, H query heads over G KV heads, with packed_cost_of_256:
+//   causal D128 H32 G8:  15 sequences in 12000 (1.28) 185/168, 32 x 1000 (1.11) 401/384,
+//                        16 x 2048 (1.06) 613/633, 8 x 4096 (1.03) 1014/1095
+//   causal D128 H16 G16: 60 of 400 .. 1500 (1.28) 377/357, 40 x 768 (1.14) 190/198, 32 x 1000
+//                        222/247; H32 G32: 60 of 400 .. 1500 766/889, 40 x 768 413/473,
+//                        100 x 300 (1.67) 372/292; few tiles: H8 G8 15 of 300 .. 2000 63/53
+//   causal D64  H16 G16: 15 of 300 .. 2000 (1.25) 65/59, 40 x 700 (1.14) 86/96; H8 G8 64 x 1024
+//                        (1.11) 111/121; H32 G8 50 x 640 (1.33) 187/154
+//   full D128   H32 G8:  100 of 100 .. 1000 (1.13) 656/623, 15 to 1779 (1.13) 128/135, 40 x 768
+//                        (1.00) 435/445; H32 G32 40 x 768 520/718, 100 x 256 268/289; H16 G16
+//                        100 x 256 135/127
+int small_query_tiles(int64_t batch, int64_t heads, int64_t kv_heads, int64_t seq, int64_t head_dim,
+                      int64_t total, bool causal) {
+  const int64_t tiles = fwd_tiles(batch, heads, seq, total, 64);
+  const bool packed = total > 0, wide = head_dim == 128;
+  if (tiles <= 512) return wide && !causal && seq >= 1024 && tiles > 384 ? 2 : 1;
+  if (causal && !wide && tiles <= 1024) return 1;
+  if (causal && wide && tiles <= 1024) return 2;
+  if (!packed) {
+    if (!causal) return 0;
+    return wide ? (tiles <= 2048 && seq <= 1024 ? 2 : 0) : (tiles <= 8192 ? 2 : 0);
   }
-  return varlen && head_dim == 128 && seq <= 2048 ? 2 : 0;
+  const bool grouped = heads >= 4 * kv_heads, few_kv = kv_heads <= 16;
+  const double cost = packed_cost_of_256(batch, seq, total, causal);
+  if (causal) {
+    if (wide ? tiles <= 2304 && seq <= 2048 : tiles <= 3072) return 2;
+    return cost >= (grouped ? 1.1 : few_kv ? 1.22 : 1.28) ? 2 : 0;
+  }
+  if (!wide) return 0;
+  if (seq <= 256 && few_kv) return 2;
+  return cost >= (grouped && seq <= 1024 ? 1.12 : 1.22) ? 2 : 0;
 }
 
 // Causal head_dim 128, equal lengths: `items` workgroups (paired_items); otherwise one
@@ -1093,7 +1135,7 @@ void launch(int small, bool causal, int64_t items, hipStream_t st, const void* q
       hipLaunchKernelGGL((attn_fwd_small_kernel<T, D, 2, true>), grid, block, 0, st, a);
     else if (small == 1)
       hipLaunchKernelGGL((attn_fwd_small_kernel<T, D, 1, false>), grid, block, 0, st, a);
-    else
+    else if constexpr (D == 128)  // small_query_tiles gives head_dim 64 no other
       hipLaunchKernelGGL((attn_fwd_small_kernel<T, D, 2, false>), grid, block, 0, st, a);
     return;
   }
@@ -1146,14 +1188,11 @@ void attn_fwd_dma_launch(int dtype, const void* q, const void* k, const void* v,
   }
   s.scale_log2 = sm_scale * 1.4426950408889634f;
   s.batch = (int)batch;
-  auto tiles_of = [&](int64_t rows) {
-    return (cu_seqlens != nullptr ? varlen_tiles(batch, total, seq, rows) : batch * cdiv(seq, rows)) *
-           heads;
-  };
-  const int small = small_query_tiles(tiles_of(64), seq, head_dim, causal, cu_seqlens != nullptr);
+  const int64_t packed = cu_seqlens != nullptr ? total : 0;
+  const int small = small_query_tiles(batch, heads, kv_heads, seq, head_dim, packed, causal);
   const int64_t rows = small ? 64 * small : 256;
   s.q_blocks = (int)cdiv(seq, rows);
-  s.tiles = (int)tiles_of(rows);
+  s.tiles = (int)fwd_tiles(batch, heads, seq, packed, rows);
   s.k_bytes = (uint32_t)head_extent_bytes(seq, head_dim, k_strides[2]);
   s.v_bytes = (uint32_t)head_extent_bytes(seq, head_dim, v_strides[2]);
   const int64_t items = cu_seqlens == nullptr ? paired_items(batch * heads, s.q_blocks)
@@ -1168,3 +1207,12 @@ void attn_fwd_dma_launch(int dtype, const void* q, const void* k, const void* v,
 }
 
 }  // namespace tk
+
+extern "C" int tk_attn_fwd_rows(int64_t batch, int64_t heads, int64_t kv_heads, int64_t seq,
+                                int64_t head_dim, int64_t total, int causal) {
+  if (batch <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || heads <= 0 || seq <= 0 || total < 0 ||
+      (head_dim != 64 && head_dim != 128))
+    return 0;
+  const int small = small_query_tiles(batch, heads, kv_heads, seq, head_dim, total, causal != 0);
+  return small ? 64 * small : 256;
+}

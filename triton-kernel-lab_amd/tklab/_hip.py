@@ -110,7 +110,12 @@ _SIGNATURES: dict[str, list[object]] = {
     "tk_roof_mfma": [_I32, _P, _I64, _I64, _P],
 }
 
-EXPORTED_SYMBOLS: tuple[str, ...] = ("tk_abi_version", "tk_last_error", *_SIGNATURES)
+# Queries: their int result is an answer, not a status.
+_QUERIES: dict[str, list[object]] = {
+    "tk_attn_fwd_rows": [_I64, _I64, _I64, _I64, _I64, _I64, _I32],
+}
+
+EXPORTED_SYMBOLS: tuple[str, ...] = ("tk_abi_version", "tk_last_error", *_QUERIES, *_SIGNATURES)
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
@@ -142,6 +147,9 @@ def load_library(path: Path | None = None) -> ctypes.CDLL:
         version = lib.tk_abi_version()
         if version != ABI_VERSION:
             raise HipLibraryError(f"{target} has ABI {version}, expected {ABI_VERSION}")
+        for name, argtypes in _QUERIES.items():
+            query_fn = getattr(lib, name)
+            query_fn.restype, query_fn.argtypes = ctypes.c_int, argtypes
         if path is None:
             _lib = lib
         return lib
@@ -197,3 +205,8 @@ def call(name: str, *args: object) -> None:
     if status != 0:
         message = load_library().tk_last_error().decode(errors="replace")
         raise HipLibraryError(f"{name} failed: {message}")
+
+
+def query(name: str, *args: int) -> int:
+    """The answer of a query entry point (:data:`_QUERIES`); needs no GPU."""
+    return getattr(load_library(), name)(*args)
