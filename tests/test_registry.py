@@ -109,7 +109,7 @@ def test_every_registered_spec_prices_its_sizes() -> None:
 
 
 def test_launch_metadata_names_the_kernels_that_launch() -> None:
-    """The GEMM/attention metadata describe the DMA kernels every registry shape takes."""
+    """The GEMM/attention metadata describe the kernels the registry shapes take."""
     import torch
 
     from tklab.kernels import flash_attention, matmul
@@ -118,14 +118,25 @@ def test_launch_metadata_names_the_kernels_that_launch() -> None:
     assert gemm["hip_kernel"] == "gemm_dma_kernel"
     assert (gemm["block_k"], gemm["num_warps"], gemm["num_stages"]) == (32, 8, 4)
     assert gemm["mma_opcode"] == "v_mfma_f32_16x16x32_f16"
-    attn = REGISTRY["attention_causal"].benchmark_metadata(1024, torch.float16)
-    assert attn["hip_kernel"] == "attn_fwd_dma_kernel"
-    assert (attn["block_m"], attn["block_n"], attn["num_warps"]) == (256, 64, 8)
-    assert attn["mma_opcode"] == "v_mfma_f32_16x16x32_f16"
+    # (block_m, waves, stages) at 512 .. 8192: four waves of 16 or 32 queries until eight of 32 fill
+    # the chip, which full attention does at half the sequence length.
+    small, wide, full = (64, 4, 3), (128, 4, 3), (256, 8, 4)
+    for name, tiles in (("attention_causal", (small, small, small, small, wide)),
+                        ("attention_noncausal", (small, small, small, full, full))):
+        spec = REGISTRY[name]
+        assert tuple(spec.sizes) == (512, 1024, 2048, 4096, 8192)
+        for size, (rows, waves, stages) in zip(spec.sizes, tiles):
+            attn = spec.benchmark_metadata(size, torch.float16)
+            kernel = "attn_fwd_dma_kernel" if rows == 256 else "attn_fwd_small_kernel"
+            assert attn["hip_kernel"] == kernel
+            assert (attn["block_m"], attn["num_warps"], attn["num_stages"]) == (rows, waves, stages)
+            assert (attn["block_n"], attn["mma_opcode"]) == (64, "v_mfma_f32_16x16x32_f16")
     a = torch.empty(64, 96, dtype=torch.bfloat16)
     b = torch.empty(96, 64, dtype=torch.bfloat16)
     assert matmul.launch_config(a, b)["hip_kernel"] == "gemm_dma_kernel"
     assert matmul.launch_config(a, b)["mma_opcode"] == "v_mfma_f32_16x16x32_bf16"
     assert matmul.launch_config(a[:, :80], b[:80])["hip_kernel"] == "gemm_kernel"
     assert matmul.launch_config(a, b.t().contiguous().t())["hip_kernel"] == "gemm_kernel"
-    assert flash_attention.FORWARD_TILE["num_stages"] == 4
+    assert flash_attention.forward_tile(4, 32, 32, 8192, 128, causal=True) == flash_attention.FORWARD_TILE
+    packed = flash_attention.forward_tile(100, 32, 8, 300, 128, causal=True, total=30000)
+    assert (packed["block_m"], packed["num_stages"]) == (128, 2)

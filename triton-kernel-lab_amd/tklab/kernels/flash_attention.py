@@ -52,17 +52,29 @@ _HEAD_DIMS = (64, 128)
 _DTYPES = (torch.float16, torch.bfloat16)
 _LOG2_E = 1.4426950408889634
 
-# Tile configuration of csrc/attention.hip (forward / backward).
-# csrc/attention_fwd.hip (Geo<D>: BM, BN, WAVES, STAGES; problems that cannot fill the chip with these
-# take 64 queries per workgroup, SmallGeo<D>, with the same results): 256 queries per workgroup as eight
-# wave64s of 32, key blocks of 64, a 4-stage buffer->LDS K/V ring, v_mfma_f32_16x16x32.
-# "num_warps" counts wave64s.
+# Tile configurations of the kernels ("num_warps" counts wave64s), key blocks of 64 and
+# v_mfma_f32_16x16x32 throughout.
+# csrc/attention_fwd.hip (Geo<D>: BM, BN, WAVES, STAGES): 256 queries per workgroup as eight waves of 32,
+# a 4-stage buffer->LDS K/V ring. Problems that cannot fill the chip with these take four waves of 16 or
+# 32 queries (SmallGeo<D, QT>), with the same results; forward_tile() says which a problem takes.
 FORWARD_TILE = {"hip_kernel": "attn_fwd_dma_kernel", "block_m": 256, "block_n": 64, "num_warps": 8,
                 "num_stages": 4}
+_SMALL_STAGES = {64: 3, 128: 2}
 FORWARD_MFMA = {torch.float16: "v_mfma_f32_16x16x32_f16", torch.bfloat16: "v_mfma_f32_16x16x32_bf16"}
 # Backward (csrc/attention_bwd.hip, attention_bwd_dq.hip): dK/dV owns 128 keys per workgroup
 # over query blocks of 64; dQ owns 256 queries over key blocks of 64.
 BACKWARD_TILE = {"block_m": 128, "block_n": 64}
+
+
+def forward_tile(
+    batch: int, heads: int, kv_heads: int, seq: int, head_dim: int, *, causal: bool, total: int = 0
+) -> dict[str, BenchmarkScalar]:
+    """Tile configuration of the forward kernel a problem launches (``total``: packed tokens)."""
+    rows = _hip.query("tk_attn_fwd_rows", batch, heads, kv_heads, seq, head_dim, total, int(causal))
+    if rows == FORWARD_TILE["block_m"]:
+        return dict(FORWARD_TILE)
+    return {**FORWARD_TILE, "hip_kernel": "attn_fwd_small_kernel", "block_m": rows, "num_warps": 4,
+            "num_stages": _SMALL_STAGES[head_dim]}
 
 
 def _validate(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
@@ -697,8 +709,9 @@ def _flops_factory(*, causal: bool) -> CostFn:
 def _metadata_factory(*, causal: bool) -> BenchmarkMetadataFn:
     """Tile configuration and problem constants in the reference's keys."""
 
-    def metadata(_size: int, dtype: torch.dtype) -> dict[str, BenchmarkScalar]:
-        return {**FORWARD_TILE, "heads": _HEADS, "head_dim": _HEAD_DIM, "causal": causal,
+    def metadata(size: int, dtype: torch.dtype) -> dict[str, BenchmarkScalar]:
+        tile = forward_tile(_BATCH, _HEADS, _HEADS, size, _HEAD_DIM, causal=causal)
+        return {**tile, "heads": _HEADS, "head_dim": _HEAD_DIM, "causal": causal,
                 "mma_opcode": FORWARD_MFMA.get(dtype, FORWARD_MFMA[torch.float16])}
 
     return metadata
