@@ -41,18 +41,31 @@ __global__ __launch_bounds__(RT >= kNormBlock ? RT : kNormBlock) void rmsnorm_fw
   // 16-byte rows go through buffer accesses with per-stream cache policies: the
   // inputs are streamed (non-temporal), the outputs stored with sc1.
   constexpr bool kBuf = ACCESS == tk::Access::kAligned, kAny = ACCESS == tk::Access::kAny;
+  // Waves leave out vectors past their row's end where a row can have whole ones: bf16 forward of
+  // 4.9k x 8193 45 -> 34 us, 9.8k x 4097 99 -> 54, 20k x 2001 43 -> 29 (one element per access 38,
+  // 59 and 36); f32 9.8k x 4097 77 -> 61.
+  constexpr bool kSkip = kAny && (RT > 64 || sizeof(T) == 4);
   const int lane = threadIdx.x % RT;
   // A wave's threads share one row (RT >= 64); readfirstlane makes that visible to
   // the compiler, so the row's buffer resource lives in scalar registers.
   const int row = __builtin_amdgcn_readfirstlane(blockIdx.x * SLOTS + threadIdx.x / RT);
   if (row >= rows) return;  // SLOTS > 1 only for barrier-free single-wave rows
 
+  // f of every element but those of vectors past the row (kSkip).
+  auto each = [&](auto&& f) {
+#pragma unroll
+    for (int i = 0; i < VALS / VEC; ++i) {
+      if (kSkip && tk::vector_span<VEC, RT, true>(i, lane).begin >= cols) continue;
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) f(i * VEC + j);
+    }
+  };
   // s is kept in the storage type: with a residual it is rounded there anyway.
   Row sv;
   if constexpr (kBuf)
     sv.template load_buf<tk::kCpolStream>(x + row * x_stride, cols, lane);
   else if constexpr (kAny)
-    sv.load_any(x + row * x_stride, cols, lane);
+    sv.template load_any<kSkip>(x + row * x_stride, cols, lane);
   else
     sv.load(x + row * x_stride, cols, lane);
   if (residual != nullptr) {
@@ -60,28 +73,26 @@ __global__ __launch_bounds__(RT >= kNormBlock ? RT : kNormBlock) void rmsnorm_fw
     if constexpr (kBuf)
       rv.template load_buf<tk::kCpolStream>(residual + row * r_stride, cols, lane);
     else if constexpr (kAny)
-      rv.load_any(residual + row * r_stride, cols, lane);
+      rv.template load_any<kSkip>(residual + row * r_stride, cols, lane);
     else
       rv.load(residual + row * r_stride, cols, lane);
-    if constexpr (kAny) rv.fix_any(cols, lane);
-    if constexpr (kAny) sv.fix_any(cols, lane);
-#pragma unroll
-    for (int e = 0; e < VALS; ++e) sv.set(e, sv.get(e) + rv.get(e));
+    if constexpr (kAny) rv.template fix_any<kSkip>(cols, lane);
+    if constexpr (kAny) sv.template fix_any<kSkip>(cols, lane);
+    each([&](int e) { sv.set(e, sv.get(e) + rv.get(e)); });
     if (residual_sum != nullptr) {
       if constexpr (kBuf)
         sv.template store_buf<tk::kCpolSc1>(residual_sum + row * s_stride, cols, lane);
       else if constexpr (kAny)
-        sv.store_any(residual_sum + row * s_stride, cols, lane);
+        sv.template store_any<kSkip>(residual_sum + row * s_stride, cols, lane);
       else
         sv.store(residual_sum + row * s_stride, cols, lane);
     }
   } else if constexpr (kAny) {
-    sv.fix_any(cols, lane);
+    sv.template fix_any<kSkip>(cols, lane);
   }
 
   float ss = 0.f;
-#pragma unroll
-  for (int e = 0; e < VALS; ++e) ss += sv.get(e) * sv.get(e);
+  each([&](int e) { ss += sv.get(e) * sv.get(e); });
   ss = tk::group_allreduce<RT>(ss, tk::SumOp{}, scratch);
   const float rstd = 1.0f / sqrtf(ss / static_cast<float>(cols) + eps);
 
@@ -90,17 +101,16 @@ __global__ __launch_bounds__(RT >= kNormBlock ? RT : kNormBlock) void rmsnorm_fw
   if (y != nullptr) {
     Row wv;
     if constexpr (kAny) {
-      wv.load_any(weight, cols, lane);
-      wv.fix_any(cols, lane);
+      wv.template load_any<kSkip>(weight, cols, lane);
+      wv.template fix_any<kSkip>(cols, lane);
     } else {
       wv.load(weight, cols, lane);
     }
-#pragma unroll
-    for (int e = 0; e < VALS; ++e) wv.set(e, sv.get(e) * rstd * wv.get(e));
+    each([&](int e) { wv.set(e, sv.get(e) * rstd * wv.get(e)); });
     if constexpr (kBuf)
       wv.template store_buf<tk::kCpolSc1>(y + row * y_stride, cols, lane);
     else if constexpr (kAny)
-      wv.store_any(y + row * y_stride, cols, lane);
+      wv.template store_any<kSkip>(y + row * y_stride, cols, lane);
     else
       wv.store(y + row * y_stride, cols, lane);
   }
@@ -148,12 +158,12 @@ __device__ __forceinline__ void load_rowset_buf(RowSet<Row>& s, const RowPtrs<T>
 
 // The same at any element boundary (rows are clamped to the group's last one instead of read with
 // no extent); stage1_row puts the elements in place.
-template <typename T, typename Row>
+template <typename T, bool SKIP, typename Row>
 __device__ __forceinline__ void load_rowset_any(RowSet<Row>& s, const RowPtrs<T>& p, int64_t row,
                                                 int cols, int lane, const float* rstd) {
-  s.x.load_any(p.x + row * p.xs, cols, lane);
-  s.dy.load_any(p.dy + row * p.dys, cols, lane);
-  if (p.inc != nullptr) s.inc.load_any(p.inc + row * p.incs, cols, lane);
+  s.x.template load_any<SKIP>(p.x + row * p.xs, cols, lane);
+  s.dy.template load_any<SKIP>(p.dy + row * p.dys, cols, lane);
+  if (p.inc != nullptr) s.inc.template load_any<SKIP>(p.inc + row * p.incs, cols, lane);
   s.r = rstd[row];
 }
 
@@ -164,10 +174,13 @@ template <typename T, int VEC, tk::Access ACCESS, int RT, int VALS, bool ACC_LDS
 __device__ __forceinline__ void stage1_row(RowSet<Row>& s, const Row& wv, const RowPtrs<T>& p,
                                            int64_t row, int cols, int lane, float* acc,
                                            float* fold, float* scratch) {
+  // As in the forward, for float32 rows: 9.8k x 4097 137 -> 109 us. In 16 bits the branches cost the
+  // software pipeline more than they save (bf16 40k x 1001 52 -> 57 us).
+  constexpr bool kSkip = ACCESS == tk::Access::kAny && sizeof(T) == 4 && RT > 64;
   if constexpr (ACCESS == tk::Access::kAny) {
-    s.x.fix_any(cols, lane);
-    s.dy.fix_any(cols, lane);
-    if (p.inc != nullptr) s.inc.fix_any(cols, lane);
+    s.x.template fix_any<kSkip>(cols, lane);
+    s.dy.template fix_any<kSkip>(cols, lane);
+    if (p.inc != nullptr) s.inc.template fix_any<kSkip>(cols, lane);
   }
   float dot = 0.f;
 #pragma unroll
@@ -193,7 +206,7 @@ __device__ __forceinline__ void stage1_row(RowSet<Row>& s, const Row& wv, const 
   if constexpr (ACCESS == tk::Access::kAligned)
     s.x.template store_buf<tk::kCpolStream>(p.dx + row * p.dxs, cols, lane);
   else if constexpr (ACCESS == tk::Access::kAny)
-    s.x.store_any(p.dx + row * p.dxs, cols, lane);
+    s.x.template store_any<kSkip>(p.dx + row * p.dxs, cols, lane);
   else
     s.x.store(p.dx + row * p.dxs, cols, lane);
 }
@@ -248,8 +261,8 @@ __global__ __launch_bounds__(bwd_block<RT>()) void rmsnorm_bwd_stage1_kernel(
   constexpr bool kAny = ACCESS == tk::Access::kAny;
   Row wv;
   if constexpr (kAny) {
-    wv.load_any(weight, cols, lane);
-    wv.fix_any(cols, lane);
+    wv.template load_any<false>(weight, cols, lane);
+    wv.template fix_any<false>(cols, lane);
   } else {
     wv.load(weight, cols, lane);
   }
@@ -270,7 +283,7 @@ __global__ __launch_bounds__(bwd_block<RT>()) void rmsnorm_bwd_stage1_kernel(
     auto extent = [&](int k) { return kAny || k < group_rows ? cols : 0; };
     auto load = [&](RowSet<Row>& s, int k) {
       if constexpr (kAny)
-        load_rowset_any<T>(s, ptr, rowk(k), extent(k), lane, rstd);
+        load_rowset_any<T, false>(s, ptr, rowk(k), extent(k), lane, rstd);
       else
         load_rowset_buf<T>(s, ptr, rowk(k), extent(k), lane, rstd);
     };
@@ -295,7 +308,7 @@ __global__ __launch_bounds__(bwd_block<RT>()) void rmsnorm_bwd_stage1_kernel(
     RowSet<Row> ra;
     for (int k = slot; k < group_rows; k += SLOTS) {
       if constexpr (kAny)
-        load_rowset_any<T>(ra, ptr, row_of(k), cols, lane, rstd);
+        load_rowset_any<T, sizeof(T) == 4>(ra, ptr, row_of(k), cols, lane, rstd);
       else
         load_rowset<T>(ra, ptr, row_of(k), cols, lane, rstd);
       stage1_row<T, VEC, ACCESS, RT, VALS, ACC_LDS>(ra, wv, ptr, row_of(k), cols, lane, acc, fold, scratch);
@@ -404,6 +417,7 @@ extern "C" int tk_rmsnorm_fwd(int dtype, const void* x, const void* residual, co
   // bf16 16384 x 4096 residual forward one wave per row (64 values per thread) ran 93 us,
   // four waves per row 88 us. Rows wider than 1024 x 16 keep the wider shape.
   tk::pick_row_shape(cols, &shape, 16);
+  tk::narrow_row_shape(dtype, cols, access, &shape);
   const int slots = shape.rt >= kNormBlock ? 1 : kNormBlock / shape.rt;
   const dim3 grid(static_cast<unsigned>(tk::cdiv(rows, slots)));
   const dim3 block(shape.rt >= kNormBlock ? shape.rt : kNormBlock);
@@ -444,6 +458,7 @@ extern "C" int tk_rmsnorm_bwd_stage1(int dtype, void* dx, const void* dy, const 
   // most 64 bytes of each row tensor per thread (32 packed 16-bit or 16 float32 values)
   // keeps that in registers without spilling.
   tk::pick_row_shape(cols, &shape, 64 / tk::elem_size(dtype));
+  tk::narrow_row_shape(dtype, cols, access, &shape);
   const dim3 grid(static_cast<unsigned>(group_count));
   hipStream_t s = tk::as_stream(stream);
   int32_t* counts = locks + group_size;
@@ -549,6 +564,7 @@ extern "C" int tk_rmsnorm_bwd_noalloc(int dtype, void* dx, void* dw, const void*
   if (check_rows("rmsnorm_bwd_noalloc", dtype, rows, cols, &shape)) return 1;
   const tk::Access access = tk::row_access(dtype, cols, vector_ok);
   tk::pick_row_shape(cols, &shape, 64 / tk::elem_size(dtype));
+  tk::narrow_row_shape(dtype, cols, access, &shape);
   hipStream_t s = tk::as_stream(stream);
   float* partial = nullptr;
   if (scratch_address("rmsnorm_bwd_noalloc", s, &partial)) return 1;

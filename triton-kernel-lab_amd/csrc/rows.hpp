@@ -126,11 +126,28 @@ __device__ __forceinline__ u32x4 any_load(const T* row, int cols, int c) {
   static_assert(VEC * sizeof(T) == 16, "16-byte vectors only");
   return load_any(row + min(c, cols - VEC));
 }
-// `end`: one past the last column of the vectors the whole group loads together. It is uniform,
-// so the groups inside the row skip the work with a scalar branch.
-template <typename T, int VEC>
-__device__ __forceinline__ u32x4 any_fix(u32x4 v, int cols, int c, int end, uint32_t fill) {
-  if (end > cols) {
+// Columns of the vectors that a wave (WAVE) or the row's whole group loads together as its vector
+// i. They are uniform, so vectors inside the row skip the work with a scalar branch; waves also
+// skip the vectors past it (`end` of a wave: 4097 columns keep one of 16 waves busy with the row's
+// end instead of all).
+struct Span {
+  int begin, end;
+};
+template <int VEC, int RT, bool WAVE>
+__device__ __forceinline__ Span vector_span(int i, int lane) {
+  if constexpr (WAVE && RT > 64) {
+    const int begin = (i * RT + __builtin_amdgcn_readfirstlane(lane & ~63)) * VEC;
+    return {begin, begin + 64 * VEC};
+  }
+  return {i * RT * VEC, (i + 1) * RT * VEC};
+}
+template <typename T, int VEC, bool WAVE>
+__device__ __forceinline__ u32x4 any_fix(u32x4 v, int cols, int c, Span span, uint32_t fill) {
+  if (WAVE && span.begin >= cols) {
+    const uint32_t word = sizeof(T) == 4 ? fill : fill | (fill << 16);
+    return u32x4{word, word, word, word};
+  }
+  if (span.end > cols) {
     v = drop_elements<int(sizeof(T))>(v, min(max(c - (cols - VEC), 0), VEC - 1));
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
@@ -145,9 +162,10 @@ __device__ __forceinline__ u32x4 any_fix(u32x4 v, int cols, int c, int end, uint
   }
   return v;
 }
-template <typename T, int VEC>
-__device__ __forceinline__ void any_store(T* row, int cols, int c, int end, u32x4 v) {
-  if (end <= cols || c + VEC <= cols) {
+template <typename T, int VEC, bool WAVE>
+__device__ __forceinline__ void any_store(T* row, int cols, int c, Span span, u32x4 v) {
+  if (WAVE && span.begin >= cols) return;
+  if (span.end <= cols || c + VEC <= cols) {
     tk::store_any(row + c, v);
   } else {
     const Vec<T, VEC> e = __builtin_bit_cast(Vec<T, VEC>, v);
@@ -236,7 +254,8 @@ __device__ __forceinline__ void load_row_any(const T* row, int cols, int lane, f
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
     const Vec<T, VEC> r = __builtin_bit_cast(
-        Vec<T, VEC>, any_fix<T, VEC>(raw[i], cols, (i * RT + lane) * VEC, (i + 1) * RT * VEC, bits));
+        Vec<T, VEC>, any_fix<T, VEC, true>(raw[i], cols, (i * RT + lane) * VEC,
+                                           vector_span<VEC, RT, true>(i, lane), bits));
 #pragma unroll
     for (int j = 0; j < VEC; ++j) v[i * VEC + j] = to_f32(r.v[j]);
   }
@@ -250,8 +269,8 @@ __device__ __forceinline__ void store_row_any(T* row, int cols, int lane, const 
     Vec<T, VEC> r;
 #pragma unroll
     for (int j = 0; j < VEC; ++j) r.v[j] = from_f32<T>(v[i * VEC + j]);
-    any_store<T, VEC>(row, cols, (i * RT + lane) * VEC, (i + 1) * RT * VEC,
-                      __builtin_bit_cast(u32x4, r));
+    any_store<T, VEC, true>(row, cols, (i * RT + lane) * VEC, vector_span<VEC, RT, true>(i, lane),
+                            __builtin_bit_cast(u32x4, r));
   }
 }
 
@@ -345,28 +364,35 @@ struct RawRow {
 
   // 16-byte variants at any element boundary: load_any issues the loads (of any row with at
   // least VEC columns), fix_any puts the elements in place and zeroes what lies past the row.
+  // SKIP: waves load no vectors past the row (a branch around each load, which costs a software
+  // pipeline more than it saves).
+  template <bool SKIP>
   __device__ __forceinline__ void load_any(const T* row, int cols, int lane) {
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
-      const u32x4 u = any_load<T, VEC>(row, cols, (i * RT + lane) * VEC);
+      u32x4 u = {0u, 0u, 0u, 0u};
+      if (!SKIP || vector_span<VEC, RT, true>(i, lane).begin < cols)
+        u = any_load<T, VEC>(row, cols, (i * RT + lane) * VEC);
 #pragma unroll
       for (int j = 0; j < 4; ++j) w[i * 4 + j] = u[j];
     }
   }
+  template <bool WAVE>
   __device__ __forceinline__ void fix_any(int cols, int lane) {
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
       u32x4 u = {w[i * 4 + 0], w[i * 4 + 1], w[i * 4 + 2], w[i * 4 + 3]};
-      u = any_fix<T, VEC>(u, cols, (i * RT + lane) * VEC, (i + 1) * RT * VEC, 0u);
+      u = any_fix<T, VEC, WAVE>(u, cols, (i * RT + lane) * VEC, vector_span<VEC, RT, WAVE>(i, lane), 0u);
 #pragma unroll
       for (int j = 0; j < 4; ++j) w[i * 4 + j] = u[j];
     }
   }
+  template <bool WAVE>
   __device__ __forceinline__ void store_any(T* row, int cols, int lane) const {
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
       const u32x4 u = {w[i * 4 + 0], w[i * 4 + 1], w[i * 4 + 2], w[i * 4 + 3]};
-      any_store<T, VEC>(row, cols, (i * RT + lane) * VEC, (i + 1) * RT * VEC, u);
+      any_store<T, VEC, WAVE>(row, cols, (i * RT + lane) * VEC, vector_span<VEC, RT, WAVE>(i, lane), u);
     }
   }
 
@@ -436,6 +462,14 @@ inline Access row_access(int dtype, int64_t cols, bool aligned) {
                                           : Access::kScalar;
 }
 
+// Rows at any boundary that one vector per lane of a wave covers hold no more than that: with 16
+// values per lane, whose other vectors are past the row, bf16 1M x 9 ran the norm in 491 us (now 263, one
+// element per access 250), its backward in 1183 (692, 1575), softmax in 325 (189, 206).
+inline void narrow_row_shape(int dtype, int64_t cols, Access access, RowShape* shape) {
+  const int vec = 16 / elem_size(dtype);
+  if (access == Access::kAny && cols <= 64 * vec) *shape = {64, vec};
+}
+
 }  // namespace tk
 
 // Expands `__VA_ARGS__` with constexpr VEC and ACCESS bound to `access`.
@@ -464,7 +498,12 @@ inline Access row_access(int dtype, int64_t cols, bool aligned) {
   } else if ((access) == tk::Access::kAny) {                                 \
     constexpr tk::Access ACCESS = tk::Access::kAny;                          \
     constexpr int VEC = 16 / int(sizeof(T));                                 \
-    TK_DISPATCH_ROW_SHAPE(shape, __VA_ARGS__)                                \
+    if ((shape).vals < 16) {                                                 \
+      constexpr int RT = 64, VALS = VEC;                                     \
+      __VA_ARGS__;                                                           \
+    } else {                                                                 \
+      TK_DISPATCH_ROW_SHAPE(shape, __VA_ARGS__)                              \
+    }                                                                        \
   } else {                                                                   \
     constexpr tk::Access ACCESS = tk::Access::kAligned;                      \
     constexpr int VEC = 16 / int(sizeof(T));                                 \

@@ -437,6 +437,7 @@ extern "C" int tk_softmax_fwd(int dtype, const void* x, void* y, int64_t rows, i
   const bool vector_ok = tk::aligned16(x) && tk::aligned16(y) && cols % vec == 0 &&
                          (x_row_stride * es) % 16 == 0 && (y_row_stride * es) % 16 == 0;
   tk::Access access = tk::row_access(dtype, cols, vector_ok);
+  tk::narrow_row_shape(dtype, cols, access, &shape);
   // Rows of 1024 threads go through aligned vectors on shifted rows when every x row starts at
   // the same place between two 16-byte boundaries as its y row (contiguous tensors do): bf16
   // 2048 x 32001 58.7 us against 66.6 us with vectors at any boundary, 2048 x 50257 95 against
