@@ -56,3 +56,15 @@ def test_softmax_of_one_vector_per_lane(dtype, rows, cols) -> None:
     torch.testing.assert_close(softmax(x).double(), torch.softmax(x.double(), -1), rtol=2e-2, atol=1e-3,
                                equal_nan=True)
     assert_close(softmax(x)[3:], torch.softmax(x[3:].double(), -1))
+
+
+# A few columns short of a row shape of 1024 threads, where the shifted row would need the next one,
+# and where it just fits.
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("cols", [16377, 16381, 16383, 16385, 32761, 32765, 32767, 65529, 65533])
+def test_contiguous_softmax_at_the_end_of_a_row_shape(dtype, cols) -> None:
+    storage = torch.full((5 * cols + 8,), float("nan"), device="cuda", dtype=dtype)
+    x = storage[3:3 + 5 * cols].view(5, cols)
+    x.copy_(torch.randn(5, cols, device="cuda", generator=torch.Generator("cuda").manual_seed(cols)) * 3)
+    assert_close(softmax(x.contiguous().clone()), torch.softmax(x.double(), -1))
+    assert_close(softmax(x), torch.softmax(x.double(), -1))

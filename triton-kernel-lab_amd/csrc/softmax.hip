@@ -442,15 +442,15 @@ extern "C" int tk_softmax_fwd(int dtype, const void* x, void* y, int64_t rows, i
   // the same place between two 16-byte boundaries as its y row (contiguous tensors do): bf16
   // 2048 x 32001 58.7 us against 66.6 us with vectors at any boundary, 2048 x 50257 95 against
   // 120. Narrower rows pay more for the element stores at their ends: fp16 16384 x 1001 15.5
-  // against 12.0 us, f32 4096 x 4097 25.1 against 23.3.
+  // against 12.0 us, f32 4096 x 4097 25.1 against 23.3. Nor where the shift needs a wider row shape
+  // (rows a few columns short of one): bf16 2441 x 16383 51 against 27 us, f32 71 against 50.
   tk::RowShape shifted;
   if (access == tk::Access::kAny &&
       (reinterpret_cast<uintptr_t>(x) - reinterpret_cast<uintptr_t>(y)) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(x) % es == 0 && ((x_row_stride - y_row_stride) * es) % 16 == 0 &&
-      tk::pick_row_shape(cols + vec - 1, &shifted) && shifted.rt == 1024) {
+      tk::pick_row_shape(cols + vec - 1, &shifted) && shifted.rt == 1024 &&
+      shape.rt == shifted.rt && shape.vals == shifted.vals)
     access = tk::Access::kShift;
-    shape = shifted;
-  }
   // Two single-wave rows per wave once that still leaves two waves per SIMD (4096 rows).
   const bool pair = shape.rt == 64 && rows >= 4096;
   const dim3 grid(static_cast<unsigned>(tk::cdiv(rows, pair ? 2 : 1)));
