@@ -210,8 +210,9 @@ int tk_gemm_rowscale(int dtype, const void* a, const void* b, const float* row_s
  * tiles, 1 <= splits <= ceil(k / 64): one workgroup each for problems with too few output tiles
  * to fill the chip. `workspace` (float32, 16-byte aligned, splits * m * n values, twice that
  * with b_up) holds the runs' sums, which are added in order of K in float32 and rounded once, so
- * the result is deterministic; all three variants add in the same order. Operands the DMA
- * kernels do not take run as the unsplit entry points. No reference counterpart
+ * the result is deterministic; all three variants add in the same order, which is not that of
+ * the unsplit entry points (those sum K in one order for every size and layout). Operands the DMA
+ * kernels do not take run as the unsplit entry points and leave the workspace alone. No reference counterpart
  * (src/tklab/kernels/matmul.py:72-164 computes each tile in one program). */
 int tk_gemm_splitk(int dtype, const void* a, const void* b, const void* b_up,
                    const float* row_scale, void* c, float* workspace, int64_t m, int64_t n,

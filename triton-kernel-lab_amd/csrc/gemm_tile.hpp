@@ -18,7 +18,8 @@ constexpr Tile kTiles[] = {{256, 256}, {256, 128}, {128, 256}, {192, 192}, {128,
 constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
 
 // Index of the tile for a problem (0 of kTiles is the 256 x 256 kernel of gemm_dma.hip). Every
-// tile sums K in the same order, so the choice never changes a result.
+// tile sums K in the same order, so the choice of a tile never changes a result; splitting K
+// (launch_split) does.
 int pick_tile(const Tile* tiles, int count, int64_t m, int64_t n, int64_t k, Variant variant);
 
 // Enqueues the small-tile kernel `tile` (1 ..) for a problem whose tile counts are filled in.

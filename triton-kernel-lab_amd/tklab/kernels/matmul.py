@@ -56,16 +56,21 @@ _MFMA = {
 _STAGED_TILES = ((256, 128), (128, 128), (64, 64))
 
 
-def _dma_rows(t: torch.Tensor) -> bool:
+def _dma_rows(rows: int, cols: int, row_stride: int, col_stride: int) -> bool:
     """Rows the DMA kernels can load: unit inner stride, whole aligned 16-byte groups, < 2 GiB."""
-    rows, cols = t.shape
     return (
-        t.stride(1) == 1
-        and cols % 8 == 0
-        and t.stride(0) % 8 == 0
-        and t.data_ptr() % 16 == 0
-        and ((rows - 1) * t.stride(0) + cols) * 2 < 2**31
+        col_stride == 1
+        and not (cols | row_stride) & 7
+        and ((rows - 1) * row_stride + cols) * 2 < 2**31
     )
+
+
+def _dma_operand(rows: int, cols: int, row_stride: int, col_stride: int) -> bool:
+    """Layouts the DMA kernels take: stored by rows or by columns (``plan``, csrc/gemm_dma.hip).
+
+    The base must be 16-byte aligned too.
+    """
+    return _dma_rows(rows, cols, row_stride, col_stride) or _dma_rows(cols, rows, col_stride, row_stride)
 
 
 def _pick_tile(m: int, n: int, k: int, tiles: tuple[tuple[int, int], ...] = _TILES) -> tuple[int, int]:
@@ -88,9 +93,15 @@ def split_k(m: int, n: int, k: int) -> int:
     128 tiles nothing is left to fill (256x4096x8192: 46.7, 2 runs 49.4). Below the least depth
     a call is shorter than its host time: with the norm of a QKV projection 1x4096x4096 19.3
     unsplit, 23.9 split, the product 8x512x3072 11.6 and 14.0; from 96 tiles HBM traffic moves
-    the line: 16x6144x4096 25.6 and 23.9, SwiGLU 8x8192x4096 38.6 and 33.0. The sizes alone
-    decide, so every layout and the fused variants add in the same order. Sums: at most 4 MiB
+    the line: 16x6144x4096 25.6 and 23.9, SwiGLU 8x8192x4096 38.6 and 33.0. Sums: at most 4 MiB
     (8 MiB with SwiGLU).
+
+    The sizes decide, so that every layout the DMA kernels take and the fused variants add in the
+    same order. Two things follow for the bits of a result (its error does not grow). A row's bits
+    depend on M where K is split: 64x4096x14336 is summed in 4 runs, the same rows among 1024 in
+    one. And operands the DMA kernels do not take (odd strides, unaligned bases) are never split,
+    so they have the bits of the unsplit product. ``tk_gemm`` and the registry's launchers never
+    split: every tile and layout sums a row alike whatever M is.
     """
     tiles = -(-m // 64) * -(-n // 64)
     depth = -(-k // 64)
@@ -126,18 +137,20 @@ def _tile_config(tile: tuple[int, int], *, staged: bool = False) -> dict[str, Be
 
 
 def launch_config(a: torch.Tensor, b: torch.Tensor) -> dict[str, BenchmarkScalar]:
-    """Tile configuration and MFMA of the kernel ``tk_gemm`` launches for ``a @ b``.
+    """Tile configuration and MFMA of the kernel ``matmul_fp32acc`` launches for ``a @ b``.
 
     Mirrors ``gemm_dma::plan`` and ``pick_tile`` (csrc/gemm_dma.hip) and ``gemm_staged``
     (csrc/gemm.hip).
     """
     (m, k), n = a.shape, b.shape[1]
     mma = {"mma_opcode": _MFMA.get(a.dtype, _MFMA[torch.float16])}
-    if (_dma_rows(a) or _dma_rows(a.t())) and (_dma_rows(b) or _dma_rows(b.t())):
+    aligned = not (a.data_ptr() | b.data_ptr()) & 15
+    if aligned and all(_dma_operand(*t.shape, *t.stride()) for t in (a, b)):
         if split_k(m, n, k) > 1:
             return {**_tile_config((64, 64)), **mma, "hip_kernel": "gemm_split_kernel"}
-        plain = _dma_rows(a) and _dma_rows(b) and k % 32 == 0
-        swapped = not _dma_rows(a) and not _dma_rows(b)  # computed as C^T = B^T A^T
+        by_rows = [_dma_rows(*t.shape, *t.stride()) for t in (a, b)]
+        plain = all(by_rows) and k % 32 == 0
+        swapped = not any(by_rows)  # computed as C^T = B^T A^T
         tile = _pick_tile(n, m, k) if swapped else _pick_tile(m, n, k)
         return {**_tile_config(tile), **mma,
                 "hip_kernel": "gemm_dma_kernel" if plain else "gemm_kernel"}
@@ -179,7 +192,7 @@ def _make_output(args: TensorArgs) -> torch.Tensor:
 
 
 def _launch_factory(*, fp16_accumulate: bool) -> LaunchFn:
-    """Launcher for one accumulation mode: allocation-free but for the sums of a split K."""
+    """Allocation-free launcher for one accumulation mode (K is never split)."""
 
     def launch(args: TensorArgs, output: torch.Tensor) -> None:
         a, b = args
@@ -190,22 +203,30 @@ def _launch_factory(*, fp16_accumulate: bool) -> LaunchFn:
             raise ValueError("output metadata must match the inputs")
         if not output.is_contiguous():
             raise ValueError("matmul output must be contiguous")
-        _enqueue(a, b, output, fp16_accumulate=fp16_accumulate)
+        _enqueue(a, b, output, fp16_accumulate=fp16_accumulate, whole=True)
 
     return launch
 
 
-def _enqueue(a: torch.Tensor, b: torch.Tensor, output: torch.Tensor, *, fp16_accumulate: bool) -> None:
-    """``output = a @ b`` for operands and an output already checked."""
-    m, k = a.shape
-    splits = split_k(m, b.shape[1], k)
-    if splits > 1:
-        enqueue_split(a, b, output, splits)
+def _enqueue(
+    a: torch.Tensor, b: torch.Tensor, output: torch.Tensor, *, fp16_accumulate: bool, whole: bool = False
+) -> None:
+    """``output = a @ b`` for operands and an output already checked; ``whole``: never split K."""
+    (m, k), n = a.shape, b.shape[1]
+    a_strides, b_strides, a_ptr, b_ptr = a.stride(), b.stride(), a.data_ptr(), b.data_ptr()
+    splits = 1 if whole else split_k(m, n, k)
+    if (splits > 1 and not (a_ptr | b_ptr) & 15 and _dma_operand(m, k, *a_strides)
+            and _dma_operand(k, n, *b_strides)):
+        sums = torch.empty(splits * m * n, device=a.device, dtype=torch.float32)
+        _hip.call(
+            "tk_gemm_splitk", _hip.dtype_code(a.dtype), a_ptr, b_ptr, None, None, output.data_ptr(),
+            sums.data_ptr(), m, n, k, splits, *a_strides, *b_strides, *b_strides, *output.stride(),
+            _hip.stream_of(a),
+        )
         return
     _hip.call(
-        "tk_gemm", _hip.dtype_code(a.dtype), a.data_ptr(), b.data_ptr(), output.data_ptr(), m,
-        b.shape[1], k, *a.stride(), *b.stride(), *output.stride(), int(fp16_accumulate),
-        _hip.stream_of(a),
+        "tk_gemm", _hip.dtype_code(a.dtype), a_ptr, b_ptr, output.data_ptr(), m, n, k, *a_strides,
+        *b_strides, *output.stride(), int(fp16_accumulate), _hip.stream_of(a),
     )
 
 
@@ -214,7 +235,7 @@ _launch_fp16acc = _launch_factory(fp16_accumulate=True)
 
 
 def matmul_fp32acc(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
-    """``a @ b`` with float32 MFMA accumulation."""
+    """``a @ b`` with float32 MFMA accumulation, summed over K in the order :func:`split_k` states."""
     _validate(a, b)
     output = _make_output((a, b))
     _enqueue(a, b, output, fp16_accumulate=False)
