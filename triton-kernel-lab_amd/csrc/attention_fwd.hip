@@ -371,7 +371,8 @@ attn_fwd_dma_kernel(FwdArgs<T> kernel_arg) {
         __builtin_amdgcn_make_buffer_rsrc((void*)Vh, (short)0, v_bytes, 0x00020000);
 
     // DMA sources (bytes from the head's base, block-relative row). Rows past the sequence
-    // end are past the buffer extent and read as zero.
+    // end are past the buffer extent and read as zero: the range check is on voffset plus
+    // soffset, which carries the block's offset.
     uint32_t k_src[G::DMA_PER_OP], v_src[G::DMA_PER_OP];
 #pragma unroll
     for (int x = 0; x < G::DMA_PER_OP; ++x) {
@@ -817,7 +818,7 @@ attn_fwd_small_kernel(FwdArgs<T> args) {
   const int kv_end = CAUSAL ? min(N, q0 + S::BM) : N;
   const int blocks = (kv_end + BN - 1) / BN;
   const uint32_t k_blk = uint32_t(BN * s.k[2]) * 2u, v_blk = uint32_t(BN * s.v[2]) * 2u;
-  // Blocks past the end reload the last one into a stage that is never read.
+  // Rows past the sequence end read as zero, as in the 256-query kernel. Blocks past the end reload the last one into a stage that is never read.
   auto load = [&](int blk, int stage) {
     blk = min(blk, blocks - 1);
     small_dma<D>(rk, rv, lds + stage * STB + wave * S::DMA_PER_OP * 1024, k_src, v_src,

@@ -96,10 +96,11 @@ constexpr int kScaleOff = 256 * 528;
 static_assert(kScaleOff + 256 * 4 <= kLdsBytes, "row scales past the LDS block");
 
 // Sources of the DMA instructions a wave issues per tile: src for full tiles, last for the
-// operand's last tile, of which kv K columns (or k-rows) lie inside K. A tile's offset travels
-// in soffset, which the buffer range check does not cover, so lanes past kv must read nothing
-// (kOob) on their own. K % 8 == 0 wherever K is contiguous, so a lane's chunk is wholly inside
-// or outside.
+// operand's last tile, of which kv K columns (or k-rows) lie inside K. What lies past K in a
+// K-contiguous operand is the next row, inside the buffer, so lanes past kv must read nothing
+// (kOob) on their own; k-rows past K are past the buffer's end (the range check covers soffset,
+// which carries a tile's offset) and follow the same rule. K % 8 == 0 wherever K is contiguous, so
+// a lane's chunk is wholly inside or outside.
 //
 // 64-wide tile of a K-contiguous operand, instruction x (0..3): rows 8 (4 wave + x) .. +7,
 // eight lanes per 128-byte row; each lane fetches the chunk that belongs at its LDS slot.
