@@ -174,6 +174,14 @@ int tk_gemm(int dtype, const void* a, const void* b, void* c, int64_t m, int64_t
             int64_t stride_bn, int64_t stride_cm, int64_t stride_cn, int acc_fp16,
             void* stream);
 
+/* The kernel and the block tile tk_gemm takes for a problem: kernel << 20 | rows << 10 | columns with
+ * kernel 1 gemm_dma_kernel (buffer->LDS DMA, row-major operands, k % 32 == 0), 2 gemm_kernel by DMA
+ * (transposed operands, other k), 3 gemm_kernel staged through registers (every other layout); 0
+ * for sizes and strides it rejects. Only the alignment of a and b counts. A query: it launches
+ * nothing, needs no GPU and sets no error. */
+int tk_gemm_tile(const void* a, const void* b, int64_t m, int64_t n, int64_t k, int64_t stride_am,
+                 int64_t stride_ak, int64_t stride_bk, int64_t stride_bn);
+
 /* GEMM with the SwiGLU nonlinearity fused into its epilogue:
  *   y = value * gate * sigmoid(gate), gate = a * b_gate, value = a * b_up,
  * with a [m, k] and both weights [k, n]; gate and value are rounded to `dtype`

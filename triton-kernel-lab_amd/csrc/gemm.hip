@@ -231,28 +231,51 @@ void launch_staged(Layout layout, bool unit, const T* a, const T* b, T* c, const
   }
 }
 
+// How the register-staged kernel takes a problem; `swap`: as C^T = B^T A^T, both row-major, where
+// both operands are transposed (the other fields are after the swap).
+struct StagedPlan {
+  bool swap, unit;
+  Layout layout;
+  int tile;
+  int64_t a_extent, b_extent;
+};
+
+StagedPlan staged_plan(int64_t m, int64_t n, int64_t k, int64_t stride_am, int64_t stride_ak,
+                       int64_t stride_bk, int64_t stride_bn) {
+  StagedPlan plan{};
+  plan.swap = stride_ak != 1 && stride_am == 1 && stride_bn != 1 && stride_bk == 1;
+  if (plan.swap) {
+    std::swap(m, n);
+    std::swap(stride_am, stride_bn);
+    std::swap(stride_ak, stride_bk);
+  }
+  const bool a_rows = stride_ak != 1 && stride_am == 1, b_wide = stride_bn != 1 && stride_bk == 1;
+  plan.a_extent = (m - 1) * stride_am + (k - 1) * stride_ak + 1;
+  plan.b_extent = (k - 1) * stride_bk + (n - 1) * stride_bn + 1;
+  // Wide loads need eight elements to load from.
+  plan.unit = (stride_ak == 1 || a_rows) && (stride_bn == 1 || b_wide) && plan.a_extent >= 8 &&
+              plan.b_extent >= 8;
+  plan.layout = plan.unit && a_rows ? Layout::TN : plan.unit && b_wide ? Layout::NT : Layout::NN;
+  const int first = plan.unit ? 0 : kFirstStrided;
+  plan.tile = first + pick_tile(kStagedTiles + first, kStagedTileCount - first, m, n, k,
+                                Variant::kPlain);
+  return plan;
+}
+
 template <typename T>
 void gemm_staged(const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k,
                  int64_t stride_am, int64_t stride_ak, int64_t stride_bk, int64_t stride_bn,
                  int64_t stride_cm, int64_t stride_cn, hipStream_t stream) {
-  if (stride_ak != 1 && stride_am == 1 && stride_bn != 1 && stride_bk == 1) {
-    // Both transposed: C^T = B^T A^T, both row-major.
+  const StagedPlan plan = staged_plan(m, n, k, stride_am, stride_ak, stride_bk, stride_bn);
+  if (plan.swap) {
     std::swap(a, b);
     std::swap(m, n);
     std::swap(stride_am, stride_bn);
     std::swap(stride_ak, stride_bk);
     std::swap(stride_cm, stride_cn);
   }
-  const bool a_rows = stride_ak != 1 && stride_am == 1, b_wide = stride_bn != 1 && stride_bk == 1;
-  const int64_t a_extent = (m - 1) * stride_am + (k - 1) * stride_ak + 1;
-  const int64_t b_extent = (k - 1) * stride_bk + (n - 1) * stride_bn + 1;
-  // Wide loads need eight elements to load from.
-  const bool unit = (stride_ak == 1 || a_rows) && (stride_bn == 1 || b_wide) && a_extent >= 8 &&
-                    b_extent >= 8;
-  const Layout layout = unit && a_rows ? Layout::TN : unit && b_wide ? Layout::NT : Layout::NN;
-  const int first = unit ? 0 : kFirstStrided;
-  const int tile = first + pick_tile(kStagedTiles + first, kStagedTileCount - first, m, n, k,
-                                     Variant::kPlain);
+  const Layout layout = plan.layout;
+  const int tile = plan.tile;
   StagedProblem sp{};
   sp.p.m = (int)m;
   sp.p.n = (int)n;
@@ -264,20 +287,40 @@ void gemm_staged(const void* a, const void* b, void* c, int64_t m, int64_t n, in
   auto operand = [](int64_t ld, int64_t inner, int64_t extent) {
     return Operand{(uint32_t)ld, (uint32_t)inner, (uint32_t)extent};
   };
-  sp.a = layout == Layout::TN ? operand(stride_ak, 1, a_extent) : operand(stride_am, stride_ak, a_extent);
-  sp.b = layout == Layout::NT ? operand(stride_bn, 1, b_extent) : operand(stride_bk, stride_bn, b_extent);
+  sp.a = layout == Layout::TN ? operand(stride_ak, 1, plan.a_extent) : operand(stride_am, stride_ak, plan.a_extent);
+  sp.b = layout == Layout::NT ? operand(stride_bn, 1, plan.b_extent) : operand(stride_bk, stride_bn, plan.b_extent);
   const T* pa = static_cast<const T*>(a);
   const T* pb = static_cast<const T*>(b);
   T* pc = static_cast<T*>(c);
   if (tile == 0)
-    launch_staged<T, 256, 128>(layout, unit, pa, pb, pc, sp, stream);
+    launch_staged<T, 256, 128>(layout, plan.unit, pa, pb, pc, sp, stream);
   else if (tile == 1)
-    launch_staged<T, 128, 128>(layout, unit, pa, pb, pc, sp, stream);
+    launch_staged<T, 128, 128>(layout, plan.unit, pa, pb, pc, sp, stream);
   else
-    launch_staged<T, 64, 64>(layout, unit, pa, pb, pc, sp, stream);
+    launch_staged<T, 64, 64>(layout, plan.unit, pa, pb, pc, sp, stream);
 }
 
 }  // namespace
+
+extern "C" int tk_gemm_tile(const void* a, const void* b, int64_t m, int64_t n, int64_t k,
+                            int64_t stride_am, int64_t stride_ak, int64_t stride_bk,
+                            int64_t stride_bn) {
+  const int64_t lim = INT32_MAX;
+  for (int64_t s : {stride_am, stride_ak, stride_bk, stride_bn})
+    if (s <= 0) return 0;
+  if (m <= 0 || n <= 0 || k <= 0 || m > lim || n > lim || k > lim ||
+      tk::extent(m, stride_am, k, stride_ak) > lim || tk::extent(k, stride_bk, n, stride_bn) > lim)
+    return 0;
+  auto pack = [](int kernel, Tile t) { return kernel << 20 | t.m << 10 | t.n; };
+  Plan plan;
+  if (tk::gemm_dma::plan(a, b, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, &plan)) {
+    const bool plain = plan.layout == Layout::NN && !plan.swap && !plan.k_tail;
+    const int tile = plan.swap ? pick_tile(kTiles, kTileCount, n, m, k, Variant::kPlain)
+                               : pick_tile(kTiles, kTileCount, m, n, k, Variant::kPlain);
+    return pack(plain ? 1 : 2, kTiles[tile]);
+  }
+  return pack(3, kStagedTiles[staged_plan(m, n, k, stride_am, stride_ak, stride_bk, stride_bn).tile]);
+}
 
 extern "C" int tk_gemm(int dtype, const void* a, const void* b, void* c, int64_t m, int64_t n,
                        int64_t k, int64_t stride_am, int64_t stride_ak, int64_t stride_bk,

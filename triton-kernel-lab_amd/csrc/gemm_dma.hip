@@ -586,8 +586,7 @@ bool gemm_split_launch(int dtype, const void* a, const void* b, const void* b_up
                           : row_scale != nullptr ? Variant::kRowScale
                                                  : Variant::kPlain;
   if (variant != Variant::kPlain &&
-      (plan.layout != Layout::NN || plan.swap ||
-       !gemm_dma_applies(a, b, m, n, k, sam, sak, sbk, sbn) ||
+      (!gemm_dma_applies(a, b, m, n, k, sam, sak, sbk, sbn) ||
        (b_up != nullptr && !gemm_dma_applies(a, b_up, m, n, k, sam, sak, suk, sun))))
     return false;
   if (plan.swap) {

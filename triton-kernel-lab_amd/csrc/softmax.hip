@@ -245,11 +245,8 @@ __device__ __forceinline__ void chunk_partial_streamed(const T* p, int n, float*
     if (ACCESS == tk::Access::kAny || c + VEC > n) {
 #pragma unroll
       for (int k = 0; k < VEC; ++k) f[k] = c + k < n ? tk::to_f32(p[c + k]) : -INFINITY;
-    } else if (c < n) {
-      tk::load_vec<T, VEC>(p + c, f);
     } else {
-#pragma unroll
-      for (int k = 0; k < VEC; ++k) f[k] = -INFINITY;
+      tk::load_vec<T, VEC>(p + c, f);
     }
   };
   float f[VEC];

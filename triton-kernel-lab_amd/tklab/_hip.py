@@ -112,6 +112,7 @@ _SIGNATURES: dict[str, list[object]] = {
 
 # Queries: their int result is an answer, not a status.
 _QUERIES: dict[str, list[object]] = {
+    "tk_gemm_tile": [_P, _P] + [_I64] * 7,
     "tk_attn_fwd_rows": [_I64, _I64, _I64, _I64, _I64, _I64, _I32],
 }
 
@@ -207,6 +208,6 @@ def call(name: str, *args: object) -> None:
         raise HipLibraryError(f"{name} failed: {message}")
 
 
-def query(name: str, *args: int) -> int:
+def query(name: str, *args: int | None) -> int:
     """The answer of a query entry point (:data:`_QUERIES`); needs no GPU."""
     return getattr(load_library(), name)(*args)

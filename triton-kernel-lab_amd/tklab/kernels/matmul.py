@@ -43,17 +43,15 @@ _DTYPES = (torch.float16, torch.bfloat16)
 # (the B operand's; A is loaded in 64-wide tiles into a ring of kAStages = 3).
 TILE = {"hip_kernel": "gemm_dma_kernel", "block_m": 256, "block_n": 256, "block_k": 32, "group_m": 4,
         "num_warps": 8, "num_stages": 4}
-# csrc/gemm_tile.hpp (kTiles): the tiles of problems too small to fill the chip with those; K step
-# 64, the stages that fit a CU's LDS (half of it for the smallest tiles, two workgroups per CU).
-_TILES = ((256, 256), (256, 128), (128, 256), (192, 192), (128, 192), (192, 128), (128, 128),
-          (128, 64), (64, 128), (64, 64))
+# tk_gemm_tile's kernels. The 256 x 256 one of gemm_dma.hip is TILE; the smaller DMA tiles
+# (csrc/gemm_tile.hpp) step K by 64 with the stages that fit a CU's LDS (half of it for the smallest
+# tiles, two workgroups per CU), the register-staged ones (csrc/gemm.hip) with two stages.
+_KERNELS = {1: "gemm_dma_kernel", 2: "gemm_kernel", 3: "gemm_kernel"}
+_STAGED = 3
 _MFMA = {
     torch.float16: "v_mfma_f32_16x16x32_f16",
     torch.bfloat16: "v_mfma_f32_16x16x32_bf16",
 }
-# csrc/gemm.hip's register-staged kernel (kStagedTiles): every other operand layout, two LDS
-# stages. The first tile takes operands with one unit stride each only.
-_STAGED_TILES = ((256, 128), (128, 128), (64, 64))
 
 
 def _dma_rows(rows: int, cols: int, row_stride: int, col_stride: int) -> bool:
@@ -71,16 +69,6 @@ def _dma_operand(rows: int, cols: int, row_stride: int, col_stride: int) -> bool
     The base must be 16-byte aligned too.
     """
     return _dma_rows(rows, cols, row_stride, col_stride) or _dma_rows(cols, rows, col_stride, row_stride)
-
-
-def _pick_tile(m: int, n: int, k: int, tiles: tuple[tuple[int, int], ...] = _TILES) -> tuple[int, int]:
-    """The tile for a problem (``pick_tile``, csrc/gemm_dma.hip)."""
-
-    def cost(tile: tuple[int, int]) -> float:
-        rounds = -(-(-(-m // tile[0]) * -(-n // tile[1])) // 256)
-        return rounds * (4000.0 + 6.1 * sum(tile) * -(-k // 64))
-
-    return min(tiles, key=cost)
 
 
 def split_k(m: int, n: int, k: int) -> int:
@@ -126,41 +114,33 @@ def enqueue_split(
     )
 
 
-def _tile_config(tile: tuple[int, int], *, staged: bool = False) -> dict[str, BenchmarkScalar]:
-    """Metadata of a tile: K step 64 and a ring that fits the LDS, except the 256 x 256 kernel's."""
-    if tile == _TILES[0]:
-        return TILE
-    stage = sum(tile) * 128
-    stages = 81920 // stage if sum(tile) <= 192 else min(5, 163840 // stage)
-    return {**TILE, "block_m": tile[0], "block_n": tile[1], "block_k": 64,
-            "group_m": 8 if tile[1] > tile[0] else 4, "num_stages": 2 if staged else stages}
+def _tile_config(rows: int, cols: int, *, kernel: int = 1) -> dict[str, BenchmarkScalar]:
+    """Metadata of a tile of one of :data:`_KERNELS`."""
+    config = {**TILE, "hip_kernel": _KERNELS[kernel], "block_m": rows, "block_n": cols}
+    if (rows, cols) == (256, 256):
+        return config
+    stage = (rows + cols) * 128
+    stages = 81920 // stage if rows + cols <= 192 else min(5, 163840 // stage)
+    return {**config, "block_k": 64, "group_m": 8 if cols > rows else 4,
+            "num_stages": 2 if kernel == _STAGED else stages}
+
+
+def _query_tile(
+    a_ptr: int, b_ptr: int, m: int, n: int, k: int, a_strides: tuple[int, ...], b_strides: tuple[int, ...]
+) -> tuple[int, int, int]:
+    """(kernel, rows, columns) of ``tk_gemm_tile``."""
+    tile = _hip.query("tk_gemm_tile", a_ptr, b_ptr, m, n, k, *a_strides, *b_strides)
+    return tile >> 20, tile >> 10 & 1023, tile & 1023
 
 
 def launch_config(a: torch.Tensor, b: torch.Tensor) -> dict[str, BenchmarkScalar]:
-    """Tile configuration and MFMA of the kernel ``matmul_fp32acc`` launches for ``a @ b``.
-
-    Mirrors ``gemm_dma::plan`` and ``pick_tile`` (csrc/gemm_dma.hip) and ``gemm_staged``
-    (csrc/gemm.hip).
-    """
+    """Tile configuration and MFMA of the kernel ``matmul_fp32acc`` launches for ``a @ b``."""
     (m, k), n = a.shape, b.shape[1]
     mma = {"mma_opcode": _MFMA.get(a.dtype, _MFMA[torch.float16])}
-    aligned = not (a.data_ptr() | b.data_ptr()) & 15
-    if aligned and all(_dma_operand(*t.shape, *t.stride()) for t in (a, b)):
-        if split_k(m, n, k) > 1:
-            return {**_tile_config((64, 64)), **mma, "hip_kernel": "gemm_split_kernel"}
-        by_rows = [_dma_rows(*t.shape, *t.stride()) for t in (a, b)]
-        plain = all(by_rows) and k % 32 == 0
-        swapped = not any(by_rows)  # computed as C^T = B^T A^T
-        tile = _pick_tile(n, m, k) if swapped else _pick_tile(m, n, k)
-        return {**_tile_config(tile), **mma,
-                "hip_kernel": "gemm_dma_kernel" if plain else "gemm_kernel"}
-    (am, ak), (bk, bn) = a.stride(), b.stride()
-    unit = (all(1 in t.stride() and (t.shape[0] - 1) * t.stride(0)
-                + (t.shape[1] - 1) * t.stride(1) >= 7 for t in (a, b)))
-    swapped = ak != 1 and am == 1 and bn != 1 and bk == 1
-    tiles = _STAGED_TILES if unit else _STAGED_TILES[1:]
-    tile = _pick_tile(n, m, k, tiles) if swapped else _pick_tile(m, n, k, tiles)
-    return {**_tile_config(tile, staged=True), **mma, "hip_kernel": "gemm_kernel"}
+    kernel, rows, cols = _query_tile(a.data_ptr(), b.data_ptr(), m, n, k, a.stride(), b.stride())
+    if kernel != _STAGED and split_k(m, n, k) > 1:
+        return {**_tile_config(64, 64), **mma, "hip_kernel": "gemm_split_kernel"}
+    return {**_tile_config(rows, cols, kernel=kernel), **mma}
 
 
 def _validate(a: torch.Tensor, b: torch.Tensor) -> None:
@@ -285,8 +265,9 @@ def _metadata_factory() -> BenchmarkMetadataFn:
     """Tile configuration in the reference's metadata keys (``matmul.py:292-312``)."""
 
     def metadata(size: int, dtype: torch.dtype) -> dict[str, BenchmarkScalar]:
-        # Registry inputs are contiguous size x size matrices (size % 32 == 0).
-        return {**_tile_config(_pick_tile(size, size, size)), "mma_opcode": _MFMA.get(dtype, _MFMA[torch.float16])}
+        # Registry inputs are contiguous, aligned size x size matrices; the launcher never splits K.
+        kernel, rows, cols = _query_tile(0, 0, size, size, size, (size, 1), (size, 1))
+        return {**_tile_config(rows, cols, kernel=kernel), "mma_opcode": _MFMA.get(dtype, _MFMA[torch.float16])}
 
     return metadata
 
