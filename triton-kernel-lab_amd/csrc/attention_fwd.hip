@@ -45,6 +45,7 @@
 #include "attention.hpp"
 #include "attention_dma.hpp"
 
+#include <cmath>
 #include <type_traits>
 
 namespace {
@@ -1064,16 +1065,27 @@ int64_t fwd_tiles(int64_t batch, int64_t heads, int64_t seq, int64_t total, int6
   return (total > 0 ? varlen_tiles(batch, total, seq, rows) : batch * tk::cdiv(seq, rows)) * heads;
 }
 
+// Queries that tiles of `rows` queries hold for a sequence of a packed batch: exactly where all have
+// one length, half a tile of padding on the mean length otherwise (the lengths are on the device).
+double packed_queries(int64_t batch, int64_t seq, int64_t total, int64_t rows) {
+  return total == batch * seq ? double(rows * tk::cdiv(seq, rows))
+                              : double(total) / double(batch) + double(rows) / 2;
+}
+
 // What 256-query tiles cost a packed batch over 128-query ones: (query, key) pairs of the whole
-// blocks a sequence needs (causal: up to each tile's last query). Sequences of one length have it
-// exactly; others count half a tile of padding on the mean length.
+// blocks a sequence needs (causal: up to each tile's last query).
 double packed_cost_of_256(int64_t batch, int64_t seq, int64_t total, bool causal) {
-  auto cost = [&](double rows) {
-    const double queries = total == batch * seq ? rows * double(tk::cdiv(seq, int64_t(rows)))
-                                                : double(total) / double(batch) + rows / 2;
-    return causal ? queries * (queries + rows) : queries;
+  auto cost = [&](int64_t rows) {
+    const double queries = packed_queries(batch, seq, total, rows);
+    return causal ? queries * (queries + double(rows)) : queries;
   };
   return cost(256) / cost(128);
+}
+
+// Rounds of one 256-query workgroup per CU that a packed batch takes, over the rounds it fills.
+double packed_idle_of_256(int64_t batch, int64_t heads, int64_t seq, int64_t total) {
+  const double rounds = double(batch * heads) * packed_queries(batch, seq, total, 256) / (256.0 * 256.0);
+  return rounds > 1 ? std::ceil(rounds) / rounds : 1.0;
 }
 
 // Query tiles per wave of the small-workgroup kernel, or 0 for the 256-query kernel. A problem
@@ -1094,12 +1106,16 @@ double packed_cost_of_256(int64_t batch, int64_t seq, int64_t total, bool causal
 //                        16 x 2048 (1.06) 613/633, 8 x 4096 (1.03) 1014/1095
 //   causal D128 H16 G16: 60 of 400 .. 1500 (1.28) 377/357, 40 x 768 (1.14) 190/198, 32 x 1000
 //                        222/247; H32 G32: 60 of 400 .. 1500 766/889, 40 x 768 413/473,
-//                        100 x 300 (1.67) 372/292; few tiles: H8 G8 15 of 300 .. 2000 63/53
+//                        100 x 300 (1.67) 372/292; H32 G16 27 x 386 (1.20) 120/100; few tiles: H8 G8
+//                        15 of 300 .. 2000 63/53
 //   causal D64  H16 G16: 15 of 300 .. 2000 (1.25) 65/59, 40 x 700 (1.14) 86/96; H8 G8 64 x 1024
-//                        (1.11) 111/121; H32 G8 50 x 640 (1.33) 187/154
+//                        (1.11) 111/121; H32 G8 50 x 640 (1.33) 187/154; H4 G4 26 x 1898 73/67
 //   full D128   H32 G8:  100 of 100 .. 1000 (1.13) 656/623, 15 to 1779 (1.13) 128/135, 40 x 768
 //                        (1.00) 435/445; H32 G32 40 x 768 520/718, 100 x 256 268/289; H16 G16
-//                        100 x 256 135/127
+//                        100 x 256 135/127; a last round of CUs half empty (packed_idle_of_256):
+//                        H16 G16 12 x 500 (1.33) 45/39, 6 x 1000 (1.33) 65/58, H8 G4 19 x 532
+//                        (1.12, cost 1.20) 46/39; none: H8 G8 12 x 500 23.1/24.4, 32 x 1000 146/174;
+//                        H32 G32 3 of 1982 (1.73, cost 1.09) 42/36, 14 to 1056 (1.12, 1.11) 121/127
 int small_query_tiles(int64_t batch, int64_t heads, int64_t kv_heads, int64_t seq, int64_t head_dim,
                       int64_t total, bool causal) {
   const int64_t tiles = fwd_tiles(batch, heads, seq, total, 64);
@@ -1114,11 +1130,14 @@ int small_query_tiles(int64_t batch, int64_t heads, int64_t kv_heads, int64_t se
   const bool grouped = heads >= 4 * kv_heads, few_kv = kv_heads <= 16;
   const double cost = packed_cost_of_256(batch, seq, total, causal);
   if (causal) {
-    if (wide ? tiles <= 2304 && seq <= 2048 : tiles <= 3072) return 2;
-    return cost >= (grouped ? 1.1 : few_kv ? 1.22 : 1.28) ? 2 : 0;
+    if (wide ? tiles <= 2304 && seq <= 2048 : tiles <= 3328) return 2;
+    return cost >= (grouped ? 1.1 : !few_kv ? 1.28 : wide ? 1.19 : 1.22) ? 2 : 0;
   }
   if (!wide) return 0;
-  if (seq <= 256 && few_kv) return 2;
+  if (few_kv && seq <= 256) return 2;
+  if (seq <= 1088 &&
+      cost * packed_idle_of_256(batch, heads, seq, total) >= (few_kv ? 1.22 : 1.4))
+    return 2;
   return cost >= (grouped && seq <= 1024 ? 1.12 : 1.22) ? 2 : 0;
 }
 
