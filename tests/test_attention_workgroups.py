@@ -58,7 +58,9 @@ def test_packed_batches_take_the_measured_workgroup(problem, rows) -> None:
     ((128, 128, [8192], 64, True), 256), ((32, 32, [1024], 128, True), 64), ((8, 8, [8192], 128, True), 128),
     ((256, 256, [512], 128, True), 128), ((64, 64, [2048], 128, True), 256), ((32, 32, [1024], 64, False), 64),
     ((64, 64, [1024], 64, False), 256), ((16, 16, [1024], 128, False), 64), ((4, 4, [8192], 128, False), 128),
-    ((48, 48, [512], 128, False), 64), ((64, 64, [1024], 128, False), 256),
+    ((8, 8, [1000] * 16, 128, True), 128), ((4, 4, [1000] * 31, 128, True), 256),
+    ((4, 4, [1000] * 27, 128, True), 128), ((1, 1, [900] * 113, 128, True), 256),
+    ((1, 1, [768] * 141, 128, True), 128), ((48, 48, [512], 128, False), 64), ((64, 64, [1024], 128, False), 256),
 ])
 def test_equal_lengths_take_the_fastest_column_of_the_table(problem, rows) -> None:
     assert _rows(*problem, packed=False) == rows

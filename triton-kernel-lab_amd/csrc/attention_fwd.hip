@@ -1094,7 +1094,9 @@ double packed_idle_of_256(int64_t batch, int64_t heads, int64_t seq, int64_t tot
 //                H16 N8192 (2048) 245/173/158, H64 N8192 (8192) 635/700/587,
 //                H128 N8192 (16384) 1176/-/1211
 //   causal D128: H32 N1024 (512) 39.6/17.3/22.0, H8 N8192 (1024) 180/167/158,
-//                H256 N512 (2048) 39.9/39.8/34.1, H64 N2048 (2048) 67.9/87.8/74.1
+//                H256 N512 (2048) 39.9/39.8/34.1, H64 N2048 (2048) 67.9/87.8/74.1,
+//                H128 N1000 (2048) 44.1/-/43.9, H124 N1000 46.8/-/50.3, H108 N1000 43.9/-/42.2,
+//                H113 N900 (1695) 44.8/-/50.2, H102 N923 (1530) 43.4/56.2/43.4
 //   full D64:    H32 N1024 (512) 22.9/14.8/17.3, H64 N1024 (1024) 25.1/27.4/26.3
 //   full D128:   H16 N1024 (256) 27.5/15.8/21.5, H7 N2048 (224) 47/27/38, H48 N512 (384)
 //                17.6/13.0/13.4, H28 N1024 (448) 27.5/22.3/22.1, H14 N2048 (448) 47.6/40.1/38.5,
@@ -1125,7 +1127,12 @@ int small_query_tiles(int64_t batch, int64_t heads, int64_t kv_heads, int64_t se
   if (causal && wide && tiles <= 1024) return 2;
   if (!packed) {
     if (!causal) return 0;
-    return wide ? (tiles <= 2048 && seq <= 1024 ? 2 : 0) : (tiles <= 8192 ? 2 : 0);
+    if (!wide) return tiles <= 8192 ? 2 : 0;
+    // From four 256-query blocks per head on, heads that do not divide over the XCDs share their
+    // L2s with others' keys, and the small workgroups read those twice as often.
+    const int64_t bh = batch * heads;
+    const int64_t most = seq <= 768 || bh % 8 == 0 ? 2048 : bh % 4 == 0 ? 1728 : 1500;
+    return tiles <= most && seq <= 1024 ? 2 : 0;
   }
   const bool grouped = heads >= 4 * kv_heads, few_kv = kv_heads <= 16;
   const double cost = packed_cost_of_256(batch, seq, total, causal);
