@@ -318,8 +318,9 @@ __global__ __launch_bounds__(kTileThreads) void gemm_kernel(const T* __restrict_
 }
 
 // Split K. A problem of few 64 x 64 tiles and a long K leaves most CUs idle while one workgroup
-// walks K, and a CU pulls ~30 GB/s whatever its ring holds (deeper rings, two K tiles per barrier
-// and nt loads changed nothing). Its K is cut into runs of whole K tiles, one workgroup each,
+// walks K at what one CU pulls: unsplit, the five problems below request 29 to 48 GB/s per CU over
+// the whole launch (64x4096x14336 43, 16x512x8192 48; deeper rings, two K tiles per barrier and nt
+// loads changed nothing). Its K is cut into runs of whole K tiles, one workgroup each,
 // whose float32 sums the second kernel adds in order of K and rounds as the unsplit epilogues
 // do. bf16, unsplit -> split, both kernels: 64x4096x14336 84.6 -> 31.9 us (4 runs, 117 MB: 3.8
 // TB/s), 16x2048x8192 37.1 -> 14.4 (8), 16x6144x4096 22.7 -> 16.7 (2), 16x512x8192 27.4 -> 10.6

@@ -74,10 +74,10 @@ def _dma_operand(rows: int, cols: int, row_stride: int, col_stride: int) -> bool
 def split_k(m: int, n: int, k: int) -> int:
     """Runs of K for ``tk_gemm_splitk``; 1: one workgroup per output tile walks all of K.
 
-    A workgroup takes ~0.3 us per 64-wide K tile of a 64 x 64 tile; the second kernel and the
-    float32 sums take ~4 us of the device and ~5 of the host. One round of the 256 CUs and runs
-    of at least 16 K tiles were the best or within 8 % of it: 64x4096x14336 (64 tiles) 84.6 us
-    unsplit, 4 runs 31.9, 6 40.1, 8 35.3; 16x512x8192 (8 tiles) 27.4, 8 runs 10.6, 16 12.0. Past
+    A workgroup takes 0.2 to 0.4 us per 64-wide K tile of a 64 x 64 tile (10 KiB with 16 rows of A,
+    16 KiB with 64); the second kernel and the float32 sums take ~4 us of the device and ~5 of the
+    host. One round of the 256 CUs and runs of at least 16 K tiles were the best or within 8 % of
+    it: 64x4096x14336 (64 tiles) 84.6 us unsplit, 4 runs 31.9, 6 40.1, 8 35.3; 16x512x8192 (8 tiles) 27.4, 8 runs 10.6, 16 12.0. Past
     128 tiles nothing is left to fill (256x4096x8192: 46.7, 2 runs 49.4). Below the least depth
     a call is shorter than its host time: with the norm of a QKV projection 1x4096x4096 19.3
     unsplit, 23.9 split, the product 8x512x3072 11.6 and 14.0; from 96 tiles HBM traffic moves
